@@ -154,8 +154,7 @@ static void build_block_sell(int n, RB rb, RE re, const int *ja, std::vector<int
 static int upload_block_sell(cfd_mesh *m, const std::vector<int> &off, const HostArray<int> &col,
                              const HostArray<int> &src, BlockSell &bs);
 
-// Rows of each level followed by -1 up to a multiple of w.
-static void pad_levels(const std::vector<int> &ptr, const std::vector<int> &rows, int w, std::vector<int> &out) {
+void pad_levels(const std::vector<int> &ptr, const std::vector<int> &rows, int w, std::vector<int> &out) {
     out.clear();
     for (size_t l = 0; l + 1 < ptr.size(); l++) {
         for (int k = ptr[l]; k < ptr[l + 1]; k++) out.push_back(rows[k]);
@@ -766,9 +765,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             pad_levels(m->upper.ptr, urows, 12, s12);
             m->upper.n12 = (int)s12.size();
             if (!rc) m->upper.slots12 = upload(m, s12.data(), s12.size(), &rc);
-            std::vector<int> zeros((size_t)N + 1, 0);
-            if (!rc) m->ready = upload(m, zeros.data(), (size_t)N, &rc);
-            if (!rc) m->epoch = upload(m, zeros.data(), 1, &rc);
             const char *sf = getenv("CFD_SYNC_FREE");
             m->sync_free = !(sf && sf[0] == '0');
             const char *gr = getenv("CFD_GRAPHS");
@@ -861,14 +857,14 @@ extern "C" int64_t cfd_footprint_bytes(int32_t N, int32_t E, int32_t B, int32_t 
     // qa, qb, lsq, res, vol, dt, boundary areas, right-hand side, update
     bytes += 8 * (kQA * (n + b) + kQB * n + 8 * n + kRES * n + n + n + 4 * b + 5 * n + 5 * n);
     // order, inverse order, inc_ptr, sptr, n2n lists, boundary node/type/tag, Roe-pass candidates and block
-    // flags, ready flags, epoch, risk
-    bytes += 4 * (n + n + (n + 1) + (n / kSlice + 2) + (n + 1) + 2 * e + 3 * b + 2 * n + (n / 4096 + 1) + n + 2);
+    // flags, risk
+    bytes += 4 * (n + n + (n + 1) + (n / kSlice + 2) + (n + 1) + 2 * e + 3 * b + 2 * n + (n / 4096 + 1) + 1);
     bytes += nsell * (4 + 4 + 3 * 8);                       // nbr, soff, isx, isy, isz
     bytes += 4 * ((n + 1) + nnz + n) + 4 * nnz;             // BSR ia, ja, iau; ILU(0) merge offsets
     bytes += 4 * 8 * nnz;                                   // ILU(0) merge map (<= 8 upper blocks per lower entry)
     bytes += 4 * (n + (n + 1) + 3 * nnz + n + 2 * n) + 4 * 8 * nnz;  // multicolour pattern, slot map, levels, merge map
-    bytes += s * 5 * n;                                     // multicolour work vector
-    bytes += 4 * (2 * n + 2 * n + (11 + 11) * lvl);        // level rows and padded slot lists
+    bytes += s * 2 * 5 * n;                                 // work vectors of the sweeps
+    bytes += 4 * (2 * n + 4 * n + 4 * 11 * lvl);           // level rows and padded slot lists
     bytes += 8 * (1024 * 65 + 4 * 65 + 6) + 4 * 4;         // reduction scratch, eigenvalue bits, flags
     bytes += 25 * s * nnz * 2 + 25 * s * n;                 // Jacobian, ILU(0) factors, inverse pivots
     bytes += s * 5 * n * (2 * (int64_t)km + 2) + 8 * 5 * n; // Krylov V, Z, w; FP64 true residual

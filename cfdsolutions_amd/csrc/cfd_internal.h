@@ -60,7 +60,7 @@ struct LevelSchedule {
     int nlevels = 0;
     int maxwidth = 0;
     // rows in level order with every level padded (-1) to a multiple of 12
-    // (sync-free sweeps, 12 rows of 5 lanes per wavefront)
+    // (single-launch sweeps, chunks of 12 rows of 5 lanes per wavefront)
     int *slots12 = nullptr;
     int n12 = 0;
 };
@@ -239,9 +239,12 @@ struct cfd_mesh {
     float *af = nullptr;      // FP32 Jacobian (mixed)
     double *lu = nullptr, *dinv = nullptr;
     float *luf = nullptr, *dinvf = nullptr;
-    double *gslu = nullptr;   // [N][25] no-pivot LU of the diagonal blocks (block GS)
-    double *rowbuf = nullptr; // [N] per-row sums of the GS sweep
+    double *gslu = nullptr;   // [N][25] LU of the diagonal blocks (block GS, LU-SGS)
+    double *gsver = nullptr;  // [gs_nver][6 N] versions of x and row sums of the sweeps of one launch
+    int gs_nver = 0;
     LevelSchedule lower, upper;
+    LevelSchedule gs;         // schedule of pipelined Gauss-Seidel sweeps (made on first use)
+    int gs_reach = 0;         // and how many of its chunks an upper neighbour can be ahead
     // multicolour ILU(0): rows ordered by the colour of a greedy colouring of
     // the node graph (in reference order), then by index, so the triangular
     // factors have one level per colour
@@ -251,11 +254,9 @@ struct cfd_mesh {
     int *mc_src = nullptr;                                // [nnz] original slot of each permuted slot
     int *mc_moff = nullptr, *mc_mqq = nullptr;            // ILU(0) merge map of the permuted pattern
     LevelSchedule mc_lower, mc_upper;
-    double *zp = nullptr;                                 // [N][5] permuted work vector
+    double *zp = nullptr;  // 2 x [N][5] work vectors of the sweeps (single-launch: handover words)
     float *zpf = nullptr;
     bool sync_free = true;    // single-launch triangular sweeps (else one launch per level)
-    int *ready = nullptr;     // [N] sweep completion epochs
-    int *epoch = nullptr;     // [1] current sweep epoch
     // block-SELL copies for the Krylov loop: A (SpMV), and the multicolour
     // ILU(0) factors split into strict lower and upper parts plus the
     // inverted diagonal blocks (one block per row, slot = row)
@@ -350,6 +351,8 @@ int cfd_ensure_fp32(cfd_mesh *m);
 // incidence lists (once per mesh) and the FP32 copy of their area vectors
 // when fp32 is set.
 int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order);  // order: kPatchNodeOrder or kPatchEdgeOrder
+// Rows of each level followed by -1 up to a multiple of w.
+void pad_levels(const std::vector<int> &ptr, const std::vector<int> &rows, int w, std::vector<int> &out);
 int cfd_ensure_ilu_map(cfd_mesh *m);  // natural-order ILU(0) merge map, on first use
 // Whether the residual of these parameters runs the flux-once patch kernel:
 // the fast build at second order, unless CFD_FLUX_ONCE=0 or 1 forces it.

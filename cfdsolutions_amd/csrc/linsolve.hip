@@ -690,35 +690,45 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int nrows, const int *__r
 }
 
 // ---------------------------------------------------------------------------
-// Sync-free triangular sweeps (ILU(0) apply): one launch per sweep instead of
-// one per level.  The factorization, once per Jacobian, stays one launch per
-// level.
-// Rows are taken in level order and every wavefront holds rows of a single
-// level (levels are padded to whole wavefronts, pad = -1), so a row waits
-// only on rows of earlier wavefronts.  Workgroups are dispatched in index
-// order, so the earliest unfinished row always has a slot and the sweep
-// always progresses.
+// Row-to-row handover: sweeps whose rows depend on one another run in one
+// launch, each row starting as soon as the rows it reads are done.
 //
-// Each XCD has its own L2 and the L2s are not coherent with one another; an
-// agent-scope acquire invalidates the whole local L2, so it must not sit in a
-// polling loop.  The values one row hands to another are written with
-// coherent (relaxed agent-scope atomic) stores that go past the L2, then the
-// row sets ready[row] = epoch with an agent-scope release store (one L2
-// write-back per finished row).  A waiting row polls the flag with coherent
-// loads, orders
-// its later loads after the poll (workgroup acquire fence: no cache
-// invalidation) and reads the handed-over values with coherent loads, which
-// bypass stale cache lines.  The epoch is read from device
-// memory (bumped by k_epoch_bump before each sweep), so ready[] never needs
-// clearing.  A wait that exceeds kSpinMax polls raises flag[3]; every waiter
-// also watches flag[3] and gives up once it is set, so a sweep always ends,
-// after at most one bounded wait.
+// A value and the fact that it is ready are one aligned word: every word of
+// the handover array holds a NaN with a payload of its own ("unset") until its
+// row stores the result, so a reader needs no flag, no fence and no ordering
+// between addresses.  The 8 XCDs' L2s are not coherent with one another, so
+// both sides use relaxed agent-scope accesses, which go past them.  (A flag per
+// row needs a release store, which writes the XCD's L2 back: 1244 us per FP64
+// sweep over the 14,161 rows in 205 levels of the 48x16x16 mesh, 6 us a level;
+// one word per value: 354 us.)  A result that is itself a NaN is stored as the
+// default NaN, so no result can look unset.
+//
+// Waves take their rows in level order, chunk w, w + W, ... of W waves, and a
+// row reads only rows of earlier chunks (levels are padded to whole chunks), so
+// the earliest unfinished chunk is always being worked on once its wave runs.
+// All waves of a launch have to be resident: a grid is at most a quarter of the
+// workgroups that the GPU holds at the kernel's registers (flow_blocks of the
+// workgroups per CU that its launch bounds ask for), for the four hardware
+// queues that can run sweeps of different streams at a time.  A wait over kSpinMax polls raises flag[3],
+// and every waiter gives up once it is set: a sweep always ends, and the solve
+// reports it.
 // ---------------------------------------------------------------------------
 constexpr int kSpinMax = 1 << 22;
+constexpr int kFlowShare = 64;  // a quarter of the 256 CUs
+constexpr int flow_blocks(int per_cu) { return kFlowShare * per_cu; }
 
-__global__ void k_epoch_bump(int *epoch) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) epoch[0] = epoch[0] + 1;
-}
+template <class T>
+struct FlowWord;
+template <>
+struct FlowWord<double> {
+    using U = unsigned long long;
+    static constexpr U unset = 0x7ff8c0ded15ea5edull, nan = 0x7ff8000000000000ull;
+};
+template <>
+struct FlowWord<float> {
+    using U = unsigned;
+    static constexpr U unset = 0x7fc5a17du, nan = 0x7fc00000u;
+};
 
 template <class T>
 __device__ __forceinline__ T ld_coh(const T *p) {
@@ -728,75 +738,156 @@ template <class T>
 __device__ __forceinline__ void st_coh(T *p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+template <class T>
+__device__ __forceinline__ typename FlowWord<T>::U flow_load(const T *p) {
+    return ld_coh(reinterpret_cast<const typename FlowWord<T>::U *>(p));
+}
+template <class T>
+__device__ __forceinline__ void flow_store(T *p, T v) {
+    using W = FlowWord<T>;
+    st_coh(reinterpret_cast<typename W::U *>(p), v == v ? __builtin_bit_cast(typename W::U, v) : W::nan);
+}
+template <class T>
+__device__ __forceinline__ void flow_unset(T *p) {
+    st_coh(reinterpret_cast<typename FlowWord<T>::U *>(p), FlowWord<T>::unset);
+}
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_flow_unset(size_t n, T *x) {
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) flow_unset(x + i);
+}
 
-__device__ __forceinline__ bool wait_ready(const int *ready, int j, int ep, int *flag) {
-    bool ok = false;
-    for (int it = 0; it < kSpinMax; it++) {
-        if (ld_coh(ready + j) == ep) {
-            ok = true;
-            break;
+// One to U blocks of a row at once, without branches: places
+// past the last block repeat it, and their products are dropped.  Lane r of the
+// row's five loads row r of every block and component r of every neighbour, all
+// before the wait, so that the entries are there when the last neighbour
+// arrives; the neighbours' components then go through LDS to the other lanes.
+// (What a row costs after its last neighbour is mostly instructions of one
+// wave: with a branch, a wait and shuffles per block the FP64 sweep of the
+// 48x16x16 mesh took 685 us, with one wait for all blocks 400 us, so 354 us;
+// the handover itself takes 0.4 us of a level's 1.7 us.)
+template <class T>
+struct FlowLds {
+    static constexpr int row = sizeof(T) == 8 ? 6 : 8;     // values of a neighbour (5), aligned for wide reads
+    static constexpr int slot = 8 * row + (sizeof(T) == 8 ? 2 : 4);  // rows of a wavefront start in different banks
+    T v[kBlock / 64][13 * slot];
+};
+template <int U, class TM, class TV>
+struct FlowBlocks {
+    TM av[U][5];
+    const TV *x;  // component r of row 0
+    int j[U], n;
+    typename FlowWord<TV>::U v[U];
+    __device__ __forceinline__ void load(int k0, int ke, int r, const int *__restrict__ ja, const TM *__restrict__ a,
+                                         const TV *xx) {
+        x = xx + r;
+        n = ke - k0;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = u < n ? k0 + u : ke - 1;
+            j[u] = ja[k];
+            v[u] = flow_load(x + 5 * (size_t)j[u]);
+#pragma unroll
+            for (int c = 0; c < 5; c++) av[u][c] = a[25 * (size_t)k + 5 * r + c];
         }
-        if ((it & 255) == 255 && ld_coh(flag + 3) != 0) break;
-        __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (!ok && ld_coh(flag + 3) == 0) atomicOr(flag + 3, 1);
-    return ok;
-}
+    // Waits until every neighbour is there: all words are read again together
+    // until none is unset, so the row goes on one read after its last
+    // neighbour's store (one word after the other costs a read, 0.4 us, each).
+    __device__ __forceinline__ void wait(int *flag) {
+        for (int it = 0;; it++) {
+            bool all = true;
+#pragma unroll
+            for (int u = 0; u < U; u++) all = all & (v[u] != FlowWord<TV>::unset);
+            if (all) return;
+            if (it >= kSpinMax || ((it & 255) == 255 && ld_coh(flag + 3) != 0)) {
+                atomicOr(flag + 3, 1);
+                return;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (v[u] == FlowWord<TV>::unset) v[u] = flow_load(x + 5 * (size_t)j[u]);
+        }
+    }
+    // t[u] = (row r of block u) . (neighbour u); sh: this row's place in LDS.
+    __device__ __forceinline__ void dots(TV *sh, int r, TV *t) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < U; u++) sh[u * FlowLds<TV>::row + r] = __builtin_bit_cast(TV, v[u]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            TV s = TV(0.0);
+#pragma unroll
+            for (int c = 0; c < 5; c++) s += (TV)av[u][c] * sh[u * FlowLds<TV>::row + c];
+            t[u] = u < n ? s : TV(0.0);
+        }
+    }
+};
 
-// The row's stores are visible device-wide before its flag is set (an
-// s_waitcnt on the coherent stores alone does not order them before the flag
-// for readers on other XCDs).
-__device__ __forceinline__ void publish_ready(int *ready, int i, int ep) {
-    __hip_atomic_store(ready + i, ep, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Same arithmetic as k_trsv_level; 12 rows of 5 lanes per wavefront.
+// One sweep of the ILU(0) apply; 12 rows of 5 lanes per wavefront, lane r owns
+// component r.  Forward: w_i = r_P(i) - sum_{k<i} L_ik w_k; backward:
+// w_i = D_i^-1 (w_i - sum_{k>i} U_ik w_k), z_P(i) = w_i, in the operation order
+// of k_trsv_level and k_trsv_mc.  perm is the row permutation P of the
+// multicolour order, NULL for the natural order.  wf, wb: handover arrays of
+// the forward and backward sweep; each sweep leaves the other one's words of
+// its rows unset for the sweep after it.
+template <class TM>
+constexpr int kTrsvPerCu = sizeof(TM) == 4 ? 4 : 2;
 template <class TM, class TV>
-__global__ __launch_bounds__(kBlock) void k_trsv_sf(int nslots, const int *__restrict__ slots,
-                                                    const int *__restrict__ ia, const int *__restrict__ ja,
-                                                    const int *__restrict__ iau, const TM *__restrict__ lu,
-                                                    const TM *__restrict__ dinv, const TV *__restrict__ rhs, TV *z,
-                                                    int backward, int *ready, const int *epoch, int *flag) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int slot = lane / 5, r = lane - 5 * slot;
-    const int t = (blockIdx.x * (kBlock / 64) + wave) * 12 + slot;
-    const int i = (slot < 12 && t < nslots) ? slots[t] : -1;
-    const int ep = epoch[0];
-    TV y = TV(0.0);
-    bool ok = true;
-    if (i >= 0) {
-        const int kb = backward ? iau[i] + 1 : ia[i];
-        const int ke = backward ? ia[i + 1] : iau[i];
-        y = backward ? ld_coh(z + 5 * (size_t)i + r) : rhs[5 * (size_t)i + r];
-        for (int kk = kb; kk < ke; kk++) {
-            const int j = ja[kk];
-            ok = wait_ready(ready, j, ep, flag) && ok;
-            const TM *A = lu + 25 * (size_t)kk + 5 * r;
-            const TV *zj = z + 5 * (size_t)j;
-            TV s = TV(0.0);
-#pragma unroll
-            for (int c = 0; c < 5; c++) s += (TV)A[c] * ld_coh(zj + c);
-            y = y - s;
-        }
-    }
-    if (backward) {
-        // gather the row's 5 components from its lanes, then apply D_i^-1
-        const int base = lane - r;
-        TV yy[5];
-#pragma unroll
-        for (int c = 0; c < 5; c++) yy[c] = __shfl(y, base + c, 64);
+__global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_trsv_flow(int nslots, const int *__restrict__ slots,
+                                                      const int *__restrict__ ia, const int *__restrict__ ja,
+                                                      const int *__restrict__ iau, const int *__restrict__ perm,
+                                                      const TM *__restrict__ lu, const TM *__restrict__ dinv,
+                                                      const TV *__restrict__ rhs, TV *wf, TV *wb, TV *z, int backward,
+                                                      int *flag) {
+    const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
+    TV *cur = backward ? wb : wf, *other = backward ? wf : wb;
+    __shared__ __align__(16) FlowLds<TV> lds;
+    TV *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<TV>::slot;
+    const int nw = gridDim.x * (kBlock / 64);
+    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); 12 * w < nslots; w += nw) {
+        const int t = 12 * w + slot;
+        const int i = slot < 12 && t < nslots ? slots[t] : -1;
+        TV y = TV(0.0);
+        TM dr[5];
+        size_t pi = 0;
         if (i >= 0) {
-            const TM *D = dinv + 25 * (size_t)i + 5 * r;
-            TV s = TV(0.0);
+            if (backward) {
 #pragma unroll
-            for (int c = 0; c < 5; c++) s += (TV)D[c] * yy[c];
-            y = s;
+                for (int c = 0; c < 5; c++) dr[c] = dinv[25 * (size_t)i + 5 * r + c];
+            }
+            const int kb = backward ? iau[i] + 1 : ia[i];
+            const int ke = backward ? ia[i + 1] : iau[i];
+            pi = 5 * (size_t)(perm ? perm[i] : i) + r;
+            y = backward ? other[5 * (size_t)i + r] : rhs[pi];
+            flow_unset(other + 5 * (size_t)i + r);
+            for (int k0 = kb; k0 < ke; k0 += 8) {
+                FlowBlocks<8, TM, TV> g;
+                TV t[8];
+                g.load(k0, ke, r, ja, lu, cur);
+                g.wait(flag);
+                g.dots(sh, r, t);
+#pragma unroll
+                for (int u = 0; u < 8; u++) y = y - t[u];
+            }
         }
+        if (backward) {
+            // gather the row's 5 components from its lanes, then apply D_i^-1
+            TV yy[5];
+#pragma unroll
+            for (int c = 0; c < 5; c++) yy[c] = __shfl(y, base + c, 64);
+            if (i >= 0) {
+                TV s = TV(0.0);
+#pragma unroll
+                for (int c = 0; c < 5; c++) s += (TV)dr[c] * yy[c];
+                y = s;
+                z[pi] = y;
+            }
+        }
+        if (i >= 0) flow_store(cur + 5 * (size_t)i + r, y);
     }
-    if (i >= 0) st_coh(z + 5 * (size_t)i + r, y);
-    if (i >= 0 && r == 0) publish_ready(ready, i, ep);
-    if (!ok) atomicOr(flag + 3, 1);
 }
 
 // Blocks of the matrix in multicolour order: dst[s] = src[map[s]].
@@ -1193,67 +1284,121 @@ __global__ __launch_bounds__(kBlock) void k_gs_lu(int N, const int *iau, const d
     for (int q = 0; q < 25; q++) lu[25 * (size_t)r + q] = L[q];
 }
 
-// One forward Gauss-Seidel row update, MC_Iterative_Jacobi.c:410-450
-__global__ __launch_bounds__(kBlock) void k_gs_level(int nrows, const int *rows, const int *ia, const int *ja,
-                                                     const int *iau, const double *a, const double *b,
-                                                     const double *lu, double *x, double *rowrms) {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= nrows) return;
-    const int r = rows[t];
-    double rhs[5], tv[5];
-    for (int m = 0; m < 5; m++) rhs[m] = b[5 * (size_t)r + m];
-    for (int j = ia[r]; j < ia[r + 1]; j++) {
-        const double *A = a + 25 * (size_t)j, *xj = x + 5 * (size_t)ja[j];
-        for (int ii = 0; ii < 5; ii++) tv[ii] = 0.0;
-        for (int ii = 0; ii < 5; ii++)
-            for (int jj = 0; jj < 5; jj++) tv[ii] += A[5 * ii + jj] * xj[jj];
-        for (int m = 0; m < 5; m++) rhs[m] -= tv[m];
-    }
-    double s = 0.0;
-    for (int m = 0; m < 5; m++) s += rhs[m] * rhs[m];
-    rowrms[r] = s;
-    const double *D = a + 25 * (size_t)iau[r];
-    double *xr = x + 5 * (size_t)r;
-    for (int ii = 0; ii < 5; ii++) tv[ii] = 0.0;
-    for (int ii = 0; ii < 5; ii++)
-        for (int jj = 0; jj < 5; jj++) tv[ii] += D[5 * ii + jj] * xr[jj];
-    for (int m = 0; m < 5; m++) rhs[m] += tv[m];
-    const double *L = lu + 25 * (size_t)r;
-    for (int ii = 0; ii < 5; ii++) {
-        tv[ii] = rhs[ii];
-        for (int jj = 0; jj < ii; jj++) tv[ii] -= L[5 * ii + jj] * tv[jj];
-    }
-    double xn[5];
-    for (int ii = 4; ii >= 0; ii--) {
-        xn[ii] = tv[ii];
-        for (int jj = 4; jj > ii; jj--) xn[ii] -= L[5 * ii + jj] * xn[jj];
-        xn[ii] = xn[ii] / L[5 * ii + ii];
-    }
-    for (int ii = 0; ii < 5; ii++) xr[ii] = xn[ii];
+// A row's 5x5 block, of which its lane r holds row r, to all its lanes; sh as
+// in FlowBlocks::dots.
+__device__ __forceinline__ const double *flow_lu(double *sh, int r, const double *lr) {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 5; q++) sh[5 * r + q] = lr[q];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return sh;
 }
 
-// LU-SGS row update with pivoted LU of the diagonal recomputed per sweep,
-// MC_Iterative_Jacobi.c:586-678 and MATH/src/LinearAlgebra.c:20-41,117-155
-__global__ __launch_bounds__(kBlock) void k_lusgs_level(int nrows, const int *rows, const int *ia, const int *ja,
-                                                        const int *iau, const double *a, const double *b, double *x) {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= nrows) return;
-    const int r = rows[t];
-    double rhs[5], tv[5];
-    for (int j = 0; j < 5; j++) rhs[j] = b[5 * (size_t)r + j];
-    const int diag = iau[r];
-    for (int j = ia[r]; j < ia[r + 1]; j++) {
-        if (j == diag) continue;
-        const double *A = a + 25 * (size_t)j, *xj = x + 5 * (size_t)ja[j];
-        for (int ii = 0; ii < 5; ii++) tv[ii] = 0.0;
-        for (int ii = 0; ii < 5; ii++)
-            for (int jj = 0; jj < 5; jj++) tv[ii] += A[5 * ii + jj] * xj[jj];
-        for (int m = 0; m < 5; m++) rhs[m] -= tv[m];
+// Forward Gauss-Seidel sweeps 0..S-1 in one launch (row update:
+// MC_Iterative_Jacobi.c:410-450), rows handed over as in k_trsv_flow: sweep s
+// writes its own version ver[s] of x, so row i of sweep s needs only its
+// lower neighbours of sweep s and its upper ones (and itself) of sweep s - 1,
+// and sweep s follows `reach` + 1 chunks behind sweep s - 1 instead of waiting
+// for its end (reach: how many chunks ahead an upper neighbour can be,
+// ensure_gs_schedule).  Items (chunk c, sweep s) go in ascending
+// c + s (reach + 1), so each needs only earlier ones.  The chain is about
+// levels + 8 S rows long instead of levels * S: 20 sweeps of the 48x16x16 mesh
+// (205 levels) took 64.3 ms with a launch per level, 2.07 ms so.
+// x0: x before the first sweep.  rowrms[s][i]: row i's sum of sweep s.
+constexpr int kGsPerCu = 2;
+__global__ __launch_bounds__(kBlock, kGsPerCu) void k_gs_flow(int N, int nchunk, int reach, int S, const int *__restrict__ slots,
+                                                    const int *__restrict__ ia, const int *__restrict__ ja,
+                                                    const int *__restrict__ iau, const double *__restrict__ a,
+                                                    const double *__restrict__ b, const double *__restrict__ lu,
+                                                    const double *x0, double *ver, double *rowrms, int *flag) {
+    const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
+    __shared__ __align__(16) FlowLds<double> lds;
+    double *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<double>::slot;
+    const int64_t items = ((int64_t)nchunk + (int64_t)(S - 1) * (reach + 1)) * S;
+    const int nw = gridDim.x * (kBlock / 64);
+    for (int64_t w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); w < items; w += nw) {
+        const int s = (int)(w % S);
+        const int64_t c = w / S - (int64_t)s * (reach + 1);
+        if (c < 0 || c >= nchunk) continue;
+        const int i = slot < 12 ? slots[12 * c + slot] : -1;
+        const double *prev = s ? ver + (size_t)(s - 1) * 5 * N : x0;
+        double *cur = ver + (size_t)s * 5 * N;
+        const size_t ri = 5 * (size_t)(i >= 0 ? i : 0) + r;
+        const int diag = i >= 0 ? iau[i] : 0;
+        double rhs = 0.0, own = 0.0, lr[5] = {};
+        if (i >= 0) {
+            const int ke = ia[i + 1];
+            rhs = b[ri];
+            // the diagonal and upper blocks' products first: their values are
+            // of the sweep before and mostly there; subtracted in block order
+#pragma unroll
+            for (int q = 0; q < 5; q++) lr[q] = lu[5 * ri + q];
+            FlowBlocks<8, double, double> g;
+            double tu[8], t[8];
+            g.load(diag, ke, r, ja, a, prev);
+            g.wait(flag);
+            g.dots(sh, r, tu);
+            own = tu[0];
+            for (int k0 = ia[i]; k0 < diag; k0 += 8) {
+                g.load(k0, diag, r, ja, a, cur);
+                g.wait(flag);
+                g.dots(sh, r, t);
+#pragma unroll
+                for (int u = 0; u < 8; u++) rhs -= t[u];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) rhs -= tu[u];
+            for (int k0 = diag + 8; k0 < ke; k0 += 8) {
+                g.load(k0, ke, r, ja, a, prev);
+                g.wait(flag);
+                g.dots(sh, r, t);
+#pragma unroll
+                for (int u = 0; u < 8; u++) rhs -= t[u];
+            }
+        }
+        double sq = 0.0;
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            const double e = __shfl(rhs, base + q, 64);
+            sq += e * e;
+        }
+        if (i >= 0 && r == 0) rowrms[(size_t)s * N + i] = sq;
+        rhs += own;
+        // every lane of the row solves with the LU factors of the diagonal block
+        const double *L = flow_lu(sh, r, lr);
+        double tv[5], xn[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            tv[q] = __shfl(rhs, base + q, 64);
+#pragma unroll
+            for (int p = 0; p < q; p++) tv[q] -= L[5 * q + p] * tv[p];
+        }
+#pragma unroll
+        for (int q = 4; q >= 0; q--) {
+            xn[q] = tv[q];
+#pragma unroll
+            for (int p = 4; p > q; p--) xn[q] -= L[5 * q + p] * xn[p];
+            xn[q] = xn[q] / L[5 * q + q];
+        }
+        double xr = xn[0];
+#pragma unroll
+        for (int q = 1; q < 5; q++) xr = r == q ? xn[q] : xr;
+        if (i >= 0) flow_store(cur + ri, xr);
     }
+}
+
+// Pivoted LU of the diagonal blocks for the LU-SGS sweeps (the same factors
+// in every sweep), MATH/src/LinearAlgebra.c:20-41: rows in pivot order, the
+// order itself as five decimal digits.
+__global__ __launch_bounds__(kBlock) void k_lusgs_lu(int N, const int *iau, const double *a, double *lu, int *piv) {
+    const int r = blockIdx.x * kBlock + threadIdx.x;
+    if (r >= N) return;
     double A[5][5];
     int P[5];
     for (int i = 0; i < 5; i++)
-        for (int j = 0; j < 5; j++) A[i][j] = a[25 * (size_t)diag + 5 * i + j];
+        for (int j = 0; j < 5; j++) A[i][j] = a[25 * (size_t)iau[r] + 5 * i + j];
     for (int i = 0; i < 5; i++) P[i] = i;
     for (int c = 0; c < 5; c++) {
         double pm = A[P[c]][c];
@@ -1272,19 +1417,78 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_level(int nrows, const int *ro
         for (int i = c + 1; i < 5; i++)
             for (int j = c + 1; j < 5; j++) A[P[i]][j] -= A[P[i]][c] * A[P[c]][j];
     }
-    double y[5], xs[5];
-    y[0] = rhs[P[0]];
-    for (int i = 1; i < 5; i++) {
-        y[i] = rhs[P[i]];
-        for (int j = 0; j < i; j++) y[i] -= y[j] * ((i == j) ? 1.0 : A[P[i]][j]);
+    int code = 0;
+    for (int i = 4; i >= 0; i--) code = 10 * code + P[i];
+    piv[r] = code;
+    for (int i = 0; i < 5; i++)
+        for (int j = 0; j < 5; j++) lu[25 * (size_t)r + 5 * i + j] = A[P[i]][j];
+}
+
+// One LU-SGS half sweep (row update: MC_Iterative_Jacobi.c:586-678,
+// MATH/src/LinearAlgebra.c:117-155) in one launch, rows handed over as in
+// k_trsv_flow: the neighbours swept before row i are read from cur, the others
+// from prev, the result of the half sweep before.  next is left unset for the
+// half sweep after this one.  Half sweeps run in opposite directions, so they
+// do not overlap.
+__global__ __launch_bounds__(kBlock, kGsPerCu) void k_lusgs_flow(int nslots, const int *__restrict__ slots,
+                                                       const int *__restrict__ ia, const int *__restrict__ ja,
+                                                       const int *__restrict__ iau, const double *__restrict__ a,
+                                                       const double *__restrict__ b, const double *__restrict__ lu,
+                                                       const int *__restrict__ piv, const double *prev, double *cur,
+                                                       double *next, int backward, int *flag) {
+    const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
+    __shared__ __align__(16) FlowLds<double> lds;
+    double *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<double>::slot;
+    const int nw = gridDim.x * (kBlock / 64);
+    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); 12 * w < nslots; w += nw) {
+        const int t = 12 * w + slot;
+        const int i = slot < 12 && t < nslots ? slots[t] : -1;
+        const size_t ri = 5 * (size_t)(i >= 0 ? i : 0) + r;
+        const int diag = i >= 0 ? iau[i] : 0;
+        int code = 0;
+        double rhs = 0.0, lr[5] = {};
+        if (i >= 0) {
+#pragma unroll
+            for (int q = 0; q < 5; q++) lr[q] = lu[5 * ri + q];
+            const int ke = ia[i + 1];
+            code = piv[i];
+            rhs = b[ri];
+            flow_unset(next + ri);
+            for (int side = 0; side < 2; side++) {
+                const double *x = side == backward ? cur : prev;
+                const int kb = side ? diag + 1 : ia[i], kn = side ? ke : diag;
+                for (int k0 = kb; k0 < kn; k0 += 8) {
+                    FlowBlocks<8, double, double> g;
+                    double t[8];
+                    g.load(k0, kn, r, ja, a, x);
+                    g.wait(flag);
+                    g.dots(sh, r, t);
+#pragma unroll
+                    for (int u = 0; u < 8; u++) rhs -= t[u];
+                }
+            }
+        }
+        const double *L = flow_lu(sh, r, lr);
+        double y[5], xs[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            y[q] = __shfl(rhs, base + code % 10, 64);
+            code /= 10;
+#pragma unroll
+            for (int p = 0; p < q; p++) y[q] -= y[p] * L[5 * q + p];
+        }
+#pragma unroll
+        for (int q = 4; q >= 0; q--) {
+            xs[q] = y[q];
+#pragma unroll
+            for (int p = 4; p > q; p--) xs[q] -= xs[p] * L[5 * q + p];
+            xs[q] /= L[5 * q + q];
+        }
+        double xr = xs[0];
+#pragma unroll
+        for (int q = 1; q < 5; q++) xr = r == q ? xs[q] : xr;
+        if (i >= 0) flow_store(cur + ri, xr);
     }
-    xs[4] = y[4] / A[P[4]][4];
-    for (int i = 3; i >= 0; i--) {
-        xs[i] = y[i];
-        for (int j = 4; j > i; j--) xs[i] -= xs[j] * A[P[i]][j];
-        xs[i] /= A[P[i]][i];
-    }
-    for (int j = 0; j < 5; j++) x[5 * (size_t)r + j] = xs[j];
 }
 
 __global__ __launch_bounds__(kBlock) void k_lusgs_init(int N, const double *b, double *x) {
@@ -1293,7 +1497,7 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_init(int N, const double *b, d
     double s = 0.0;
     for (int j = 0; j < 5; j++) s += b[5 * (size_t)r + j];
     s /= 5;
-    for (int j = 0; j < 5; j++) x[5 * (size_t)r + j] = s;
+    for (int j = 0; j < 5; j++) flow_store(x + 5 * (size_t)r + j, s);  // read as handover words
 }
 
 // ---------------------------------------------------------------------------
@@ -1563,8 +1767,11 @@ __global__ __launch_bounds__(kBlock) void k_xupdate(size_t n, int nv, const TV *
     }
 }
 
+// Partial sums of blockIdx.y vectors of n values, vector k into column k of
+// the partials.
 __global__ __launch_bounds__(kBlock) void k_vsum_partial(size_t n, const double *v, double *part) {
     __shared__ double sh[kBlock];
+    v += (size_t)blockIdx.y * n;
     double acc = 0.0;
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) acc += v[i];
     sh[threadIdx.x] = acc;
@@ -1573,7 +1780,7 @@ __global__ __launch_bounds__(kBlock) void k_vsum_partial(size_t n, const double 
         if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[(size_t)blockIdx.x * (kMaxKrylov + 1)] = sh[0];
+    if (threadIdx.x == 0) part[(size_t)blockIdx.x * (kMaxKrylov + 1) + blockIdx.y] = sh[0];
 }
 
 __global__ void k_fill(size_t n, double v, double *x) {
@@ -1815,6 +2022,20 @@ void spmv(cfd_mesh *m, const TX *x, TY *y, const double *bsub) {
                            0, m->stream, m->N, m->ia, m->ja, bsr_a<TM>(m), x, y, bsub);
 }
 
+// Whether the sweeps of this preconditioner run in one launch each: always in
+// the natural order (hundreds of levels), in the multicolour order (8 colours
+// on the bump channels) up to kFlowMcRows rows.  There a launch per colour
+// costs more than the handovers; above, all waves of a colour together keep
+// more loads in flight than the resident waves of one launch.  Whole implicit
+// steps, mixed precision: 14,161 rows 4.74 ms against 5.96 ms with a launch
+// per colour, 45,625 rows (ten steps) 43.1 against 48.7 ms, 104,448 rows 21.4
+// against 19.8 ms.
+constexpr int kFlowMcRows = 65536;
+bool flow_sweeps(const cfd_mesh *m, int kind) {
+    return m->sync_free &&
+           (kind == CFD_PREC_ILU0 || (kind == CFD_PREC_ILU0_MC && !m->use_sell && m->N <= kFlowMcRows));
+}
+
 template <class TV>
 TV *mc_work(cfd_mesh *m);
 template <>
@@ -1825,7 +2046,17 @@ float *mc_work<float>(cfd_mesh *m) { return m->zpf; }
 template <class TM, class TV>
 void apply_prec(cfd_mesh *m, int kind, const TM *lu, const TM *dinv, const TV *r, TV *z) {
     const size_t L = 5 * (size_t)m->N;
-    if (kind == CFD_PREC_ILU0_MC && !m->use_sell) {
+    if (flow_sweeps(m, kind)) {
+        const bool mc = kind == CFD_PREC_ILU0_MC;
+        TV *wf = mc_work<TV>(m);
+        for (int pass = 0; pass < 2; pass++) {
+            const LevelSchedule &ls = mc ? (pass ? m->mc_upper : m->mc_lower) : (pass ? m->upper : m->lower);
+            hipLaunchKernelGGL((k_trsv_flow<TM, TV>), dim3(std::min((ls.n12 + 47) / 48, flow_blocks(kTrsvPerCu<TM>))),
+                               dim3(kBlock), 0, m->stream, ls.n12, ls.slots12, mc ? m->mc_ia : m->ia, mc ? m->mc_ja : m->ja,
+                               mc ? m->mc_iau : m->iau, mc ? m->mc_perm : nullptr, lu, dinv, r, wf, wf + L, z, pass,
+                               m->flag);
+        }
+    } else if (kind == CFD_PREC_ILU0_MC && !m->use_sell) {
         TV *wk = mc_work<TV>(m);
         for (int pass = 0; pass < 2; pass++) {
             const LevelSchedule &ls = pass ? m->mc_upper : m->mc_lower;
@@ -1867,13 +2098,6 @@ void apply_prec(cfd_mesh *m, int kind, const TM *lu, const TM *dinv, const TV *r
                 hipLaunchKernelGGL((k_trsv_mc_sell<TM, TV>), dim3(g), dim3(kBlock), 0, m->stream, r0, r1, m->mc_ia,
                                    m->mc_iau, m->mc_perm, bs.off, bs.col, val, dv, r, wk, z, pass);
             }
-        }
-    } else if (kind == CFD_PREC_ILU0 && m->sync_free) {
-        for (int pass = 0; pass < 2; pass++) {
-            const LevelSchedule &ls = pass ? m->upper : m->lower;
-            hipLaunchKernelGGL(k_epoch_bump, dim3(1), dim3(64), 0, m->stream, m->epoch);
-            hipLaunchKernelGGL((k_trsv_sf<TM, TV>), dim3((ls.n12 + 47) / 48), dim3(kBlock), 0, m->stream, ls.n12,
-                               ls.slots12, m->ia, m->ja, m->iau, lu, dinv, r, z, pass, m->ready, m->epoch, m->flag);
         }
     } else if (kind == CFD_PREC_ILU0) {
         for (int pass = 0; pass < 2; pass++) {
@@ -1941,8 +2165,8 @@ void cgs_pass(cfd_mesh *m, int nv, const TV *V, size_t ld, int hoff, TV *w, int 
 // precision.
 int ensure_krylov(cfd_mesh *m, int mk, bool mixed) {
     const size_t L = 5 * (size_t)m->N;
-    if (mixed && !m->zpf) m->zpf = (float *)cfd_dalloc(m, sizeof(float) * L);
-    if (!mixed && !m->zp) m->zp = (double *)cfd_dalloc(m, sizeof(double) * L);
+    if (mixed && !m->zpf) m->zpf = (float *)cfd_dalloc(m, sizeof(float) * 2 * L);
+    if (!mixed && !m->zp) m->zp = (double *)cfd_dalloc(m, sizeof(double) * 2 * L);
     if ((mixed && !m->zpf) || (!mixed && !m->zp))
         return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (multicolour work vector)");
     if (!m->r) m->r = (double *)cfd_dalloc(m, sizeof(double) * L);
@@ -2385,34 +2609,99 @@ void drop_krylov_graphs(cfd_mesh *m) {
     }
 }
 
+// The schedule of k_gs_flow (host, on the mesh's first Gauss-Seidel solve).
+// Row i of sweep s takes step p_i + lag s: p_i is the least number above the
+// p of every lower neighbour and at least p_k + 1 - lag for every upper
+// neighbour k.  The passes below raise p to that; they end for every lag from
+// the number of levels on, and in three passes for lag 8 on the bump channels
+// (lag 7 is the least there; the levels by themselves jump by up to 50 from a
+// row to an upper neighbour).  reach: the largest number of chunks from a row
+// to an upper neighbour.
+static int ensure_gs_schedule(cfd_mesh *m) {
+    if (m->gs.slots12) return CFD_OK;
+    const int N = m->N;
+    std::vector<int> p(N), chunk(N), s12, rows(N);
+    for (int lag = 8;; lag *= 2) {
+        std::fill(p.begin(), p.end(), 0);
+        bool raised = true;
+        for (int pass = 0; pass < 16 && raised; pass++) {
+            raised = false;
+            for (int i = 0; i < N; i++) {
+                int t = p[i];
+                for (int k = m->h_ia[i]; k < m->h_iau[i]; k++) t = std::max(t, p[m->h_ja[k]] + 1);
+                for (int k = m->h_iau[i] + 1; k < m->h_ia[i + 1]; k++) t = std::max(t, p[m->h_ja[k]] + 1 - lag);
+                raised = raised || t > p[i];
+                p[i] = t;
+            }
+        }
+        if (!raised) break;
+    }
+    LevelSchedule &ls = m->gs;
+    ls.nlevels = *std::max_element(p.begin(), p.end()) + 1;
+    ls.ptr.assign(ls.nlevels + 1, 0);
+    for (int i = 0; i < N; i++) ls.ptr[p[i] + 1]++;
+    for (int l = 0; l < ls.nlevels; l++) ls.ptr[l + 1] += ls.ptr[l];
+    std::vector<int> at(ls.ptr.begin(), ls.ptr.end() - 1);
+    for (int i = 0; i < N; i++) rows[at[p[i]]++] = i;
+    pad_levels(ls.ptr, rows, 12, s12);
+    for (size_t t = 0; t < s12.size(); t++)
+        if (s12[t] >= 0) chunk[s12[t]] = (int)(t / 12);
+    m->gs_reach = 0;
+    for (int i = 0; i < N; i++)
+        for (int k = m->h_iau[i] + 1; k < m->h_ia[i + 1]; k++)
+            m->gs_reach = std::max(m->gs_reach, chunk[m->h_ja[k]] - chunk[i]);
+    int *d = (int *)cfd_dalloc(m, sizeof(int) * s12.size());
+    if (!d) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (sweep schedule)");
+    CFD_HIP(m, cfd_memcpy(d, s12.data(), sizeof(int) * s12.size(), hipMemcpyHostToDevice));
+    ls.slots12 = d;
+    ls.n12 = (int)s12.size();
+    return CFD_OK;
+}
+
+// Scratch of the Gauss-Seidel sweeps, all of it written before it is read.
+struct GsScratch {
+    double *lu;    // [N][25] LU factors of the diagonal blocks
+    double *rows;  // [nver][N] per-row sums of the RMS of each sweep
+    double *ver;   // [nver][N][5] x after each sweep
+    int nver;      // sweeps per launch
+};
+
 // Forward block Gauss-Seidel sweeps of MC_Iterative_Block_LU_Jacobi_CRS
-// (MATH/src/MC_Iterative_Jacobi.c:346-535) with the LU factors of the
-// diagonal blocks in gslu ([N][25]) and the per-row sums of the RMS in rowbuf
-// ([N]); both are written in full before they are read.
-static int gs_sweeps(cfd_mesh *m, int sweeps, double *gslu, double *rowbuf, cfd_linsolve_stats *st) {
+// (MATH/src/MC_Iterative_Jacobi.c:346-535), up to g.nver to a launch; the
+// sweeps end with the first whose RMS is small enough, so x is its version.
+// More than one sweep to a launch needs the schedule ls and reach of
+// ensure_gs_schedule; one at a time runs on any lower level schedule.
+static int gs_sweeps(cfd_mesh *m, int sweeps, const LevelSchedule &ls, int reach, const GsScratch &g,
+                     cfd_linsolve_stats *st) {
     const size_t L = 5 * (size_t)m->N;
     hipLaunchKernelGGL(k_gs_lu, dim3((m->N + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream, m->N, m->iau, m->a,
-                       gslu);
+                       g.lu);
     hipLaunchKernelGGL(k_fill, dim3(grid_cap(L, 4096)), dim3(kBlock), 0, m->stream, L, 0.0, m->x);
+    const int nchunk = ls.n12 / 12, np = grid_cap(m->N, kDotParts);
     double rms = 0.0;
-    int it;
-    for (it = 0; it < sweeps; it++) {
-        for (int l = 0; l < m->lower.nlevels; l++) {
-            const int b0 = m->lower.ptr[l], nr = m->lower.ptr[l + 1] - b0;
-            hipLaunchKernelGGL(k_gs_level, dim3((nr + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream, nr,
-                               m->lower.rows + b0, m->ia, m->ja, m->iau, m->a, m->b, gslu, m->x, rowbuf);
-        }
-        // row RMS: ordered reduction of the per-row sums
-        const int np = grid_cap(m->N, kDotParts);
-        hipLaunchKernelGGL(k_vsum_partial, dim3(np), dim3(kBlock), 0, m->stream, (size_t)m->N, rowbuf, m->red);
-        hipLaunchKernelGGL(k_mdot_final, dim3(1), dim3(64), 0, m->stream, np, 1, m->red, m->redout);
-        CFD_HIP(m, hipMemcpyAsync(m->hred, m->redout, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    int it = 0;
+    for (bool done = false; it < sweeps && !done;) {
+        const int S = std::min(g.nver, sweeps - it);
+        hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(S * L, 4096)), dim3(kBlock), 0, m->stream, S * L, g.ver);
+        hipLaunchKernelGGL(k_gs_flow, dim3((int)std::min<int64_t>(((int64_t)nchunk * S + 3) / 4, flow_blocks(kGsPerCu))),
+                           dim3(kBlock), 0, m->stream, m->N, nchunk, reach, S, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, g.lu,
+                           m->x, g.ver, g.rows, m->flag);
+        // row RMS of each sweep: ordered reduction of the per-row sums
+        hipLaunchKernelGGL(k_vsum_partial, dim3(np, S), dim3(kBlock), 0, m->stream, (size_t)m->N, g.rows, m->red);
+        hipLaunchKernelGGL(k_mdot_final, dim3(S), dim3(64), 0, m->stream, np, S, m->red, m->redout);
+        CFD_HIP(m, hipMemcpyAsync(m->hred, m->redout, sizeof(double) * S, hipMemcpyDeviceToHost, m->stream));
+        CFD_HIP(m, hipMemcpyAsync(m->hflag, m->flag, 4 * sizeof(int), hipMemcpyDeviceToHost, m->stream));
         CFD_HIP(m, hipStreamSynchronize(m->stream));
-        rms = sqrt(m->hred[0] / (double)m->N);
-        if (rms < 100.0 * DBL_EPSILON) {
-            it++;
-            break;
+        if (m->hflag[3]) return cfd_set_error(m->ctx, CFD_E_HIP, "Gauss-Seidel sweep exceeded its wait bound");
+        int last = S;
+        for (int s = 0; s < S && !done; s++) {
+            rms = sqrt(m->hred[s] / (double)m->N);
+            done = rms < 100.0 * DBL_EPSILON;
+            if (done) last = s + 1;
         }
+        it += last;
+        CFD_HIP(m, hipMemcpyAsync(m->x, g.ver + (size_t)(last - 1) * L, sizeof(double) * L, hipMemcpyDeviceToDevice,
+                                  m->stream));
     }
     st->iterations = it;
     st->final_res = rms;
@@ -2420,12 +2709,13 @@ static int gs_sweeps(cfd_mesh *m, int sweeps, double *gslu, double *rowbuf, cfd_
 }
 
 // Scratch of cfd_linsolve_gs_noalloc: the LU factors of the diagonal blocks
-// (25 values per row) and the per-row sums (1 per row) of meshes of up to
-// kNoAllocMaxNodes nodes, 6.8 MB.  Each GPU holds its own copy until the
-// process ends; host code uses the address hipGetSymbolAddress returns for
-// the current GPU (kept per context), never the array's name.  Every call on
-// a GPU shares that GPU's copy, so calls that overlap on one GPU race.
-static __device__ __align__(256) double scratch[26 * (size_t)kNoAllocMaxNodes];
+// (25 values per row), the per-row sums (1) and x after the sweep (5) of
+// meshes of up to kNoAllocMaxNodes nodes, 8.1 MB.  Each GPU holds its own copy
+// until the process ends; host code uses the address hipGetSymbolAddress
+// returns for the current GPU (kept per context), never the array's name.
+// Every call on a GPU shares that GPU's copy, so calls that overlap on one GPU
+// race.
+static __device__ __align__(256) double scratch[31 * (size_t)kNoAllocMaxNodes];
 
 double *noalloc_scratch_address(hipError_t *err) {
     void *p = nullptr;
@@ -2443,12 +2733,24 @@ int run_gs_noalloc(cfd_mesh *m, int sweeps, cfd_linsolve_stats *st) {
                              m->N, kNoAllocMaxNodes);
     if (!m->ctx->noalloc_scratch)
         return cfd_set_error(m->ctx, CFD_E_HIP, "cfd_linsolve_gs_noalloc: scratch array address unavailable");
-    double *gslu = m->ctx->noalloc_scratch, *rowbuf = gslu + 25 * (size_t)kNoAllocMaxNodes;
-    const int rc = gs_sweeps(m, sweeps > 0 ? sweeps : 10000, gslu, rowbuf, st);
+    double *base = m->ctx->noalloc_scratch;
+    const size_t n = kNoAllocMaxNodes;
+    CFD_HIP(m, hipMemsetAsync(m->flag, 0, 4 * sizeof(int), m->stream));
+    const GsScratch g{base, base + 25 * n, base + 26 * n, 1};
+    const int rc = gs_sweeps(m, sweeps > 0 ? sweeps : 10000, m->lower, 0, g, st);
     if (rc) return rc;
     CFD_HIP(m, hipGetLastError());
     CFD_HIP(m, hipStreamSynchronize(m->stream));
     return CFD_OK;
+}
+
+// Gauss-Seidel sweeps per launch: each keeps a version of x (48 bytes per node
+// with its row sums).  A further sweep in a launch costs reach + 1 chunks of
+// the chain, a further launch the whole chain, so as many as fit 512 MB, 32 at
+// most.
+static int gs_versions(const cfd_mesh *m, int sweeps) {
+    const int64_t fit = (512LL << 20) / (48 * (int64_t)m->N);
+    return (int)std::max<int64_t>(1, std::min<int64_t>({fit, 32, sweeps}));
 }
 
 int run_linsolve(cfd_mesh *m, const cfd_linsolve_opts *o, cfd_linsolve_stats *st) {
@@ -2458,26 +2760,42 @@ int run_linsolve(cfd_mesh *m, const cfd_linsolve_opts *o, cfd_linsolve_stats *st
     if (o->solver == CFD_SOLVER_BLOCK_GS || o->solver == CFD_SOLVER_LUSGS) {
         if (m->jac_mixed) return cfd_set_error(m->ctx, CFD_E_ARG, "reference sweeps need an FP64 Jacobian");
         const int sweeps = o->sweeps > 0 ? o->sweeps : (o->solver == CFD_SOLVER_BLOCK_GS ? 10000 : 100);
-        if (o->solver == CFD_SOLVER_BLOCK_GS) {
-            if (!m->gslu) m->gslu = (double *)cfd_dalloc(m, sizeof(double) * 25 * (size_t)m->N);
-            if (!m->rowbuf) m->rowbuf = (double *)cfd_dalloc(m, sizeof(double) * (size_t)m->N);
-            if (!m->gslu || !m->rowbuf) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
-            int rc = gs_sweeps(m, sweeps, m->gslu, m->rowbuf, st);
+        const bool gs = o->solver == CFD_SOLVER_BLOCK_GS;
+        const int nver = gs ? gs_versions(m, sweeps) : 3;
+        if (!m->gslu) m->gslu = (double *)cfd_dalloc(m, sizeof(double) * 25 * (size_t)m->N);
+        if (m->gs_nver < nver) {
+            if (m->gs_nver) CFD_HIP(m, hipStreamSynchronize(m->stream));
+            cfd_dfree(m, m->gsver);
+            m->gsver = (double *)cfd_dalloc(m, sizeof(double) * 6 * (size_t)m->N * nver);
+            m->gs_nver = m->gsver ? nver : 0;
+        }
+        if (!m->gslu || !m->gsver) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
+        const size_t L = 5 * (size_t)m->N;
+        double *ver = m->gsver;  // [nver][N][5], then [nver][N] row sums (GS) or the pivot orders (LU-SGS)
+        if (gs) {
+            int rc = ensure_gs_schedule(m);
+            if (!rc) rc = gs_sweeps(m, sweeps, m->gs, m->gs_reach, GsScratch{m->gslu, ver + L * nver, ver, nver}, st);
             if (rc) return rc;
         } else {
+            int *piv = (int *)(ver + 3 * L);
             hipLaunchKernelGGL(k_lusgs_init, dim3((m->N + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream, m->N,
                                m->b, m->x);
-            for (int it = 0; it < sweeps; it++) {
-                for (int pass = 0; pass < 2; pass++) {
-                    const LevelSchedule &ls = pass ? m->upper : m->lower;
-                    for (int l = 0; l < ls.nlevels; l++) {
-                        const int b0 = ls.ptr[l], nr = ls.ptr[l + 1] - b0;
-                        hipLaunchKernelGGL(k_lusgs_level, dim3((nr + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream,
-                                           nr, ls.rows + b0, m->ia, m->ja, m->iau, m->a, m->b, m->x);
-                    }
-                }
+            hipLaunchKernelGGL(k_lusgs_lu, dim3((m->N + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream, m->N, m->iau,
+                               m->a, m->gslu, piv);
+            hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(L, 4096)), dim3(kBlock), 0, m->stream, L, ver);
+            // half sweep h writes version h % 3, reads h - 1 and clears h + 1
+            for (int h = 0; h < 2 * sweeps; h++) {
+                const LevelSchedule &ls = h % 2 ? m->upper : m->lower;
+                hipLaunchKernelGGL(k_lusgs_flow, dim3(std::min((ls.n12 + 47) / 48, flow_blocks(kGsPerCu))), dim3(kBlock),
+                                   0, m->stream, ls.n12, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, m->gslu, piv,
+                                   h ? ver + (h + 2) % 3 * L : m->x, ver + h % 3 * L, ver + (h + 1) % 3 * L, h % 2,
+                                   m->flag);
             }
+            CFD_HIP(m, hipMemcpyAsync(m->x, ver + (2 * sweeps - 1) % 3 * L, sizeof(double) * L,
+                                      hipMemcpyDeviceToDevice, m->stream));
+            CFD_HIP(m, hipGetLastError());
             st->iterations = sweeps;
+            return read_solve_flags(m);
         }
         CFD_HIP(m, hipGetLastError());
         CFD_HIP(m, hipStreamSynchronize(m->stream));
@@ -2548,6 +2866,21 @@ int ensure_sell(cfd_mesh *m, int precond, bool half, bool half_a) {
     return CFD_OK;
 }
 
+// The rows of a schedule in whole chunks of 12 (LevelSchedule::slots12), for
+// schedules that do not hold them from the mesh's creation.
+int ensure_slots12(cfd_mesh *m, LevelSchedule &ls) {
+    if (ls.slots12) return CFD_OK;
+    std::vector<int> rows(m->N), s12;
+    CFD_HIP(m, cfd_memcpy(rows.data(), ls.rows, sizeof(int) * rows.size(), hipMemcpyDeviceToHost));
+    pad_levels(ls.ptr, rows, 12, s12);
+    int *d = (int *)cfd_dalloc(m, sizeof(int) * s12.size());
+    if (!d) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (sweep schedule)");
+    CFD_HIP(m, cfd_memcpy(d, s12.data(), sizeof(int) * s12.size(), hipMemcpyHostToDevice));
+    ls.slots12 = d;
+    ls.n12 = (int)s12.size();
+    return CFD_OK;
+}
+
 int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
     if (o->krylov_m < 1 || o->krylov_m > kMaxKrylov)
         return cfd_set_error(m->ctx, CFD_E_ARG, "krylov_m must be in [1, %d]", kMaxKrylov);
@@ -2563,6 +2896,17 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
         return cfd_set_error(m->ctx, CFD_E_ARG, "Jacobian precision does not match linsolve precision");
     int rc = ensure_krylov(m, o->krylov_m, mixed);
     if (rc) return rc;
+    if (flow_sweeps(m, o->precond)) {
+        rc = ensure_slots12(m, m->mc_lower);
+        if (!rc) rc = ensure_slots12(m, m->mc_upper);
+        if (rc) return rc;
+        const size_t n = 10 * (size_t)m->N;
+        if (mixed)
+            hipLaunchKernelGGL(k_flow_unset<float>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, m->zpf);
+        else
+            hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, m->zp);
+        CFD_HIP(m, hipGetLastError());
+    }
     rc = mixed ? ensure_sell<float>(m, o->precond, half, half_a)
                : ensure_sell<double>(m, o->precond, false, false);
     if (rc) return rc;

@@ -297,7 +297,7 @@ int cfd_linsolve(cfd_mesh *mesh, const cfd_linsolve_opts *o, cfd_linsolve_stats 
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It allocates nothing: the LU factors of
  * the diagonal blocks and the per-row sums live in a file-scope device array
- * sized for meshes of at most 32,768 nodes (6.8 MB per GPU, held until the
+ * sized for meshes of at most 32,768 nodes (8.1 MB per GPU, held until the
  * process ends); larger meshes get CFD_E_ARG.  Same results as cfd_linsolve,
  * bit for bit.  Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU race. */

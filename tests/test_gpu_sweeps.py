@@ -1,0 +1,134 @@
+"""Single-launch sweeps (rows handed over value by value) on patterns where their bookkeeping can go wrong: fewer rows
+than one chunk of 12, a last chunk that is not full, rows with more neighbours than one group of eight on either side
+of the diagonal, chains (one row per level) and graphs without edges between most rows.
+
+Gauss-Seidel and LU-SGS follow the oracle's operation order, so x is equal bit for bit; the ILU(0) sweeps equal the
+launch-per-level kernels bit for bit.
+"""
+import os
+import types
+
+import numpy as np
+import pytest
+
+from cfdsolutions_amd import cfd
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+UNSET = 0x7FF8C0DED15EA5ED  # the NaN payload that marks a value as not yet handed over
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = cfd.Context(0)
+    yield c
+    c.close()
+
+
+def graph(kind, n, seed=5):
+    """A mesh-shaped node graph: the arrays cfd_mesh_create takes, with metrics that only have to be finite."""
+    rng = np.random.default_rng(seed)
+    e = set()
+    if kind == "chain":
+        e = {(i, i + 1) for i in range(n - 1)}
+    elif kind == "hub":  # node n/2 has 40 lower and 40 upper neighbours, the others a few
+        h = n // 2
+        e = {(i, i + 1) for i in range(n - 1)} | {(min(h, j), max(h, j)) for j in range(h - 40, h + 41) if j != h}
+    elif kind == "random":
+        while len(e) < 4 * n:
+            i, j = rng.integers(0, n, 2)
+            if i != j:
+                e.add((int(min(i, j)), int(max(i, j))))
+    else:  # sparse: most rows have no neighbour
+        e = {(0, n - 1)}
+    e = np.array(sorted(e), np.int32)
+    both = np.concatenate([e, e[:, ::-1]])
+    both = both[np.lexsort((both[:, 1], both[:, 0]))]
+    ia = np.concatenate([[0], np.cumsum(np.bincount(both[:, 0], minlength=n))]).astype(np.int32)
+    return types.SimpleNamespace(
+        n_node=n, edge=e, edge_area=rng.standard_normal((len(e), 3)), bedge=np.array([[0, n]], np.int32),
+        bedge_area=np.ones((1, 3)), bedge_type=np.zeros(1, np.int32), bedge_tag=np.ones(1, np.int32),
+        xyz=rng.standard_normal((n, 3)), vol=np.ones(n), n2n_ia=ia, n2n_ja=both[:, 1].astype(np.int32))
+
+
+def system(ctx, kind, n, env=None):
+    """The device mesh of the graph holding a diagonally dominant block system, and that system."""
+    old = {k: os.environ.get(k) for k in (env or {})}
+    os.environ.update(env or {})
+    try:
+        m = graph(kind, n)
+        p = cfd.make_params()
+        dm = cfd.DeviceMesh(ctx, m, p)
+    finally:
+        for k, v in old.items():
+            os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
+    ia, ja, iau = dm.bsr_structure()
+    rng = np.random.default_rng(n)
+    a = rng.uniform(-1.0, 1.0, (ja.size, 25))
+    a[iau] += (np.diff(ia)[:, None] * 3.0 + 2.0) * np.eye(5).ravel()
+    b = rng.uniform(-1.0, 1.0, (n, 5))
+    dm.jacobian_set(a, b)
+    return dm, ia, ja, iau, a, b
+
+
+SHAPES = [("chain", 2), ("chain", 30), ("sparse", 11), ("sparse", 64), ("random", 97), ("random", 1300), ("hub", 173)]
+
+
+@pytest.mark.parametrize("kind,n", SHAPES)
+@pytest.mark.parametrize("sweeps", [1, 2, 33])  # one, two pipelined, more than one launch's 32
+def test_gauss_seidel_equals_oracle(ctx, kind, n, sweeps):
+    print("gs", kind, n, sweeps, flush=True)
+    dm, ia, ja, iau, a, b = system(ctx, kind, n)
+    st = dm.linsolve(solver=cfd.SOLVER_BLOCK_GS, sweeps=sweeps)
+    x, rms = orc.block_gs(ia, ja, iau, a, b, st.iterations)
+    assert np.array_equal(dm.get(cfd.FIELD_X), x)
+    # the row sums are added in another order: n + 5 roundings each
+    assert abs(st.final_res - rms) <= 2.0 * (n + 5) * np.finfo(float).eps * rms
+    if st.iterations < sweeps:  # it stopped: at its own bound, and not a sweep late
+        assert st.final_res < 100.0 * np.finfo(float).eps
+        _, before = orc.block_gs(ia, ja, iau, a, b, st.iterations - 1)
+        assert before >= 99.0 * np.finfo(float).eps
+    rc, st2 = dm.linsolve_gs_noalloc(sweeps)
+    assert rc == 0 and st2.iterations == st.iterations and st2.final_res == st.final_res
+    assert np.array_equal(dm.get(cfd.FIELD_X), x)
+    dm.close()
+
+
+@pytest.mark.parametrize("kind,n", SHAPES)
+@pytest.mark.parametrize("sweeps", [1, 2, 5])
+def test_lusgs_equals_oracle(ctx, kind, n, sweeps):
+    print("lusgs", kind, n, sweeps, flush=True)
+    dm, ia, ja, iau, a, b = system(ctx, kind, n)
+    dm.linsolve(solver=cfd.SOLVER_LUSGS, sweeps=sweeps)
+    assert np.array_equal(dm.get(cfd.FIELD_X), orc.lusgs(ia, ja, iau, a, b, sweeps))
+    dm.close()
+
+
+@pytest.mark.parametrize("kind,n", SHAPES)
+@pytest.mark.parametrize("precond", [cfd.PREC_ILU0, cfd.PREC_ILU0_MC])
+def test_ilu_sweeps_equal_level_launches(ctx, kind, n, precond):
+    print("ilu", kind, n, precond, flush=True)
+    out = []
+    for flow in "01":
+        dm, *_ = system(ctx, kind, n, env={"CFD_SYNC_FREE": flow})
+        st = dm.linsolve(precond=precond, krylov_m=10, max_restarts=1, rtol=1e-12)
+        st = dm.linsolve(precond=precond, krylov_m=10, max_restarts=1, rtol=1e-12)  # on used handover words
+        out.append((st.iterations, st.final_res, dm.get(cfd.FIELD_X)))
+        dm.close()
+    assert out[0][:2] == out[1][:2] and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("solver", [cfd.SOLVER_BLOCK_GS, cfd.SOLVER_LUSGS])
+def test_a_right_hand_side_of_unset_words_is_a_nan_like_any_other(ctx, solver):
+    """Results that are NaN are handed over as the default NaN: a right-hand side that holds the mark itself makes x NaN
+    where the oracle's is, and no row waits for it."""
+    print("unset payload", solver, flush=True)
+    dm, ia, ja, iau, a, b = system(ctx, "random", 97)
+    b[40] = np.array([UNSET], np.uint64).view(np.float64)[0]
+    dm.jacobian_set(a, b)
+    dm.linsolve(solver=solver, sweeps=2)
+    x = orc.block_gs(ia, ja, iau, a, b, 2)[0] if solver == cfd.SOLVER_BLOCK_GS else orc.lusgs(ia, ja, iau, a, b, 2)
+    assert np.isnan(x).any()
+    np.testing.assert_array_equal(dm.get(cfd.FIELD_X), x)
+    dm.close()
