@@ -193,9 +193,10 @@ static void build_levels(const std::vector<int> &ia, const std::vector<int> &ja,
     for (int i = 0; i < N; i++) rows[pos[lev[i]]++] = i;
 }
 
+// pad: entries past the n copied ones that kernels may read (and ignore).
 template <class T>
-static T *upload(cfd_mesh *m, const T *h, size_t n, int *rc) {
-    T *d = (T *)cfd_dalloc(m, sizeof(T) * n);
+static T *upload(cfd_mesh *m, const T *h, size_t n, int *rc, size_t pad = 0) {
+    T *d = (T *)cfd_dalloc(m, sizeof(T) * (n + pad));
     if (!d) {
         *rc = cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
         return nullptr;
@@ -567,8 +568,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             },
             64);
         phase("off-diagonal slots");
-        // (the natural-order ILU(0) merge map is built on first use,
-        // cfd_ensure_ilu_map)
         std::vector<int> lrows, urows;
         build_levels(m->h_ia, m->h_ja, m->h_iau, N, false, m->lower.ptr, lrows, m->lower.maxwidth);
         build_levels(m->h_ia, m->h_ja, m->h_iau, N, true, m->upper.ptr, urows, m->upper.maxwidth);
@@ -579,8 +578,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         // reference order; rows sorted by (colour, index)
         std::vector<int> mperm(N), mia(N + 1, 0), miau(N), mlrows, murows;
         HostArray<int> mja(m->nnz), msrc(m->nnz);  // filled in full below
-        std::unique_ptr<int[]> mmoff, mmqq;
-        int64_t mc_nmap = 0;
         {
             // Greedy colouring in reference order.  The cases of a union hold
             // ascending node ranges with no edge between them, so each range
@@ -660,11 +657,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
                 }
             });
             phase("multicolour: pattern");
-            if (!build_merge_map_par(mia.data(), mja.data(), miau.data(), N, mmoff, mmqq, mc_nmap)) {
-                cfd_mesh_destroy(m);
-                return cfd_set_error(ctx, CFD_E_ARG, "cfd_mesh_create: ILU(0) merge map too large");
-            }
-            phase("multicolour: merge map");
             build_levels_by_colour(mia.data(), mja.data(), miau.data(), N, false, m->mc_cstart, m->mc_lower.ptr, mlrows,
                                    m->mc_lower.maxwidth);
             build_levels_by_colour(mia.data(), mja.data(), miau.data(), N, true, m->mc_cstart, m->mc_upper.ptr, murows,
@@ -724,15 +716,13 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         if (!rc) m->d.sa = upload(m, sa.data(), sa.size(), &rc);
         if (!rc) m->d.vol = upload(m, vol.data(), vol.size(), &rc);
         if (!rc) m->ia = upload(m, m->h_ia.data(), m->h_ia.size(), &rc);
-        if (!rc) m->ja = upload(m, m->h_ja.data(), m->h_ja.size(), &rc);
+        if (!rc) m->ja = upload(m, m->h_ja.data(), m->h_ja.size(), &rc, kIluPad);
         if (!rc) m->iau = upload(m, m->h_iau.data(), m->h_iau.size(), &rc);
         if (!rc) m->mc_perm = upload(m, mperm.data(), mperm.size(), &rc);
         if (!rc) m->mc_ia = upload(m, mia.data(), mia.size(), &rc);
-        if (!rc) m->mc_ja = upload(m, mja.data(), mja.size(), &rc);
+        if (!rc) m->mc_ja = upload(m, mja.data(), mja.size(), &rc, kIluPad);
         if (!rc) m->mc_iau = upload(m, miau.data(), miau.size(), &rc);
         if (!rc) m->mc_src = upload(m, msrc.data(), msrc.size(), &rc);
-        if (!rc) m->mc_moff = upload(m, mmoff.get(), (size_t)m->nnz, &rc);
-        if (!rc) m->mc_mqq = upload(m, mmqq.get(), (size_t)std::max<int64_t>(mc_nmap, 1), &rc);
         phase("uploads");
         if (!rc) {  // block-SELL patterns of A and of the multicolour factors
             std::vector<int> off;
@@ -822,25 +812,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
     return CFD_OK;
 }
 
-// The natural-order ILU(0) merge map (cfd_mesh::ilu_moff, ilu_mqq), built
-// and uploaded on the first natural-order factorisation: the multicolour
-// factorisation, the sweeps and the Gauss-Seidel solvers do not use it.
-int cfd_ensure_ilu_map(cfd_mesh *m) {
-    if (m->ilu_moff) return CFD_OK;
-    std::unique_ptr<int[]> moff, mqq;
-    int64_t total = 0;
-    if (!build_merge_map_par(m->h_ia.data(), m->h_ja.data(), m->h_iau.data(), m->N, moff, mqq, total))
-        return cfd_set_error(m->ctx, CFD_E_ARG, "ILU(0) merge map too large");
-    int rc = CFD_OK;
-    int *mo = upload(m, moff.get(), (size_t)m->nnz, &rc);
-    int *mq = rc ? nullptr : upload(m, mqq.get(), (size_t)std::max<int64_t>(total, 1), &rc);
-    if (rc) return rc;
-    m->ilu_moff = mo;
-    m->ilu_mqq = mq;
-    m->ilu_nmap = total;
-    return CFD_OK;
-}
-
 extern "C" int64_t cfd_mesh_device_bytes(const cfd_mesh *m) { return m ? m->bytes : 0; }
 
 // Device bytes of a mesh handle after a steady solve with FGMRES(km): every
@@ -860,9 +831,8 @@ extern "C" int64_t cfd_footprint_bytes(int32_t N, int32_t E, int32_t B, int32_t 
     // flags, risk
     bytes += 4 * (n + n + (n + 1) + (n / kSlice + 2) + (n + 1) + 2 * e + 3 * b + 2 * n + (n / 4096 + 1) + 1);
     bytes += nsell * (4 + 4 + 3 * 8);                       // nbr, soff, isx, isy, isz
-    bytes += 4 * ((n + 1) + nnz + n) + 4 * nnz;             // BSR ia, ja, iau; ILU(0) merge offsets
-    bytes += 4 * 8 * nnz;                                   // ILU(0) merge map (<= 8 upper blocks per lower entry)
-    bytes += 4 * (n + (n + 1) + 3 * nnz + n + 2 * n) + 4 * 8 * nnz;  // multicolour pattern, slot map, levels, merge map
+    bytes += 4 * ((n + 1) + nnz + n);                       // BSR ia, ja, iau
+    bytes += 4 * (n + (n + 1) + 2 * nnz + n + 2 * n);       // multicolour pattern, slot map, levels
     bytes += s * 2 * 5 * n;                                 // work vectors of the sweeps
     bytes += 4 * (2 * n + 4 * n + 4 * 11 * lvl);           // level rows and padded slot lists
     bytes += 8 * (1024 * 65 + 4 * 65 + 6) + 4 * 4;         // reduction scratch, eigenvalue bits, flags

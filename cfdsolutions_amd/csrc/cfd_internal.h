@@ -65,6 +65,7 @@ struct LevelSchedule {
     int n12 = 0;
 };
 
+constexpr int kIluPad = 8;       // column entries of the ILU(0) that are read together; ja and mc_ja are padded by as many
 constexpr int kMaxKrylov = 64;   // largest FGMRES restart length
 constexpr int kDotParts = 512;   // partial sums of one Krylov dot product, at most
 // Blocks of 256 threads for a Krylov dot product over n entries: one entry per
@@ -230,11 +231,6 @@ struct cfd_mesh {
     int nnz = 0;
     std::vector<int> h_ia, h_ja, h_iau;
     int *ia = nullptr, *ja = nullptr, *iau = nullptr;
-    // ILU(0) merge map: for lower entry kk = (i, k) of the BSR pattern and the
-    // t-th upper block of row k, ilu_mqq[ilu_moff[kk] + t] is the slot of the
-    // block of row i in the same column, or -1
-    int *ilu_moff = nullptr, *ilu_mqq = nullptr;  // built on first use (cfd_ensure_ilu_map)
-    int64_t ilu_nmap = 0;
     double *a = nullptr, *b = nullptr, *x = nullptr;
     float *af = nullptr;      // FP32 Jacobian (mixed)
     double *lu = nullptr, *dinv = nullptr;
@@ -252,7 +248,6 @@ struct cfd_mesh {
     int *mc_perm = nullptr;                               // [N] original row of each permuted row
     int *mc_ia = nullptr, *mc_ja = nullptr, *mc_iau = nullptr;  // permuted BSR pattern
     int *mc_src = nullptr;                                // [nnz] original slot of each permuted slot
-    int *mc_moff = nullptr, *mc_mqq = nullptr;            // ILU(0) merge map of the permuted pattern
     LevelSchedule mc_lower, mc_upper;
     double *zp = nullptr;  // 2 x [N][5] work vectors of the sweeps (single-launch: handover words)
     float *zpf = nullptr;
@@ -353,7 +348,6 @@ int cfd_ensure_fp32(cfd_mesh *m);
 int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order);  // order: kPatchNodeOrder or kPatchEdgeOrder
 // Rows of each level followed by -1 up to a multiple of w.
 void pad_levels(const std::vector<int> &ptr, const std::vector<int> &rows, int w, std::vector<int> &out);
-int cfd_ensure_ilu_map(cfd_mesh *m);  // natural-order ILU(0) merge map, on first use
 // Whether the residual of these parameters runs the flux-once patch kernel:
 // the fast build at second order, unless CFD_FLUX_ONCE=0 or 1 forces it.
 bool cfd_residual_uses_patches(const cfd_params *p);

@@ -499,124 +499,217 @@ __device__ bool inv5(const double *A, double *Ai) {
     return true;
 }
 
-template <class TM>
-__device__ __forceinline__ void bmul(const TM *A, const TM *B, TM *C) {
-#pragma unroll
-    for (int r = 0; r < 5; r++)
-#pragma unroll
-        for (int c = 0; c < 5; c++) {
-            TM s = TM(0.0);
-#pragma unroll
-            for (int t = 0; t < 5; t++) s += A[5 * r + t] * B[5 * t + c];
-            C[5 * r + c] = s;
-        }
-}
+// ---------------------------------------------------------------------------
+// Block ILU(0), the rows of one level: Saad Alg. 10.4 in block form, the
+// operations of orc_ilu0 on every entry in its order.  Factors in TM; the
+// pivot inverse is computed in FP64.
+//
+// G groups of five lanes share a block row, 12 / G rows to a wavefront: lane r of
+// group g holds row r of the row's blocks g, g + G, ... in registers from the
+// first load to the store (blocks past the kSets of a lane stay in lu, read and
+// written by the lane that owns them).  For the lower block (i, k) every group
+// forms L_ik = A_ik D_k^-1 for itself, finds which of row k's upper columns its own
+// blocks have, and subtracts L_ik U_kj; the updates of one k run side by side.
+// A level's time is that of one row's chain over its lower blocks (narrow
+// levels) or instructions and reads of row k's blocks (wide ones), so narrow
+// levels take one row per wavefront and wide ones three.  With a row's blocks in
+// memory and one group per row, a level of the 48x16x16 mesh took 46 us (FP64,
+// natural order) and 72 us (FP32, multicolour), now 16.6 and 24 us; a colour of
+// 45,625 rows 74 us, now 35; of 815,425 rows 441 us (FP32), now 433, without
+// the pass that copied A into the pattern's order (0.89 ms a factorisation).
+// ---------------------------------------------------------------------------
+// One row per wavefront up to this many rows (four wavefronts per SIMD): at
+// 1,770 rows of a level 24 us against 30 us with three rows, at 5,700 44 us
+// against 35 us (FP32).
+constexpr int kIluNarrowRows = 4096;
+template <int G>
+constexpr int kIluSets = (16 + G - 1) / G;
 
-// ---------------------------------------------------------------------------
-// Block ILU(0), one level: Saad Alg. 10.4 in block form, identical to
-// orc_ilu0.  Factors in TM; the pivot inverse is computed in FP64.
-// ---------------------------------------------------------------------------
-template <class TM>
+template <class TM, int G>
 __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__restrict__ rows,
                                                       const int *__restrict__ ia, const int *__restrict__ ja,
-                                                      const int *__restrict__ iau, const int *__restrict__ moff,
-                                                      const int *__restrict__ mqq, TM *lu, TM *dinv,
+                                                      const int *__restrict__ iau, const int *__restrict__ src,
+                                                      const TM *__restrict__ a, TM *lu, TM *dinv,
                                                       const TM *__restrict__ luk, const TM *__restrict__ dinvk,
                                                       int *flag) {
     // luk / dinvk view the blocks and inverse pivots of rows of earlier
     // levels, which this launch only reads (it writes rows of one level).
-    // 12 rows of 5 lanes per wavefront; lane r owns row r of every block of
-    // its block row, so the products of two 5x5 blocks are split by rows with
-    // the per-entry summation order of bmul.
+    // src: slot of A for each slot of the pattern (NULL: the same).
+    constexpr int NS = kIluSets<G>, RW = 12 / G, W = 5 * G;
+    __shared__ double diag[kBlock / 64][RW][25];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int slot = lane / 5, r = lane - 5 * slot;
-    const int t = (blockIdx.x * (kBlock / 64) + wave) * 12 + slot;
-    const bool active = slot < 12 && t < nrows;
+    const int rs = lane / W, base = rs * W, in = lane - base, g = in / 5, r = in - 5 * g;
+    const int t = (blockIdx.x * (kBlock / 64) + wave) * RW + rs;
+    const bool active = rs < RW && t < nrows;
     const int i = active ? rows[t] : 0;
-    TM drow[5] = {TM(0.0), TM(0.0), TM(0.0), TM(0.0), TM(0.0)};
-    if (active) {
-        // the lanes of a block row hold one row each of every block they
-        // load; a product needs the other rows, which come from the group's
-        // lanes by shuffles (the five lanes of a row run every loop together)
-        const int gbase = lane - r;
-        for (int kk = ia[i]; kk < iau[i]; kk++) {
-            const int k = ja[kk];
-            TM *Lk = lu + 25 * (size_t)kk + 5 * r;
-            const TM *Dk = dinvk + 25 * (size_t)k + 5 * r;
-            TM Lr[5], U[5], Dr[5];
+    const int b0 = active ? ia[i] : 0, n = active ? ia[i + 1] - b0 : 0, nl = active ? iau[i] - b0 : 0;
+    int col[NS], up[NS], nu[NS];  // the blocks' columns; for lower ones the upper blocks of that row
+    TM T[NS][5];
 #pragma unroll
-            for (int q = 0; q < 5; q++) U[q] = Lk[q];
+    for (int s = 0; s < NS; s++) {
+        const int b = s * G + g;
+        col[s] = -1;
+        up[s] = nu[s] = 0;
+        if (b < n) {
+            col[s] = ja[b0 + b];
+            const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
 #pragma unroll
-            for (int c = 0; c < 5; c++) Dr[c] = Dk[c];
-#pragma unroll
-            for (int c = 0; c < 5; c++) {
-                TM s = TM(0.0);
-#pragma unroll
-                for (int q = 0; q < 5; q++) s += U[q] * __shfl(Dr[c], gbase + q, 64);
-                Lr[c] = s;
+            for (int c = 0; c < 5; c++) T[s][c] = A[c];
+            if (b < nl) {
+                up[s] = iau[col[s]] + 1;
+                nu[s] = ia[col[s] + 1] - up[s];
             }
+        }
+    }
+    for (int b = NS * G + g; b < n; b += G) {
+        const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
+        for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+    }
+    for (int l = 0; __any(l < nl); l++) {
+        const int so = l / G, from = base + 5 * (l - so * G);
+        int k = 0, p0 = 0, np = 0;
+        TM Ar[5] = {};
 #pragma unroll
-            for (int c = 0; c < 5; c++) Lk[c] = Lr[c];
-            // upper blocks of row k that meet a block of row i, in ascending
-            // column order (the precomputed merge of the two rows), CH at a
-            // time: their slots, rows and targets are loaded before any
-            // target is updated.  The targets are distinct blocks of row i, so
-            // each update is the one-at-a-time arithmetic.
-            constexpr int CH = sizeof(TM) == 4 ? 8 : 4;
-            const int p0 = iau[k] + 1, np = ia[k + 1] - p0, m0 = moff[kk];
-            for (int t2 = 0; t2 < np; t2 += CH) {
-                int qs[CH];
-                TM ur[CH][5], tv[CH][5];
+        for (int s = 0; s < NS; s++)
+            if (so == s) {
+                k = __shfl(col[s], from, 64);
+                p0 = __shfl(up[s], from, 64);
+                np = __shfl(nu[s], from, 64);
 #pragma unroll
-                for (int u = 0; u < CH; u++) qs[u] = t2 + u < np ? mqq[m0 + t2 + u] : -1;
+                for (int c = 0; c < 5; c++) Ar[c] = __shfl(T[s][c], from + r, 64);
+            }
+        if (so >= NS) {
+            for (int c = 0; c < 5; c++) {
+                if (l < nl && 5 * g == from - base) Ar[c] = lu[25 * (size_t)(b0 + l) + 5 * r + c];
+                Ar[c] = __shfl(Ar[c], from + r, 64);
+            }
+            if (l < nl) {
+                k = ja[b0 + l];
+                p0 = iau[k] + 1;
+                np = ia[k + 1] - p0;
+            }
+        }
+        if (l >= nl) continue;
+        TM D[25], L[5];
 #pragma unroll
-                for (int u = 0; u < CH; u++)
-                    if (qs[u] >= 0) {
-                        const TM *Up = luk + 25 * (size_t)(p0 + t2 + u) + 5 * r;
+        for (int q = 0; q < 25; q++) D[q] = dinvk[25 * (size_t)k + q];
+        // which of row k's upper blocks meets each of this lane's blocks; eight
+        // columns at a time (ja is padded by kIluPad entries)
+        int hit[NS];
 #pragma unroll
-                        for (int c = 0; c < 5; c++) ur[u][c] = Up[c];
+        for (int s = 0; s < NS; s++) hit[s] = -1;
+        for (int c0 = 0; c0 < np; c0 += kIluPad) {
+            int cq[kIluPad];
 #pragma unroll
-                        for (int c = 0; c < 5; c++) tv[u][c] = lu[25 * (size_t)qs[u] + 5 * r + c];
-                    }
+            for (int q = 0; q < kIluPad; q++) cq[q] = ja[p0 + c0 + q];
 #pragma unroll
-                for (int u = 0; u < CH; u++) {
-                    if (qs[u] < 0) continue;
-                    TM *T = lu + 25 * (size_t)qs[u] + 5 * r;
+            for (int q = 0; q < kIluPad; q++)
 #pragma unroll
+                for (int s = 0; s < NS; s++) hit[s] = (cq[q] == col[s]) & (c0 + q < np) ? c0 + q : hit[s];
+        }
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+            TM s = TM(0.0);
+#pragma unroll
+            for (int q = 0; q < 5; q++) s += Ar[q] * D[5 * q + c];
+            L[c] = s;
+        }
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            if (s * G + g == l) {
+#pragma unroll
+                for (int c = 0; c < 5; c++) T[s][c] = L[c];
+            } else if (hit[s] >= 0) {
+                const TM *U = luk + 25 * (size_t)(p0 + hit[s]);
+                TM u[25];
+#pragma unroll
+                for (int q = 0; q < 25; q++) u[q] = U[q];
+#pragma unroll
+                for (int c = 0; c < 5; c++) {
+                    TM v = TM(0.0);
+#pragma unroll
+                    for (int q = 0; q < 5; q++) v += L[q] * u[5 * q + c];
+                    T[s][c] = T[s][c] - v;
+                }
+            }
+        }
+        for (int b = NS * G + g; b < n; b += G) {
+            TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
+            if (b == l) {
+                for (int c = 0; c < 5; c++) B[c] = L[c];
+            } else if (b > l) {
+                const int cb = ja[b0 + b];
+                for (int q = 0; q < np; q++) {
+                    if (ja[p0 + q] != cb) continue;
+                    const TM *U = luk + 25 * (size_t)(p0 + q);
                     for (int c = 0; c < 5; c++) {
-                        TM s = TM(0.0);
-#pragma unroll
-                        for (int q = 0; q < 5; q++) s += Lr[q] * __shfl(ur[u][c], gbase + q, 64);
-                        T[c] = tv[u][c] - s;
+                        TM v = TM(0.0);
+                        for (int z = 0; z < 5; z++) v += L[z] * U[5 * z + c];
+                        B[c] = B[c] - v;
                     }
                 }
             }
         }
-        const TM *Dp = lu + 25 * (size_t)iau[i] + 5 * r;
-#pragma unroll
-        for (int c = 0; c < 5; c++) drow[c] = Dp[c];
     }
-    // every lane of the row gathers the diagonal block and inverts it (FP64)
-    const int base = lane - r;
-    double Dg[25], Di[25];
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const int b = s * G + g;
+        if (b >= n) continue;
+        TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+            B[c] = T[s][c];
+            if (b == nl) diag[wave][rs][5 * r + c] = (double)T[s][c];
+        }
+    }
+    for (int b = NS * G + g; b < n; b += G)
+        if (b == nl)
+            for (int c = 0; c < 5; c++) diag[wave][rs][5 * r + c] = (double)lu[25 * (size_t)(b0 + b) + 5 * r + c];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // Gauss-Jordan inverse of inv5 with one column of [D | I] to a lane (the
+    // row's first ten lanes): the same operations on every entry
+    double m[5];
 #pragma unroll
     for (int q = 0; q < 5; q++)
+        m[q] = !active ? 0.0 : in < 5 ? diag[wave][rs][5 * q + in] : (in - 5 == q ? 1.0 : 0.0);
+    bool singular = false;
 #pragma unroll
-        for (int c = 0; c < 5; c++) Dg[5 * q + c] = (double)__shfl(drow[c], base + q, 64);
-    if (!active) return;
-    if (!inv5(Dg, Di)) {
-        if (r == 0) atomicAdd(flag + 2, 1);
-        for (int q = 0; q < 25; q++) Di[q] = 0.0;
+    for (int c = 0; c < 5; c++) {
+        double p[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) p[q] = __shfl(m[q], base + c, 64);
+        int piv = c;
+        double best = fabs(p[c]);
+#pragma unroll
+        for (int q = c + 1; q < 5; q++) {
+            const double v = fabs(p[q]);
+            if (v > best) {
+                piv = q;
+                best = v;
+            }
+        }
+#pragma unroll
+        for (int q = c + 1; q < 5; q++) {
+            const bool sw = piv == q;
+            const double x = m[c], y = p[c];
+            m[c] = sw ? m[q] : x;
+            m[q] = sw ? x : m[q];
+            p[c] = sw ? p[q] : y;
+            p[q] = sw ? y : p[q];
+        }
+        singular = singular || p[c] == 0.0;
+        m[c] = m[c] / p[c];
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+            if (q != c) m[q] = m[q] - p[q] * m[c];
     }
-    // row r of the inverse, picked with selects (an index by r would put Di in
-    // scratch memory)
-    double dr[5] = {Di[0], Di[1], Di[2], Di[3], Di[4]};
+    if (!active) return;
+    if (singular && in == 0) atomicAdd(flag + 2, 1);
+    if (in >= 5 && in < 10)
 #pragma unroll
-    for (int rr = 1; rr < 5; rr++)
-#pragma unroll
-        for (int c = 0; c < 5; c++) dr[c] = r == rr ? Di[5 * rr + c] : dr[c];
-#pragma unroll
-    for (int c = 0; c < 5; c++) dinv[25 * (size_t)i + 5 * r + c] = (TM)dr[c];
+        for (int q = 0; q < 5; q++) dinv[25 * (size_t)i + 5 * q + in - 5] = singular ? TM(0.0) : (TM)m[q];
 }
 
 // Inverse diagonal blocks (block-Jacobi).
@@ -887,16 +980,6 @@ __global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_trsv_flow(int nslots
             }
         }
         if (i >= 0) flow_store(cur + 5 * (size_t)i + r, y);
-    }
-}
-
-// Blocks of the matrix in multicolour order: dst[s] = src[map[s]].
-template <class TS, class TD>
-__global__ __launch_bounds__(kBlock) void k_gather_blocks(size_t nnz, const int *__restrict__ map,
-                                                          const TS *__restrict__ src, TD *__restrict__ dst) {
-    for (size_t t = blockIdx.x * (size_t)kBlock + threadIdx.x; t < 25 * nnz; t += (size_t)gridDim.x * kBlock) {
-        const size_t s = t / 25, q = t - 25 * s;
-        dst[t] = (TD)src[25 * (size_t)map[s] + q];
     }
 }
 
@@ -1959,17 +2042,27 @@ const double *bsr_a<double>(cfd_mesh *m) { return m->a; }
 template <>
 const float *bsr_a<float>(cfd_mesh *m) { return m->af; }
 
+// ILU(0) factors of A's blocks (in the pattern's order through src), a launch
+// per level.
+template <class TM>
+void ilu0_levels(cfd_mesh *m, const LevelSchedule &ls, const int *ia, const int *ja, const int *iau, const int *src,
+                 const TM *a, TM *lu, TM *dinv) {
+    for (int l = 0; l < ls.nlevels; l++) {
+        const int b0 = ls.ptr[l], nr = ls.ptr[l + 1] - b0;
+#define CFD_ILU(G)                                                                                                    \
+    hipLaunchKernelGGL((k_ilu0_level<TM, G>), dim3((nr + 4 * (12 / G) - 1) / (4 * (12 / G))), dim3(kBlock), 0,         \
+                       m->stream, nr, ls.rows + b0, ia, ja, iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, \
+                       m->flag)
+        if (nr <= kIluNarrowRows) CFD_ILU(12);
+        else CFD_ILU(4);
+#undef CFD_ILU
+    }
+}
+
 template <class TM>
 int build_prec(cfd_mesh *m, int kind, const TM *a, TM *lu, TM *dinv, bool half) {
     if (kind == CFD_PREC_ILU0_MC) {
-        hipLaunchKernelGGL((k_gather_blocks<TM, TM>), dim3(grid_cap(25 * (size_t)m->nnz, 8192)), dim3(kBlock), 0,
-                           m->stream, (size_t)m->nnz, m->mc_src, a, lu);
-        for (int l = 0; l < m->mc_lower.nlevels; l++) {
-            const int b0 = m->mc_lower.ptr[l], nr = m->mc_lower.ptr[l + 1] - b0;
-            hipLaunchKernelGGL(k_ilu0_level<TM>, dim3((nr + 47) / 48), dim3(kBlock), 0, m->stream, nr,
-                               m->mc_lower.rows + b0, m->mc_ia, m->mc_ja, m->mc_iau, m->mc_moff, m->mc_mqq, lu, dinv,
-                               lu, dinv, m->flag);
-        }
+        ilu0_levels(m, m->mc_lower, m->mc_ia, m->mc_ja, m->mc_iau, m->mc_src, a, lu, dinv);
         // block-SELL copies for the sweeps, FP16 with mixed = 2
         if constexpr (std::is_same<TM, float>::value) {
             if (half) {
@@ -1990,15 +2083,7 @@ int build_prec(cfd_mesh *m, int kind, const TM *a, TM *lu, TM *dinv, bool half) 
                                (size_t)m->N, nullptr, dinv, SellVals<TM>::d(m));
         }
     } else if (kind == CFD_PREC_ILU0) {
-        const int rc = cfd_ensure_ilu_map(m);
-        if (rc) return rc;
-        CFD_HIP(m, hipMemcpyAsync(lu, a, sizeof(TM) * 25 * (size_t)m->nnz, hipMemcpyDeviceToDevice, m->stream));
-        for (int l = 0; l < m->lower.nlevels; l++) {
-            const int b0 = m->lower.ptr[l], nr = m->lower.ptr[l + 1] - b0;
-            hipLaunchKernelGGL(k_ilu0_level<TM>, dim3((nr + 47) / 48), dim3(kBlock), 0, m->stream, nr,
-                               m->lower.rows + b0, m->ia, m->ja, m->iau, m->ilu_moff, m->ilu_mqq, lu, dinv, lu, dinv,
-                               m->flag);
-        }
+        ilu0_levels(m, m->lower, m->ia, m->ja, m->iau, nullptr, a, lu, dinv);
     } else if (kind == CFD_PREC_BJACOBI) {
         hipLaunchKernelGGL((k_block_inv<TM, TM>), dim3((m->N + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream,
                            m->N, m->iau, a, dinv, m->flag);

@@ -132,3 +132,51 @@ def test_a_right_hand_side_of_unset_words_is_a_nan_like_any_other(ctx, solver):
     assert np.isnan(x).any()
     np.testing.assert_array_equal(dm.get(cfd.FIELD_X), x)
     dm.close()
+
+
+def multicolour(ia, ja, iau, a, b):
+    """The system with its rows in the order of a greedy colouring (in row order), ties by row."""
+    n = ia.size - 1
+    colour = np.full(n, -1)
+    for i in range(n):
+        used = set(colour[ja[ia[i]:ia[i + 1]]])
+        c = 0
+        while c in used:
+            c += 1
+        colour[i] = c
+    perm = np.argsort(colour, kind="stable")
+    inv = np.empty(n, np.int64)
+    inv[perm] = np.arange(n)
+    row = inv[np.repeat(np.arange(n), np.diff(ia))]
+    at = np.lexsort((inv[ja], row))
+    pia = np.concatenate([[0], np.cumsum(np.diff(ia)[perm])]).astype(np.int32)
+    pja = inv[ja][at].astype(np.int32)
+    piau = np.flatnonzero(pja == row[at]).astype(np.int32)
+    return perm, pia, pja, piau, a[at], b[perm]
+
+
+@pytest.mark.parametrize("kind,n,precond", [
+    ("chain", 30, cfd.PREC_ILU0), ("sparse", 64, cfd.PREC_ILU0), ("random", 1300, cfd.PREC_ILU0),
+    ("hub", 173, cfd.PREC_ILU0),  # a row of 81 blocks, 40 of them lower: more than a lane group keeps in registers
+    ("hub", 173, cfd.PREC_ILU0_MC),
+    ("hub", 30000, cfd.PREC_ILU0_MC),  # colours of more rows than the one-row-per-wavefront kernel takes
+    ("random", 30000, cfd.PREC_ILU0_MC)])
+def test_ilu_factors_equal_oracle(ctx, kind, n, precond):
+    """One FGMRES step without restarts gives x = y M^-1 b: its direction is the oracle's preconditioned b.  Each entry
+    of b / ||b|| is rounded once, and the systems' inverses amplify that little (dominance 3 per neighbour against row
+    sums of at most 5 half on average): 64 roundings bound it with room."""
+    print("ilu factors", kind, n, precond, flush=True)
+    dm, ia, ja, iau, a, b = system(ctx, kind, n)
+    dm.linsolve(precond=precond, krylov_m=1, max_restarts=0, rtol=1e-30)
+    x = dm.get(cfd.FIELD_X)
+    dm.close()
+    if precond == cfd.PREC_ILU0_MC:
+        perm, ia, ja, iau, a, b = multicolour(ia, ja, iau, a, b)
+        x = x[perm]
+    lu, dinv, rc = orc.ilu0(ia, ja, iau, a)
+    assert rc == 0
+    z = orc.ilu0_apply(ia, ja, iau, lu, dinv, b).reshape(-1, 5)
+    x, z = x / np.linalg.norm(x), z / np.linalg.norm(z)
+    if np.vdot(x, z) < 0:
+        x = -x
+    assert np.linalg.norm(x - z) <= 64 * np.finfo(float).eps
