@@ -844,6 +844,19 @@ template <class T>
 __device__ __forceinline__ void flow_unset(T *p) {
     st_coh(reinterpret_cast<typename FlowWord<T>::U *>(p), FlowWord<T>::unset);
 }
+// The value of word p, of which v has been read already.
+template <class T>
+__device__ __forceinline__ T flow_wait(const T *p, typename FlowWord<T>::U v, int *flag) {
+    for (int it = 0; v == FlowWord<T>::unset; it++) {
+        if (it >= kSpinMax || ((it & 255) == 255 && ld_coh(flag + 3) != 0)) {
+            atomicOr(flag + 3, 1);
+            break;
+        }
+        v = flow_load(p);
+    }
+    return __builtin_bit_cast(T, v);
+}
+
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_flow_unset(size_t n, T *x) {
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) flow_unset(x + i);
@@ -1586,240 +1599,230 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_init(int N, const double *b, d
 // ---------------------------------------------------------------------------
 // Krylov vector kernels (deterministic reductions)
 // ---------------------------------------------------------------------------
-// part[blk][k] = sum over the block's elements of V_k . w, k < nv
-// Partial dot products of w with V_0..V_{nv-1} over this block's strided
-// elements [o + i0, o + n) (step `stride`), stored in part[0..nv).  The
-// products are accumulated in register chunks of 8 vectors (w is re-read per
-// chunk): each (thread, vector) sum visits the same elements in the same order
-// and each vector goes through the same block tree, whatever the chunking.
-template <class TV, bool DEEP = false>
-__device__ __forceinline__ void block_dots(size_t o, size_t i0, size_t n, size_t stride, int nv,
-                                           const TV *__restrict__ V, size_t ld, const TV *__restrict__ w,
-                                           double *__restrict__ part) {
-    __shared__ double wsum[8][kBlock / 64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int k0 = 0; k0 < nv; k0 += 8) {
-        double acc[8];
-#pragma unroll
-        for (int kk = 0; kk < 8; kk++) acc[kk] = 0.0;
-        // DEEP: four strides at a time, all their loads issued before the
-        // products are added in the same order as one stride at a time (for
-        // threads with many strides to walk; it costs registers, so short
-        // walks keep the single-stride loop and its occupancy)
-        size_t i = i0;
-        for (; DEEP && i + 3 * stride < n; i += 4 * stride) {
-            TV wv[4], vv[4][8];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                wv[u] = w[o + i + u * stride];
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (k0 + kk < nv) vv[u][kk] = V[ld * (k0 + kk) + o + i + u * stride];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const double wi = (double)wv[u];
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (k0 + kk < nv) acc[kk] += (double)vv[u][kk] * wi;
-            }
-        }
-        for (; i < n; i += stride) {
-            const double wi = (double)w[o + i];
-#pragma unroll
-            for (int kk = 0; kk < 8; kk++)
-                if (k0 + kk < nv) acc[kk] += (double)V[ld * (k0 + kk) + o + i] * wi;
-        }
-        // block sum: a butterfly within each wavefront (every lane ends with
-        // the same value), then the four wavefront sums in order
-#pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
-            if (k0 + kk >= nv) break;
-            double v = acc[kk];
-#pragma unroll
-            for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh, 64);
-            if (lane == 0) wsum[kk][wave] = v;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (int kk = 0; kk < 8 && k0 + kk < nv; kk++)
-                part[k0 + kk] = ((wsum[kk][0] + wsum[kk][1]) + wsum[kk][2]) + wsum[kk][3];
-        __syncthreads();
-    }
+// Sum over the wavefront, in every lane: the butterfly 32, 16, 8, 4, 2, 1.  Its
+// last four steps stay within rows of 16 lanes whose values repeat with the
+// step's period, so a rotation brings each lane its partner's value without
+// the LDS crossbar.
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + N, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + N, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v += __shfl_xor(v, 32, 64);
+    v += __shfl_xor(v, 16, 64);
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    v += row_ror<1>(v);
+    return v;
 }
 
-template <class TV, bool DEEP>
-__global__ __launch_bounds__(kBlock) void k_mdot(size_t n, int nv, const TV *__restrict__ V, size_t ld,
-                                                 const TV *__restrict__ w, double *__restrict__ part) {
-    block_dots<TV, DEEP>(0, blockIdx.x * (size_t)kBlock + threadIdx.x, n, (size_t)gridDim.x * kBlock, nv, V, ld, w,
-                   part + (size_t)blockIdx.x * (kMaxKrylov + 1));
+// wave_sum of four values at once: the steps 32 and 16 exchange halves of two
+// values' lanes, so that one addition serves both and the four sums end in one
+// register, in the rows of 16 lanes: value 0 in row 0, 2 in 1, 1 in 2, 3 in 3.
+__device__ __forceinline__ double swap_add32(double a, double b) {
+    const long long x = __builtin_bit_cast(long long, a), y = __builtin_bit_cast(long long, b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+    const long long x = __builtin_bit_cast(long long, a), y = __builtin_bit_cast(long long, b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double wave_sum4(double v0, double v1, double v2, double v3) {
+    double v = swap_add16(swap_add32(v0, v1), swap_add32(v2, v3));
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    v += row_ror<1>(v);
+    return v;
 }
 
-// Sum of the partials of dot k (block k): lane l adds partials l, l+64, ...
-// in order, then the 64 lane sums are combined by a fixed butterfly.
-__device__ __forceinline__ double wave_sum_parts(const double *part, int p0, int np, int k) {
-    const int lane = threadIdx.x;
-    double s = 0.0;
-    for (int p = lane; p < np; p += 64) s += part[(size_t)(p0 + p) * (kMaxKrylov + 1) + k];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    return s;
-}
+// Gram-Schmidt passes over the entries o + i0, o + i0 + stride, ... < o + n of a
+// thread, in that order:
+//   kDots        acc[k] += V_ki w_i
+//   kUpdateDots  w_i -= h_k V_ki for k ascending (as CGS in the oracle), rounded
+//                once to TV and stored; then acc[k] += V_ki w_i
+//   kUpdateNorm  the same update; then acc[0] += w_i w_i
+// U entries go together, so that their loads overlap: a thread takes one round
+// trip to memory for U of its entries.
+// kUpdateDots keeps the entries' V values in registers between the update and
+// the products: a grid has at most kDotParts blocks, two wavefronts per SIMD,
+// so registers are free (rereading them from the caches took 166 us at 24
+// vectors of 4.08M FP32 entries, this 130 us with the final sums).
+enum GsMode { kDots, kUpdateDots, kUpdateNorm };
 
-__global__ __launch_bounds__(64) void k_mdot_final(int nparts, int nv, const double *part, double *out) {
-    const int k = blockIdx.x;
-    const double s = wave_sum_parts(part, 0, nparts, k);
-    if (threadIdx.x == 0) out[k] = s;
-}
-
-// U entries i, i + stride, ... of the pass: their updates (the loads of 8
-// vectors for all U entries issued together), stores, and products.
-// hold (LDS, [NVMAX][kBlock], one entry per call): the entry's V values are
-// kept there between the update and the products instead of being read again
-// from memory (the same values).
-template <class TV, int NVMAX, bool NORM, int U, bool LHOLD = false>
-__device__ __forceinline__ void cgs_entries(size_t o, size_t i, size_t stride, int nv, const TV *__restrict__ V,
-                                            size_t ld, const double *h, TV *__restrict__ w, double *acc,
-                                            TV *hold = nullptr) {
-    static_assert(!LHOLD || (U == 1 && !NORM), "hold: one entry, dots pass");
-    constexpr int NC = (NVMAX + 7) / 8;
+template <class TV, int NVMAX, GsMode M, int U>
+__device__ __forceinline__ void gs_entries(size_t o, size_t i, size_t stride, int nv, const TV *__restrict__ V,
+                                           size_t ld, const double *__restrict__ h, TV *__restrict__ w, double *acc) {
+    constexpr int NC = (NVMAX + 7) / 8, HOLD = M == kUpdateDots ? NVMAX : 8;
     double wi[U];
+    TV vv[U][HOLD];
 #pragma unroll
     for (int u = 0; u < U; u++) wi[u] = (double)w[o + i + u * stride];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        if (8 * c < nv) {
-            TV vv[U][8];
+        if (8 * c >= nv) continue;
 #pragma unroll
-            for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (8 * c + kk < nv) vv[u][kk] = V[ld * (8 * c + kk) + o + i + u * stride];
+            for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
+                if (k < nv) vv[u][M == kUpdateDots ? k : k - 8 * c] = V[ld * k + o + i + u * stride];
+        if (M == kUpdateDots) continue;
 #pragma unroll
-            for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (8 * c + kk < nv) wi[u] = wi[u] - h[8 * c + kk] * (double)vv[u][kk];
-            if (LHOLD) {
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (8 * c + kk < nv) hold[(8 * c + kk) * kBlock + threadIdx.x] = vv[0][kk];
-            }
-        }
+            for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
+                if (k < nv) {
+                    if (M == kDots) acc[k] += (double)vv[u][k - 8 * c] * wi[u];
+                    else wi[u] = wi[u] - h[k] * (double)vv[u][k - 8 * c];
+                }
     }
-    double wd[U];
+    if (M == kDots) return;
+    if (M == kUpdateDots) {
+#pragma unroll
+        for (int k = 0; k < NVMAX; k++)
+            if (k < nv) {
+                const double hk = h[k];
+#pragma unroll
+                for (int u = 0; u < U; u++) wi[u] = wi[u] - hk * (double)vv[u][M == kUpdateDots ? k : 0];
+            }
+    }
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const TV wt = (TV)wi[u];
         w[o + i + u * stride] = wt;
-        wd[u] = (double)wt;
+        wi[u] = (double)wt;
+        if (M == kUpdateNorm) acc[0] += wi[u] * wi[u];
     }
-    if (NORM) {
+    if (M == kUpdateDots) {
+        // (the empty asm: an FP32 value is converted again rather than kept in
+        // FP64 from the update on, which would double its registers)
+        if (sizeof(TV) == 4) {
 #pragma unroll
-        for (int u = 0; u < U; u++) acc[0] += wd[u] * wd[u];
-        return;
-    }
-    // read V again rather than hold its values across the update
-    asm volatile("" ::: "memory");
+            for (int k = 0; k < NVMAX; k++)
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-        if (8 * c < nv) {
-            TV vv[U][8];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (8 * c + kk < nv)
-                        vv[u][kk] = LHOLD ? hold[(8 * c + kk) * kBlock + threadIdx.x]
-                                          : V[ld * (8 * c + kk) + o + i + u * stride];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    if (8 * c + kk < nv) acc[8 * c + kk] += (double)vv[u][kk] * wd[u];
+                for (int u = 0; u < U; u++)
+                    if (k < nv) asm volatile("" : "+v"(vv[u][M == kUpdateDots ? k : 0]));
         }
+#pragma unroll
+        for (int k = 0; k < NVMAX; k++)
+            if (k < nv) {
+#pragma unroll
+                for (int u = 0; u < U; u++) acc[k] += (double)vv[u][M == kUpdateDots ? k : 0] * wi[u];
+            }
     }
 }
 
-// One fused CGS pass over this thread's strided entries of [o + i0, o + n)
-// (the entries block_dots visits, in its order): each entry first loses its
-// projections on V_0..V_{nv-1} (w_i -= h_k V_ki for k ascending, as CGS in
-// the oracle, rounded once to TV) and is stored; then its products with
-// V_0..V_{nv-1} (or, NORM, its square) are added to the partial sums, which
-// go through block_dots' block tree into part[0..nv) (part[0]).  The results
-// are those of the update over all entries followed by block_dots, bit for
-// bit, with one pass over w instead of three and the second read of each
-// V_ki served by the cache.  DEEP (threads with many entries to walk):
-// entries go four at a time (two for long bases) while four remain, so their
-// loads overlap; it costs registers, so short walks take one entry at a time.
-// h: nv coefficients in LDS; nv <= NVMAX.
-template <class TV, int NVMAX, bool NORM, bool DEEP, bool LHOLD = false>
-__device__ __forceinline__ void block_cgs_pass(size_t o, size_t i0, size_t n, size_t stride, int nv,
-                                               const TV *__restrict__ V, size_t ld, const double *h,
-                                               TV *__restrict__ w, double *__restrict__ part) {
-    static_assert(!LHOLD || (!DEEP && !NORM), "hold: one entry at a time, dots pass");
-    constexpr int NA = NORM ? 1 : NVMAX;
-    constexpr int U = !DEEP ? 1 : NVMAX > 24 ? 2 : 4;
+// Where the sums of one partition (a mesh, or a case of a union) go.
+struct GsSums {
+    double *words;  // [nd][P] partial sums of its P blocks, handed over as in k_trsv_flow; unset between launches
+    double *out;    // [nd]
+    double *host;   // [nd] the same in pinned host memory
+};
+
+// Block b of the P of a partition: the pass over its entries, then its partial
+// sums (a butterfly within each wavefront, the four wavefront sums in order)
+// into the words of dot k, and in the wavefronts of the last blocks the final
+// sums: lane l adds partials l, l + 64, ... in order, then the butterfly.  They
+// wait only for blocks dispatched before them or with them.  (A launch of its
+// own for the final sums took 4-5 us, three times per Arnoldi step, and a copy
+// of the sums to the host 3 us.)
+template <class TV, int NVMAX, GsMode M, int U>
+__device__ __forceinline__ void gs_block(size_t o, int b, int P, size_t n, int nv, const TV *__restrict__ V, size_t ld,
+                                         const double *__restrict__ h, TV *__restrict__ w, const GsSums &g,
+                                         int *flag) {
+    constexpr int NA = M == kUpdateNorm ? 1 : NVMAX;
     __shared__ double wsum[NA][kBlock / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t stride = (size_t)P * kBlock;
     double acc[NA];
 #pragma unroll
     for (int k = 0; k < NA; k++) acc[k] = 0.0;
-    size_t i = i0;
+    size_t i = b * (size_t)kBlock + threadIdx.x;
     if (U > 1)
         for (; i + (U - 1) * stride < n; i += U * stride)
-            cgs_entries<TV, NVMAX, NORM, U>(o, i, stride, nv, V, ld, h, w, acc);
-    if (LHOLD) {
-        __shared__ TV hold[LHOLD ? NVMAX : 1][kBlock];
-        for (; i < n; i += stride) cgs_entries<TV, NVMAX, NORM, 1, LHOLD>(o, i, stride, nv, V, ld, h, w, acc, &hold[0][0]);
+            gs_entries<TV, NVMAX, M, U>(o, i, stride, nv, V, ld, h, w, acc);
+    for (; i < n; i += stride) gs_entries<TV, NVMAX, M, 1>(o, i, stride, nv, V, ld, h, w, acc);
+    const int nd = M == kUpdateNorm ? 1 : nv;
+    if (NA == 1) {
+        const double v = wave_sum(acc[0]);
+        if (lane == 0) wsum[0][wave] = v;
     } else {
-        for (; i < n; i += stride) cgs_entries<TV, NVMAX, NORM, 1>(o, i, stride, nv, V, ld, h, w, acc);
+        const int row = lane >> 4, at = row == 1 ? 2 : row == 2 ? 1 : row;
+#pragma unroll
+        for (int k = 0; k < NA; k += 4)
+            if (k < nd) {
+                const double v = wave_sum4(acc[k], k + 1 < NA ? acc[k + 1 < NA ? k + 1 : 0] : 0.0,
+                                           k + 2 < NA ? acc[k + 2 < NA ? k + 2 : 0] : 0.0,
+                                           k + 3 < NA ? acc[k + 3 < NA ? k + 3 : 0] : 0.0);
+                if ((lane & 15) == 0 && k + at < nd) wsum[k + at][wave] = v;
+            }
     }
-    const int nd = NORM ? 1 : nv;
+    __syncthreads();
+    for (int k = threadIdx.x; k < nd; k += kBlock)
+        flow_store(g.words + (size_t)k * P + b, ((wsum[k][0] + wsum[k][1]) + wsum[k][2]) + wsum[k][3]);
+    for (int k = (P - 1 - b) * (kBlock / 64) + wave; k < nd; k += P * (kBlock / 64)) {
+        double *p = g.words + (size_t)k * P;
+        double s = 0.0;
+        for (int q = lane; q < P; q += 64 * 8) {
+            unsigned long long v[8];
 #pragma unroll
-    for (int k = 0; k < NA; k++) {
-        if (k < nd) {
-            double v = acc[k];
+            for (int u = 0; u < 8; u++)
+                if (q + 64 * u < P) v[u] = flow_load(p + q + 64 * u);
 #pragma unroll
-            for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh, 64);
-            if (lane == 0) wsum[k][wave] = v;
+            for (int u = 0; u < 8; u++)
+                if (q + 64 * u < P) {
+                    s += flow_wait(p + q + 64 * u, v[u], flag);
+                    flow_unset(p + q + 64 * u);
+                }
+        }
+        s = wave_sum(s);
+        if (lane == 0) {
+            g.out[k] = s;
+            g.host[k] = s;
         }
     }
-    __syncthreads();
-    for (int k = threadIdx.x; k < nd; k += kBlock) part[k] = ((wsum[k][0] + wsum[k][1]) + wsum[k][2]) + wsum[k][3];
 }
 
-// w -= V h, then the dots of w with V_0..V_{nv-1} (DOTS) or with itself
-// (NORM) into part[block][..] (grid: dot_parts(n) blocks, as k_mdot).
-template <class TV, int NVMAX, bool NORM, bool DEEP>
-__global__ __launch_bounds__(kBlock) void k_cgs_pass(size_t n, int nv, const TV *__restrict__ V, size_t ld,
-                                                     const double *__restrict__ hdev, TV *__restrict__ w,
-                                                     double *__restrict__ part) {
-    __shared__ double h[kMaxKrylov + 1];
-    for (int k = threadIdx.x; k < nv; k += kBlock) h[k] = hdev[k];
-    __syncthreads();
-    block_cgs_pass<TV, NVMAX, NORM, DEEP>(0, blockIdx.x * (size_t)kBlock + threadIdx.x, n, (size_t)gridDim.x * kBlock, nv,
-                                    V, ld, h, w, part + (size_t)blockIdx.x * (kMaxKrylov + 1));
+template <class TV, int NVMAX, GsMode M, int U>
+__global__ __launch_bounds__(kBlock, 2) void k_gs(size_t n, int nv, const TV *__restrict__ V, size_t ld,
+                                               const double *__restrict__ h, TV *__restrict__ w, GsSums g, int *flag) {
+    gs_block<TV, NVMAX, M, U>(0, blockIdx.x, gridDim.x, n, nv, V, ld, h, w, g, flag);
 }
 
-// The same over a union of cases: block (c, b) of the segment map updates
-// and reduces case c's range with case c's coefficients out[c][slot..].
-template <class TV, int NVMAX, bool NORM>
-__global__ __launch_bounds__(kBlock) void k_cgs_pass_seg(const int2 *__restrict__ blk, const int *__restrict__ first,
-                                                         const int *__restrict__ off, const int *__restrict__ len,
-                                                         int nv, const TV *__restrict__ V, size_t ld,
-                                                         const double *__restrict__ out, int slot, TV *__restrict__ w,
-                                                         double *__restrict__ part) {
+// The same over a union of cases: block (c, b) of the segment map takes case
+// c's range with its coefficients h[c] and leaves the sums in out[c] (rows of
+// kBOut).  Blocks of a case are consecutive, and its last ones add up
+// its partials, so however many cases there are, they wait for few.
+template <class TV, int NVMAX, GsMode M>
+__global__ __launch_bounds__(kBlock, 2) void k_gs_seg(const int2 *__restrict__ blk, const int *__restrict__ first,
+                                                      const int *__restrict__ off, const int *__restrict__ len, int nv,
+                                                      const TV *__restrict__ V, size_t ld,
+                                                      const double *__restrict__ h, double *out, double *host,
+                                                      TV *__restrict__ w, double *words, int *flag) {
     const int2 cb = blk[blockIdx.x];
-    __shared__ double h[kMaxKrylov + 1];
-    for (int k = threadIdx.x; k < nv; k += kBlock) h[k] = out[(size_t)cb.x * kBOut + slot + k];
-    __syncthreads();
-    const size_t P = (size_t)(first[cb.x + 1] - first[cb.x]);
-    // (the FP32 dots pass with up to 41 vectors keeps each entry's V values
-    // in LDS: a case's blocks give each thread one or a few entries)
-    constexpr bool hold = !NORM && sizeof(TV) == 4 && NVMAX <= 41;
-    block_cgs_pass<TV, NVMAX, NORM, false, hold>((size_t)off[cb.x], cb.y * (size_t)kBlock + threadIdx.x,
-                                                 (size_t)len[cb.x], P * kBlock, nv, V, ld, h, w,
-                                                 part + (size_t)blockIdx.x * (kMaxKrylov + 1));
+    const int f = first[cb.x], P = first[cb.x + 1] - f;
+    const size_t oc = (size_t)cb.x * kBOut;
+    const GsSums g{words + (size_t)f * (kMaxKrylov + 1), out + oc, host + oc};
+    gs_block<TV, NVMAX, M, 1>((size_t)off[cb.x], cb.y, P, (size_t)len[cb.x], nv, V, ld, h + oc, w, g, flag);
+}
+
+// Final sums of k_vsum_partial: dot k (block k) adds partials as gs_block does.
+__global__ __launch_bounds__(64) void k_mdot_final(int nparts, int nv, const double *part, double *out) {
+    const int k = blockIdx.x;
+    double s = 0.0;
+    for (int p = threadIdx.x; p < nparts; p += 64) s += part[(size_t)p * (kMaxKrylov + 1) + k];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) out[k] = s;
 }
 
 // dst = src * (1/scale) with scale read from the device (scale = out[idx])
@@ -1871,29 +1874,6 @@ __global__ void k_fill(size_t n, double v, double *x) {
 }
 
 // ---- union of independent cases (batched solves) ------------------------
-// Per-case dot products: block (c, b) of the segment map reduces over case
-// c's range with the stride of an nb[c]-block launch on that case alone, so
-// each case's dots are bit-identical to k_mdot on the case by itself.
-template <class TV>
-__global__ __launch_bounds__(kBlock) void k_mdot_seg(const int2 *__restrict__ blk, const int *__restrict__ first,
-                                                     const int *__restrict__ off, const int *__restrict__ len, int nv,
-                                                     const TV *__restrict__ V, size_t ld, const TV *__restrict__ w,
-                                                     double *__restrict__ part) {
-    const int2 cb = blk[blockIdx.x];
-    const size_t P = (size_t)(first[cb.x + 1] - first[cb.x]);
-    block_dots<TV>((size_t)off[cb.x], cb.y * (size_t)kBlock + threadIdx.x, (size_t)len[cb.x], P * kBlock, nv, V, ld,
-                   w, part + (size_t)blockIdx.x * (kMaxKrylov + 1));
-}
-
-// out[c][slot + k] = sum of case c's partials, combined as k_mdot_final
-// (grid: dots x cases)
-__global__ __launch_bounds__(64) void k_mdot_seg_final(const int *first, int nv, const double *part, double *out,
-                                                       int slot) {
-    const int k = blockIdx.x, c = blockIdx.y;
-    const double s = wave_sum_parts(part, first[c], first[c + 1] - first[c], k);
-    if (threadIdx.x == 0) out[(size_t)c * kBOut + slot + k] = s;
-}
-
 // dst = src / sqrt(out[c][slot]) (Arnoldi normalisation, per case)
 template <class TS, class TD>
 __global__ __launch_bounds__(kBlock) void k_scale_dev_seg(size_t n, const int *__restrict__ ecase, const TS *src,
@@ -2202,44 +2182,40 @@ void apply_prec(cfd_mesh *m, int kind, const TM *lu, const TM *dinv, const TV *r
     }
 }
 
-// dots of w with V_0..V_{nv-1}; results in m->redout + off (device)
-template <class TV>
-void mdot(cfd_mesh *m, int nv, const TV *V, size_t ld, const TV *w, int off) {
-    const size_t L = 5 * (size_t)m->N;
-    const int np = dot_parts(L);
-    if (L >= 4 * (size_t)np * kBlock)  // each thread walks four strides or more
-        hipLaunchKernelGGL((k_mdot<TV, true>), dim3(np), dim3(kBlock), 0, m->stream, L, nv, V, ld, w, m->red);
-    else
-        hipLaunchKernelGGL((k_mdot<TV, false>), dim3(np), dim3(kBlock), 0, m->stream, L, nv, V, ld, w, m->red);
-    hipLaunchKernelGGL(k_mdot_final, dim3(nv), dim3(64), 0, m->stream, np, nv, m->red, m->redout + off);
+// Entries that a thread of k_gs takes together: as many as registers hold
+// where each walks four strides or more, else one.
+template <class TV, int NVMAX>
+constexpr int gs_unroll(GsMode M) {
+    if (M != kUpdateDots || NVMAX == 8) return 4;
+    if (sizeof(TV) == 4) return NVMAX <= 32 ? 4 : NVMAX <= 41 ? 2 : 1;
+    return NVMAX <= 16 ? 2 : 1;
 }
 
-// w -= V_{0..nv-1} h (h = m->redout + hoff on the device), then the dots of
-// the new w with V_0..V_{nv-1} (or, NORM, its squared norm) into
-// m->redout + off: the update and mdot in one pass (the same results).
-template <class TV, bool NORM>
-void cgs_pass(cfd_mesh *m, int nv, const TV *V, size_t ld, int hoff, TV *w, int off) {
+// One Gram-Schmidt pass of w against V_0..V_{nv-1} (coefficients at m->redout +
+// hoff); sums to m->redout + off and m->hred + off.
+template <class TV, GsMode M>
+void gs_pass(cfd_mesh *m, int nv, const TV *V, size_t ld, int hoff, TV *w, int off) {
     const size_t L = 5 * (size_t)m->N;
     const int np = dot_parts(L);
     const double *h = m->redout + hoff;
-    const bool deep = L >= 4 * (size_t)np * kBlock;  // each thread walks four strides or more
-    dim3 g(np), b(kBlock);
+    const GsSums g{m->red, m->redout + off, m->hred + off};
+    const bool deep = L >= 4 * (size_t)np * kBlock;
     // NVMAX: the fewest unrolled vectors that cover nv
-#define CFD_CGS(NVMAX)                                                                                          \
-    do {                                                                                                         \
-        if (deep) hipLaunchKernelGGL((k_cgs_pass<TV, NVMAX, NORM, true>), g, b, 0, m->stream, L, nv, V, ld, h, w, \
-                                     m->red);                                                                    \
-        else hipLaunchKernelGGL((k_cgs_pass<TV, NVMAX, NORM, false>), g, b, 0, m->stream, L, nv, V, ld, h, w,     \
-                                m->red);                                                                         \
+#define CFD_GS(NVMAX)                                                                                               \
+    do {                                                                                                            \
+        if (deep)                                                                                                   \
+            hipLaunchKernelGGL((k_gs<TV, NVMAX, M, gs_unroll<TV, NVMAX>(M)>), dim3(np), dim3(kBlock), 0,            \
+                               m->stream, L, nv, V, ld, h, w, g, m->flag);                                          \
+        else                                                                                                        \
+            hipLaunchKernelGGL((k_gs<TV, NVMAX, M, 1>), dim3(np), dim3(kBlock), 0, m->stream, L, nv, V, ld,  \
+                               h, w, g, m->flag);                                                                   \
     } while (0)
-    if (nv <= 8) CFD_CGS(8);
-    else if (nv <= 16) CFD_CGS(16);
-    else if (nv <= 32) CFD_CGS(32);
-    else if (nv <= 41) CFD_CGS(41);
-    else CFD_CGS(kMaxKrylov + 1);
-#undef CFD_CGS
-    const int nd = NORM ? 1 : nv;
-    hipLaunchKernelGGL(k_mdot_final, dim3(nd), dim3(64), 0, m->stream, np, nd, m->red, m->redout + off);
+    if (nv <= 8) CFD_GS(8);
+    else if (nv <= 16) CFD_GS(16);
+    else if (nv <= 32) CFD_GS(32);
+    else if (nv <= 41) CFD_GS(41);
+    else CFD_GS(kMaxKrylov + 1);
+#undef CFD_GS
 }
 
 // Krylov basis of one storage type for restart length mk.  Each precision
@@ -2286,8 +2262,8 @@ int ensure_krylov(cfd_mesh *m, int mk, bool mixed) {
 }
 
 // One Arnoldi step j of FGMRES: V_j = w / ||w|| (j > 0, norm of the previous
-// step), Z_j = M^-1 V_j, w = A Z_j, two CGS passes against V_0..V_j, ||w||^2,
-// and the copy of the Hessenberg column to the host.  The sequence depends
+// step), Z_j = M^-1 V_j, w = A Z_j, two CGS passes against V_0..V_j and
+// ||w||^2, whose sums the passes leave on the host too.  The sequence depends
 // only on j and the mesh's buffers, so it is captured once per j as a graph.
 template <class TM, class TV>
 void arnoldi_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V, TV *Z, TV *w, int j) {
@@ -2302,10 +2278,9 @@ void arnoldi_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V,
     spmv<TM, TV, TV>(m, zj, w, nullptr);
     // CGS2: h1 = V^T w, w -= V h1, h2 = V^T w, w -= V h2, ||w||^2 (each
     // update fused with the reduction after it)
-    mdot<TV>(m, j + 1, V, L, w, 0);
-    cgs_pass<TV, false>(m, j + 1, V, L, 0, w, kMaxKrylov + 1);
-    cgs_pass<TV, true>(m, j + 1, V, L, kMaxKrylov + 1, w, 2 * (kMaxKrylov + 1));
-    hipMemcpyAsync(m->hred, m->redout, sizeof(double) * (2 * (kMaxKrylov + 1) + 1), hipMemcpyDeviceToHost, m->stream);
+    gs_pass<TV, kDots>(m, j + 1, V, L, 0, w, 0);
+    gs_pass<TV, kUpdateDots>(m, j + 1, V, L, 0, w, kMaxKrylov + 1);
+    gs_pass<TV, kUpdateNorm>(m, j + 1, V, L, kMaxKrylov + 1, w, 2 * (kMaxKrylov + 1));
 }
 
 // Enqueues Arnoldi step j, replaying its captured graph (captured on first use).
@@ -2363,34 +2338,20 @@ int enqueue_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V, 
     return CFD_OK;
 }
 
-// Per-case dots of V_0..V_{nv-1} with w into m->bred[c][slot..] (union of cases).
-template <class TV>
-void mdot_seg(cfd_mesh *m, int nv, const TV *V, size_t ld, const TV *w, int slot) {
+// The same per case of a union: coefficients at m->bred[c][hslot..], sums to
+// m->bred[c][slot..] and m->hbred[c][slot..].
+template <class TV, GsMode M>
+void gs_pass_seg(cfd_mesh *m, int nv, const TV *V, size_t ld, int hslot, TV *w, int slot) {
     const SegMap &sg = m->seg_dot;
-    hipLaunchKernelGGL(k_mdot_seg<TV>, dim3(sg.nblocks), dim3(kBlock), 0, m->stream, sg.blk, sg.first, sg.off, sg.len,
-                       nv, V, ld, w, m->bpart);
-    hipLaunchKernelGGL(k_mdot_seg_final, dim3(nv, m->ncase), dim3(64), 0, m->stream, sg.first, nv, m->bpart, m->bred,
-                       slot);
-}
-
-// Per case: w -= V h_c (h_c = m->bred[c][hslot..]), then the dots of the new
-// w with V_0..V_{nv-1} (or, NORM, its squared norm) into m->bred[c][slot..].
-template <class TV, bool NORM>
-void cgs_pass_seg(cfd_mesh *m, int nv, const TV *V, size_t ld, int hslot, TV *w, int slot) {
-    const SegMap &sg = m->seg_dot;
-    dim3 g(sg.nblocks), b(kBlock);
-#define CFD_CGS_SEG(NVMAX, NORM_)                                                                                   \
-    hipLaunchKernelGGL((k_cgs_pass_seg<TV, NVMAX, NORM_>), g, b, 0, m->stream, sg.blk, sg.first, sg.off, sg.len, nv, \
-                       V, ld, m->bred, hslot, w, m->bpart)
-    if (nv <= 8) CFD_CGS_SEG(8, NORM);
-    else if (nv <= 16) CFD_CGS_SEG(16, NORM);
-    else if (nv <= 32) CFD_CGS_SEG(32, NORM);
-    else if (nv <= 41) CFD_CGS_SEG(41, NORM);
-    else CFD_CGS_SEG(kMaxKrylov + 1, NORM);
-#undef CFD_CGS_SEG
-    const int nd = NORM ? 1 : nv;
-    hipLaunchKernelGGL(k_mdot_seg_final, dim3(nd, m->ncase), dim3(64), 0, m->stream, sg.first, nd, m->bpart, m->bred,
-                       slot);
+#define CFD_GS_SEG(NVMAX)                                                                                            \
+    hipLaunchKernelGGL((k_gs_seg<TV, NVMAX, M>), dim3(sg.nblocks), dim3(kBlock), 0, m->stream, sg.blk, sg.first,     \
+                       sg.off, sg.len, nv, V, ld, m->bred + hslot, m->bred + slot, m->hbred + slot, w, m->bpart, m->flag)
+    if (nv <= 8) CFD_GS_SEG(8);
+    else if (nv <= 16) CFD_GS_SEG(16);
+    else if (nv <= 32) CFD_GS_SEG(32);
+    else if (nv <= 41) CFD_GS_SEG(41);
+    else CFD_GS_SEG(kMaxKrylov + 1);
+#undef CFD_GS_SEG
 }
 
 // Arnoldi step j of the batched FGMRES: the operations of arnoldi_step with
@@ -2406,10 +2367,9 @@ void arnoldi_step_batch(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, 
                            m->bred, 2 * (kMaxKrylov + 1));
     apply_prec<TM, TV>(m, m->prec_kind, lu, dinv, vj, zj);
     spmv<TM, TV, TV>(m, zj, w, nullptr);
-    mdot_seg<TV>(m, j + 1, V, L, w, 0);
-    cgs_pass_seg<TV, false>(m, j + 1, V, L, 0, w, kMaxKrylov + 1);
-    cgs_pass_seg<TV, true>(m, j + 1, V, L, kMaxKrylov + 1, w, 2 * (kMaxKrylov + 1));
-    hipMemcpyAsync(m->hbred, m->bred, sizeof(double) * kBOut * (size_t)m->ncase, hipMemcpyDeviceToHost, m->stream);
+    gs_pass_seg<TV, kDots>(m, j + 1, V, L, 0, w, 0);
+    gs_pass_seg<TV, kUpdateDots>(m, j + 1, V, L, 0, w, kMaxKrylov + 1);
+    gs_pass_seg<TV, kUpdateNorm>(m, j + 1, V, L, kMaxKrylov + 1, w, 2 * (kMaxKrylov + 1));
 }
 
 template <class TM, class TV>
@@ -2482,8 +2442,7 @@ int fgmres_batch(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM 
     const size_t ldc = kMaxKrylov + 1;
     hipLaunchKernelGGL(k_fill, dim3(gN), dim3(kBlock), 0, m->stream, L, 0.0, m->x);
     CFD_HIP(m, hipMemcpyAsync(m->r, m->b, sizeof(double) * L, hipMemcpyDeviceToDevice, m->stream));
-    mdot_seg<double>(m, 1, m->r, 0, m->r, 0);
-    CFD_HIP(m, hipMemcpyAsync(m->hbred, m->bred, sizeof(double) * kBOut * K, hipMemcpyDeviceToHost, m->stream));
+    gs_pass_seg<double, kDots>(m, 1, m->r, 0, 0, m->r, 0);
     CFD_HIP(m, hipStreamSynchronize(m->stream));
     std::vector<double> beta(K), tol(K), res(K);
     std::vector<char> live(K), cyc(K), step(K);
@@ -2580,8 +2539,7 @@ int fgmres_batch(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM 
         if (!any) break;
         // true residual for the restart
         spmv<TM, double, double>(m, m->x, m->r, m->b);
-        mdot_seg<double>(m, 1, m->r, 0, m->r, 0);
-        CFD_HIP(m, hipMemcpyAsync(m->hbred, m->bred, sizeof(double) * kBOut * K, hipMemcpyDeviceToHost, m->stream));
+        gs_pass_seg<double, kDots>(m, 1, m->r, 0, 0, m->r, 0);
         CFD_HIP(m, hipStreamSynchronize(m->stream));
         for (int c = 0; c < K; c++) {
             if (!live[c]) continue;
@@ -2608,8 +2566,7 @@ int fgmres(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM *lu, c
     // x0 = 0; r0 = b
     hipLaunchKernelGGL(k_fill, dim3(gN), dim3(kBlock), 0, m->stream, L, 0.0, m->x);
     CFD_HIP(m, hipMemcpyAsync(m->r, m->b, sizeof(double) * L, hipMemcpyDeviceToDevice, m->stream));
-    mdot<double>(m, 1, m->r, 0, m->r, 0);
-    CFD_HIP(m, hipMemcpyAsync(hr, m->redout, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    gs_pass<double, kDots>(m, 1, m->r, 0, 0, m->r, 0);
     CFD_HIP(m, hipStreamSynchronize(m->stream));
     const double bnorm = sqrt(hr[0]);
     const double tol = o->rtol * bnorm;
@@ -2664,8 +2621,7 @@ int fgmres(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM *lu, c
         if (res <= tol) break;
         // true residual for the restart
         spmv<TM, double, double>(m, m->x, m->r, m->b);
-        mdot<double>(m, 1, m->r, 0, m->r, 0);
-        CFD_HIP(m, hipMemcpyAsync(hr, m->redout, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+        gs_pass<double, kDots>(m, 1, m->r, 0, 0, m->r, 0);
         CFD_HIP(m, hipStreamSynchronize(m->stream));
         beta = sqrt(hr[0]);
         res = beta;
@@ -2981,6 +2937,11 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
         return cfd_set_error(m->ctx, CFD_E_ARG, "Jacobian precision does not match linsolve precision");
     int rc = ensure_krylov(m, o->krylov_m, mixed);
     if (rc) return rc;
+    // the partial sums of the Gram-Schmidt passes (their buffers serve other
+    // reductions between linear solves)
+    const size_t nw = (size_t)(kMaxKrylov + 1) * (m->ncase ? m->seg_dot.nblocks : dot_parts(5 * (size_t)m->N));
+    hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(nw, 4096)), dim3(kBlock), 0, m->stream, nw,
+                       m->ncase ? m->bpart : m->red);
     if (flow_sweeps(m, o->precond)) {
         rc = ensure_slots12(m, m->mc_lower);
         if (!rc) rc = ensure_slots12(m, m->mc_upper);
