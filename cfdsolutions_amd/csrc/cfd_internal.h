@@ -11,15 +11,29 @@
 #include <mutex>
 #include <shared_mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
 #include "cfd_hip.h"
 
+// Pinned host memory through which fields cross to and from the caller's
+// arrays, in two slots; made on first use, grown to what a field needs (two
+// times kFieldSlot at most) and given back with the context.  lock: held by the
+// one transfer that uses it.
+constexpr size_t kFieldSlot = 16u << 20;
+struct FieldStaging {
+    std::mutex lock;
+    char *slot[2] = {nullptr, nullptr};
+    size_t bytes = 0;  // of each slot
+    hipEvent_t done[2] = {nullptr, nullptr};
+};
+
 struct cfd_ctx {
     int device = 0;
     std::mutex lock;  // guards err
     std::string err;
+    FieldStaging staging;
     // device address of this GPU's copy of the scratch array of
     // cfd_linsolve_gs_noalloc (looked up when the context is created), or
     // NULL if the lookup failed
@@ -121,7 +135,13 @@ void cfd_parallel_for(int64_t n, F fn, int64_t grain = 1 << 14) {
     }
     std::vector<std::thread> th;
     th.reserve(nt - 1);
-    for (int t = 1; t < nt; t++) th.emplace_back(fn, n * t / nt, n * (t + 1) / nt);
+    for (int t = 1; t < nt; t++) {
+        try {
+            th.emplace_back(fn, n * t / nt, n * (t + 1) / nt);
+        } catch (const std::system_error &) {  // no thread to be had: this one does its part
+            fn(n * t / nt, n * (t + 1) / nt);
+        }
+    }
     fn((int64_t)0, n / nt);
     for (auto &x : th) x.join();
 }
