@@ -844,7 +844,7 @@ extern "C" int64_t cfd_footprint_bytes(int32_t N, int32_t E, int32_t B, int32_t 
     bytes += nsell * (4 + 4 + 3 * 8);                       // nbr, soff, isx, isy, isz
     bytes += 4 * ((n + 1) + nnz + n);                       // BSR ia, ja, iau
     bytes += 4 * (n + (n + 1) + 2 * nnz + n + 2 * n);       // multicolour pattern, slot map, levels
-    bytes += s * 2 * 5 * n;                                 // work vectors of the sweeps
+    bytes += s * 6 * 5 * n;                                 // work vectors of the sweeps
     bytes += 4 * (2 * n + 4 * n + 4 * 11 * lvl);           // level rows and padded slot lists
     bytes += 8 * (1024 * 65 + 4 * 65 + 6) + 4 * 4;         // reduction scratch, eigenvalue bits, flags
     bytes += 25 * s * nnz * 2 + 25 * s * n;                 // Jacobian, ILU(0) factors, inverse pivots

@@ -269,7 +269,8 @@ struct cfd_mesh {
     int *mc_ia = nullptr, *mc_ja = nullptr, *mc_iau = nullptr;  // permuted BSR pattern
     int *mc_src = nullptr;                                // [nnz] original slot of each permuted slot
     LevelSchedule mc_lower, mc_upper;
-    double *zp = nullptr;  // 2 x [N][5] work vectors of the sweeps (single-launch: handover words)
+    double *zp = nullptr;  // nzp64 x [N][5] work vectors of the sweeps (single-launch: handover words)
+    int nzp64 = 0, nzp32 = 0;
     float *zpf = nullptr;
     bool sync_free = true;    // single-launch triangular sweeps (else one launch per level)
     // block-SELL copies for the Krylov loop: A (SpMV), and the multicolour

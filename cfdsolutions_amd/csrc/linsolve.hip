@@ -605,7 +605,7 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
 #pragma unroll
             for (int q = 0; q < kIluPad; q++)
 #pragma unroll
-                for (int s = 0; s < NS; s++) hit[s] = (cq[q] == col[s]) & (c0 + q < np) ? c0 + q : hit[s];
+                for (int s = 0; s < NS; s++) hit[s] = ((cq[q] == col[s]) & (c0 + q < np)) ? c0 + q : hit[s];
         }
 #pragma unroll
         for (int c = 0; c < 5; c++) {
@@ -914,14 +914,29 @@ struct FlowBlocks {
                 if (v[u] == FlowWord<TV>::unset) v[u] = flow_load(x + 5 * (size_t)j[u]);
         }
     }
-    // t[u] = (row r of block u) . (neighbour u); sh: this row's place in LDS.
-    __device__ __forceinline__ void dots(TV *sh, int r, TV *t) {
+    __device__ __forceinline__ void share(TV *sh, int r) {
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int u = 0; u < U; u++) sh[u * FlowLds<TV>::row + r] = __builtin_bit_cast(TV, v[u]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // s plus the products one after the other, as k_spmv adds them.
+    __device__ __forceinline__ TV add_dots(TV *sh, int r, TV s) {
+        share(sh, r);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            TV q = s;
+#pragma unroll
+            for (int c = 0; c < 5; c++) q += (TV)av[u][c] * sh[u * FlowLds<TV>::row + c];
+            s = u < n ? q : s;
+        }
+        return s;
+    }
+    // t[u] = (row r of block u) . (neighbour u); sh: this row's place in LDS.
+    __device__ __forceinline__ void dots(TV *sh, int r, TV *t) {
+        share(sh, r);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             TV s = TV(0.0);
@@ -932,51 +947,95 @@ struct FlowBlocks {
     }
 };
 
-// One sweep of the ILU(0) apply; 12 rows of 5 lanes per wavefront, lane r owns
-// component r.  Forward: w_i = r_P(i) - sum_{k<i} L_ik w_k; backward:
-// w_i = D_i^-1 (w_i - sum_{k>i} U_ik w_k), z_P(i) = w_i, in the operation order
-// of k_trsv_level and k_trsv_mc.  perm is the row permutation P of the
-// multicolour order, NULL for the natural order.  wf, wb: handover arrays of
-// the forward and backward sweep; each sweep leaves the other one's words of
-// its rows unset for the sweep after it.
+// The ILU(0) apply and the product that follows it in an Arnoldi step, in one
+// launch; 12 rows of 5 lanes per wavefront, lane r owns component r.  Items, in
+// the order the wavefronts take them:
+//   forward    w_i = r_P(i) - sum_{k<i} L_ik w_k, r = V_j, here also normalised and
+//              stored from the last step's w where norm2 is given (k_scale_dev)
+//   backward   z_P(i) = w_i = D_i^-1 (w_i - sum_{k>i} U_ik w_k)
+//   product    y_i = sum_k A_ik z_k
+// in the operation order of k_trsv_level, k_trsv_mc and k_spmv.  P is the row
+// permutation perm of the multicolour order (NULL: the natural order); A is in
+// the reference's order.  Handover words: of the forward sweep, the backward
+// sweep and (where P is given) of z in the reference's order.  The other set of
+// words is left unset for the next launch, so nothing is cleared while it is
+// read.  A backward row starts when its own neighbours are done, a product
+// while the last rows still run, and four launches are saved: ten mixed steps on
+// 45,625 rows 36.6 -> 34.3 ms, a step on 14,161 rows 2% (the chain of the
+// colours, 57 us, bounds it).
+template <class TM, class TV>
+struct FlowStep {
+    int nf, nb, np;          // padded rows of the sweeps' schedules, rows of the product (0: none)
+    const int *sf, *sb;      // the schedules
+    const int *ia, *ja, *iau, *perm;
+    const TM *lu, *dinv;
+    const TV *w;             // last step's w (norm2) or unused
+    const double *norm2;     // its squared norm, or NULL
+    TV *v, *z, *y;           // V_j, Z_j, the product
+    const int *aia, *aja;
+    const TM *a;
+    TV *words, *other;       // this launch's set of handover words and the next one's
+    size_t L;
+    int *flag;
+};
+
 template <class TM>
 constexpr int kTrsvPerCu = sizeof(TM) == 4 ? 4 : 2;
 template <class TM, class TV>
-__global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_trsv_flow(int nslots, const int *__restrict__ slots,
-                                                      const int *__restrict__ ia, const int *__restrict__ ja,
-                                                      const int *__restrict__ iau, const int *__restrict__ perm,
-                                                      const TM *__restrict__ lu, const TM *__restrict__ dinv,
-                                                      const TV *__restrict__ rhs, TV *wf, TV *wb, TV *z, int backward,
-                                                      int *flag) {
+__global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_arnoldi_flow(FlowStep<TM, TV> f) {
     const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
-    TV *cur = backward ? wb : wf, *other = backward ? wf : wb;
+    TV *wf = f.words, *wb = f.words + f.L, *wz = f.perm ? wb + f.L : wb;
     __shared__ __align__(16) FlowLds<TV> lds;
     TV *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<TV>::slot;
+    const double denom = f.norm2 ? sqrt(f.norm2[0]) : 1.0;
+    const int cf = (f.nf + 11) / 12, cb = (f.nb + 11) / 12, cp = (f.np + 11) / 12;
     const int nw = gridDim.x * (kBlock / 64);
-    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); 12 * w < nslots; w += nw) {
-        const int t = 12 * w + slot;
-        const int i = slot < 12 && t < nslots ? slots[t] : -1;
+    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); w < cf + cb + cp; w += nw) {
+        FlowBlocks<8, TM, TV> g;
+        if (w >= cf + cb) {
+            const int i = 12 * (w - cf - cb) + slot;
+            if (slot < 12 && i < f.np) {
+                const int ke = f.aia[i + 1];
+                TV s = TV(0.0);
+                for (int k0 = f.aia[i]; k0 < ke; k0 += 8) {
+                    g.load(k0, ke, r, f.aja, f.a, wz);
+                    g.wait(f.flag);
+                    s = g.add_dots(sh, r, s);
+                }
+                f.y[5 * (size_t)i + r] = s;
+            }
+            continue;
+        }
+        const bool backward = w >= cf;
+        TV *cur = backward ? wb : wf;
+        const int t = 12 * (backward ? w - cf : w) + slot;
+        const int i = slot < 12 && t < (backward ? f.nb : f.nf) ? (backward ? f.sb : f.sf)[t] : -1;
+        const size_t ri = 5 * (size_t)(i >= 0 ? i : 0) + r;
         TV y = TV(0.0);
         TM dr[5];
         size_t pi = 0;
         if (i >= 0) {
+            pi = 5 * (size_t)(f.perm ? f.perm[i] : i) + r;
+            const int kb = backward ? f.iau[i] + 1 : f.ia[i];
+            const int ke = backward ? f.ia[i + 1] : f.iau[i];
             if (backward) {
 #pragma unroll
-                for (int c = 0; c < 5; c++) dr[c] = dinv[25 * (size_t)i + 5 * r + c];
+                for (int c = 0; c < 5; c++) dr[c] = f.dinv[25 * (size_t)i + 5 * r + c];
+                y = flow_wait(wf + ri, flow_load(wf + ri), f.flag);
+            } else {
+                y = f.norm2 ? (TV)((double)f.w[pi] / denom) : f.v[pi];
+                if (f.norm2) f.v[pi] = y;
+                flow_unset(f.other + ri);
+                flow_unset(f.other + f.L + ri);
+                if (f.perm) flow_unset(f.other + 2 * f.L + ri);
             }
-            const int kb = backward ? iau[i] + 1 : ia[i];
-            const int ke = backward ? ia[i + 1] : iau[i];
-            pi = 5 * (size_t)(perm ? perm[i] : i) + r;
-            y = backward ? other[5 * (size_t)i + r] : rhs[pi];
-            flow_unset(other + 5 * (size_t)i + r);
             for (int k0 = kb; k0 < ke; k0 += 8) {
-                FlowBlocks<8, TM, TV> g;
-                TV t[8];
-                g.load(k0, ke, r, ja, lu, cur);
-                g.wait(flag);
-                g.dots(sh, r, t);
+                TV t8[8];
+                g.load(k0, ke, r, f.ja, f.lu, cur);
+                g.wait(f.flag);
+                g.dots(sh, r, t8);
 #pragma unroll
-                for (int u = 0; u < 8; u++) y = y - t[u];
+                for (int u = 0; u < 8; u++) y = y - t8[u];
             }
         }
         if (backward) {
@@ -989,10 +1048,11 @@ __global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_trsv_flow(int nslots
 #pragma unroll
                 for (int c = 0; c < 5; c++) s += (TV)dr[c] * yy[c];
                 y = s;
-                z[pi] = y;
+                f.z[pi] = y;
+                if (f.perm) flow_store(wz + pi, y);
             }
         }
-        if (i >= 0) flow_store(cur + 5 * (size_t)i + r, y);
+        if (i >= 0) flow_store(cur + ri, y);
     }
 }
 
@@ -1393,7 +1453,7 @@ __device__ __forceinline__ const double *flow_lu(double *sh, int r, const double
 }
 
 // Forward Gauss-Seidel sweeps 0..S-1 in one launch (row update:
-// MC_Iterative_Jacobi.c:410-450), rows handed over as in k_trsv_flow: sweep s
+// MC_Iterative_Jacobi.c:410-450), rows handed over as in k_arnoldi_flow: sweep s
 // writes its own version ver[s] of x, so row i of sweep s needs only its
 // lower neighbours of sweep s and its upper ones (and itself) of sweep s - 1,
 // and sweep s follows `reach` + 1 chunks behind sweep s - 1 instead of waiting
@@ -1522,7 +1582,7 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_lu(int N, const int *iau, cons
 
 // One LU-SGS half sweep (row update: MC_Iterative_Jacobi.c:586-678,
 // MATH/src/LinearAlgebra.c:117-155) in one launch, rows handed over as in
-// k_trsv_flow: the neighbours swept before row i are read from cur, the others
+// k_arnoldi_flow: the neighbours swept before row i are read from cur, the others
 // from prev, the result of the half sweep before.  next is left unset for the
 // half sweep after this one.  Half sweeps run in opposite directions, so they
 // do not overlap.
@@ -1724,7 +1784,7 @@ __device__ __forceinline__ void gs_entries(size_t o, size_t i, size_t stride, in
 
 // Where the sums of one partition (a mesh, or a case of a union) go.
 struct GsSums {
-    double *words;  // [nd][P] partial sums of its P blocks, handed over as in k_trsv_flow; unset between launches
+    double *words;  // [nd][P] partial sums of its P blocks, handed over as in k_arnoldi_flow; unset between launches
     double *out;    // [nd]
     double *host;   // [nd] the same in pinned host memory
 };
@@ -2091,10 +2151,10 @@ void spmv(cfd_mesh *m, const TX *x, TY *y, const double *bsub) {
 // the natural order (hundreds of levels), in the multicolour order (8 colours
 // on the bump channels) up to kFlowMcRows rows.  There a launch per colour
 // costs more than the handovers; above, all waves of a colour together keep
-// more loads in flight than the resident waves of one launch.  Whole implicit
-// steps, mixed precision: 14,161 rows 4.74 ms against 5.96 ms with a launch
-// per colour, 45,625 rows (ten steps) 43.1 against 48.7 ms, 104,448 rows 21.4
-// against 19.8 ms.
+// more loads in flight than the resident waves of one launch.  With nothing
+// else changed, whole mixed steps took 4.74 ms against 5.96 ms with a launch
+// per colour at 14,161 rows, 43.1 against 48.7 ms (ten steps) at 45,625 rows,
+// 21.4 against 19.8 ms at 104,448 rows.
 constexpr int kFlowMcRows = 65536;
 bool flow_sweeps(const cfd_mesh *m, int kind) {
     return m->sync_free &&
@@ -2111,17 +2171,7 @@ float *mc_work<float>(cfd_mesh *m) { return m->zpf; }
 template <class TM, class TV>
 void apply_prec(cfd_mesh *m, int kind, const TM *lu, const TM *dinv, const TV *r, TV *z) {
     const size_t L = 5 * (size_t)m->N;
-    if (flow_sweeps(m, kind)) {
-        const bool mc = kind == CFD_PREC_ILU0_MC;
-        TV *wf = mc_work<TV>(m);
-        for (int pass = 0; pass < 2; pass++) {
-            const LevelSchedule &ls = mc ? (pass ? m->mc_upper : m->mc_lower) : (pass ? m->upper : m->lower);
-            hipLaunchKernelGGL((k_trsv_flow<TM, TV>), dim3(std::min((ls.n12 + 47) / 48, flow_blocks(kTrsvPerCu<TM>))),
-                               dim3(kBlock), 0, m->stream, ls.n12, ls.slots12, mc ? m->mc_ia : m->ia, mc ? m->mc_ja : m->ja,
-                               mc ? m->mc_iau : m->iau, mc ? m->mc_perm : nullptr, lu, dinv, r, wf, wf + L, z, pass,
-                               m->flag);
-        }
-    } else if (kind == CFD_PREC_ILU0_MC && !m->use_sell) {
+    if (kind == CFD_PREC_ILU0_MC && !m->use_sell) {
         TV *wk = mc_work<TV>(m);
         for (int pass = 0; pass < 2; pass++) {
             const LevelSchedule &ls = pass ? m->mc_upper : m->mc_lower;
@@ -2218,18 +2268,39 @@ void gs_pass(cfd_mesh *m, int nv, const TV *V, size_t ld, int hoff, TV *w, int o
 #undef CFD_GS
 }
 
+// The two sets of handover words of k_arnoldi_flow in the sweeps' work vector;
+// step j of a cycle uses set j % 2 and leaves the other unset.
+constexpr size_t kFlowWords = 3;  // vectors of a set
+
 // Krylov basis of one storage type for restart length mk.  Each precision
 // keeps its own basis, so alternating FP64 and mixed solves on one mesh
 // allocates each once; a basis too short for a larger mk is replaced (the
 // old one freed, after the stream is idle and the graphs captured on it are
 // dropped), so the mesh's footprint never grows past one basis per
 // precision.
-int ensure_krylov(cfd_mesh *m, int mk, bool mixed) {
+int ensure_krylov(cfd_mesh *m, int mk, int precond, bool mixed) {
     const size_t L = 5 * (size_t)m->N;
-    if (mixed && !m->zpf) m->zpf = (float *)cfd_dalloc(m, sizeof(float) * 2 * L);
-    if (!mixed && !m->zp) m->zp = (double *)cfd_dalloc(m, sizeof(double) * 2 * L);
-    if ((mixed && !m->zpf) || (!mixed && !m->zp))
-        return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (multicolour work vector)");
+    // the sweeps' work vector: two sets of handover words where they run in one
+    // launch, else the permuted vector
+    const int want = flow_sweeps(m, precond) ? 2 * (int)kFlowWords : 1;
+    int &nzp = mixed ? m->nzp32 : m->nzp64;
+    if (nzp < want) {
+        if (nzp) {
+            CFD_HIP(m, hipStreamSynchronize(m->stream));
+            drop_krylov_graphs(m);
+        }
+        nzp = 0;
+        if (mixed) {
+            cfd_dfree(m, m->zpf);
+            m->zpf = (float *)cfd_dalloc(m, sizeof(float) * want * L);
+        } else {
+            cfd_dfree(m, m->zp);
+            m->zp = (double *)cfd_dalloc(m, sizeof(double) * want * L);
+        }
+        if (mixed ? !m->zpf : !m->zp)
+            return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (work vector of the sweeps)");
+        nzp = want;
+    }
     if (!m->r) m->r = (double *)cfd_dalloc(m, sizeof(double) * L);
     if (!m->r) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (Krylov)");
     int &have = mixed ? m->kry_m32 : m->kry_m64;
@@ -2261,6 +2332,52 @@ int ensure_krylov(cfd_mesh *m, int mk, bool mixed) {
     return CFD_OK;
 }
 
+// Steps 1-3 of arnoldi_step in one launch: V_j (from w, where norm2 is given),
+// Z_j and, on the BSR arrays, w = A Z_j; returns whether w was formed.
+template <class TM, class TV>
+bool flow_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *vj, TV *zj, TV *w, int j,
+               const double *norm2) {
+    const size_t L = 5 * (size_t)m->N;
+    const bool mc = m->prec_kind == CFD_PREC_ILU0_MC;
+    const LevelSchedule &lo = mc ? m->mc_lower : m->lower, &up = mc ? m->mc_upper : m->upper;
+    TV *set = mc_work<TV>(m);
+    FlowStep<TM, TV> f{};
+    f.nf = lo.n12;
+    f.nb = up.n12;
+    f.np = m->use_sell ? 0 : m->N;
+    f.sf = lo.slots12;
+    f.sb = up.slots12;
+    f.ia = mc ? m->mc_ia : m->ia;
+    f.ja = mc ? m->mc_ja : m->ja;
+    f.iau = mc ? m->mc_iau : m->iau;
+    f.perm = mc ? m->mc_perm : nullptr;
+    f.lu = lu;
+    f.dinv = dinv;
+    f.w = w;
+    f.norm2 = norm2;
+    f.v = vj;
+    f.z = zj;
+    f.y = w;
+    f.aia = m->ia;
+    f.aja = m->ja;
+    f.a = a;
+    f.words = set + (j & 1) * kFlowWords * L;
+    f.other = set + (1 - (j & 1)) * kFlowWords * L;
+    f.L = L;
+    f.flag = m->flag;
+    const int chunks = (f.nf + 11) / 12 + (f.nb + 11) / 12 + (f.np + 11) / 12;
+    hipLaunchKernelGGL((k_arnoldi_flow<TM, TV>), dim3(std::min((chunks + 3) / 4, flow_blocks(kTrsvPerCu<TM>))),
+                       dim3(kBlock), 0, m->stream, f);
+    return f.np > 0;
+}
+
+// Unsets the first set of handover words, before step 0 of a cycle.
+template <class TV>
+void flow_begin(cfd_mesh *m) {
+    const size_t n = kFlowWords * 5 * (size_t)m->N;
+    hipLaunchKernelGGL(k_flow_unset<TV>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, mc_work<TV>(m));
+}
+
 // One Arnoldi step j of FGMRES: V_j = w / ||w|| (j > 0, norm of the previous
 // step), Z_j = M^-1 V_j, w = A Z_j, two CGS passes against V_0..V_j and
 // ||w||^2, whose sums the passes leave on the host too.  The sequence depends
@@ -2271,11 +2388,15 @@ void arnoldi_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V,
     const int gN = grid_cap(L, 4096);
     const int gS = (int)((L + kBlock - 1) / kBlock);
     TV *vj = V + L * j, *zj = Z + L * j;
-    if (j > 0)
-        hipLaunchKernelGGL((k_scale_dev<TV, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, w, vj,
-                           m->redout + 2 * (kMaxKrylov + 1));
-    apply_prec<TM, TV>(m, m->prec_kind, lu, dinv, vj, zj);
-    spmv<TM, TV, TV>(m, zj, w, nullptr);
+    const double *norm2 = j > 0 ? m->redout + 2 * (kMaxKrylov + 1) : nullptr;
+    bool product = false;
+    if (flow_sweeps(m, m->prec_kind)) {
+        product = flow_step<TM, TV>(m, a, lu, dinv, vj, zj, w, j, norm2);
+    } else {
+        if (norm2) hipLaunchKernelGGL((k_scale_dev<TV, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, w, vj, norm2);
+        apply_prec<TM, TV>(m, m->prec_kind, lu, dinv, vj, zj);
+    }
+    if (!product) spmv<TM, TV, TV>(m, zj, w, nullptr);
     // CGS2: h1 = V^T w, w -= V h1, h2 = V^T w, w -= V h2, ||w||^2 (each
     // update fused with the reduction after it)
     gs_pass<TV, kDots>(m, j + 1, V, L, 0, w, 0);
@@ -2365,8 +2486,10 @@ void arnoldi_step_batch(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, 
     if (j > 0)
         hipLaunchKernelGGL((k_scale_dev_seg<TV, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, m->ecase, w, vj,
                            m->bred, 2 * (kMaxKrylov + 1));
-    apply_prec<TM, TV>(m, m->prec_kind, lu, dinv, vj, zj);
-    spmv<TM, TV, TV>(m, zj, w, nullptr);
+    bool product = false;
+    if (flow_sweeps(m, m->prec_kind)) product = flow_step<TM, TV>(m, a, lu, dinv, vj, zj, w, j, nullptr);
+    else apply_prec<TM, TV>(m, m->prec_kind, lu, dinv, vj, zj);
+    if (!product) spmv<TM, TV, TV>(m, zj, w, nullptr);
     gs_pass_seg<TV, kDots>(m, j + 1, V, L, 0, w, 0);
     gs_pass_seg<TV, kUpdateDots>(m, j + 1, V, L, 0, w, kMaxKrylov + 1);
     gs_pass_seg<TV, kUpdateNorm>(m, j + 1, V, L, kMaxKrylov + 1, w, 2 * (kMaxKrylov + 1));
@@ -2472,6 +2595,7 @@ int fgmres_batch(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM 
         CFD_HIP(m, hipMemcpyAsync(m->bcoef, m->hbcoef, sizeof(double) * ldc * K, hipMemcpyHostToDevice, m->stream));
         hipLaunchKernelGGL((k_scale_seg<double, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, m->ecase, m->r, V,
                            m->bcoef);
+        if (flow_sweeps(m, m->prec_kind)) flow_begin<TV>(m);
         for (int j = 0; j < mk; j++) {
             int rc = enqueue_step_batch<TM, TV>(m, a, lu, dinv, V, Z, w, j, mk);
             if (rc) return rc;
@@ -2577,6 +2701,7 @@ int fgmres(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM *lu, c
     for (int cycle = 0; cycle <= o->max_restarts && beta > tol && beta > 0.0; cycle++) {
         cycles++;
         hipLaunchKernelGGL((k_scale<double, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, m->r, V, beta);
+        if (flow_sweeps(m, m->prec_kind)) flow_begin<TV>(m);
         for (int i = 0; i <= mk; i++) gv[i] = 0.0;
         gv[0] = beta;
         int kdim = 0;
@@ -2935,7 +3060,7 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
     const bool half = o->mixed >= 2 && sell_mc, half_a = o->mixed == 3 && sell_mc;
     if (mixed != m->jac_mixed)
         return cfd_set_error(m->ctx, CFD_E_ARG, "Jacobian precision does not match linsolve precision");
-    int rc = ensure_krylov(m, o->krylov_m, mixed);
+    int rc = ensure_krylov(m, o->krylov_m, o->precond, mixed);
     if (rc) return rc;
     // the partial sums of the Gram-Schmidt passes (their buffers serve other
     // reductions between linear solves)
@@ -2946,12 +3071,6 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
         rc = ensure_slots12(m, m->mc_lower);
         if (!rc) rc = ensure_slots12(m, m->mc_upper);
         if (rc) return rc;
-        const size_t n = 10 * (size_t)m->N;
-        if (mixed)
-            hipLaunchKernelGGL(k_flow_unset<float>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, m->zpf);
-        else
-            hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, m->zp);
-        CFD_HIP(m, hipGetLastError());
     }
     rc = mixed ? ensure_sell<float>(m, o->precond, half, half_a)
                : ensure_sell<double>(m, o->precond, false, false);
