@@ -130,41 +130,6 @@ extern "C" const char *cfd_last_error(const cfd_ctx *ctx) {
 // mesh creation
 // ---------------------------------------------------------------------------
 
-// Pattern of a block-SELL layout (BlockSell) over rows 0..n-1: row i holds
-// the BSR slots rb(i) .. re(i)-1 in that order, with block columns ja[slot].
-template <class RB, class RE>
-static void build_block_sell(int n, RB rb, RE re, const int *ja, std::vector<int> &off, HostArray<int> &col,
-                             HostArray<int> &src) {
-    const int ns = (n + 63) / 64;
-    off.assign(ns + 1, 0);
-    for (int sl = 0; sl < ns; sl++) {
-        int w = 0;
-        for (int i = 64 * sl; i < std::min(n, 64 * sl + 64); i++) w = std::max(w, re(i) - rb(i));
-        off[sl + 1] = off[sl] + 64 * w;
-    }
-    col = HostArray<int>((size_t)off[ns]);
-    src = HostArray<int>((size_t)off[ns]);
-    // every slot of a slice written by the thread that owns the slice; padding
-    // slots get column 0 and source -1
-    cfd_parallel_for(ns, [&](int64_t s0, int64_t s1) {
-        for (int sl = (int)s0; sl < (int)s1; sl++) {
-            const int w = (off[sl + 1] - off[sl]) / 64;
-            for (int l = 0; l < 64; l++) {
-                const int i = 64 * sl + l;
-                const int len = i < n ? re(i) - rb(i) : 0;
-                for (int k = 0; k < w; k++) {
-                    const size_t q = (size_t)off[sl] + 64 * (size_t)k + l;
-                    col[q] = k < len ? ja[rb(i) + k] : 0;
-                    src[q] = k < len ? rb(i) + k : -1;
-                }
-            }
-        }
-    }, 1 << 8);
-}
-
-static int upload_block_sell(cfd_mesh *m, const std::vector<int> &off, const HostArray<int> &col,
-                             const HostArray<int> &src, BlockSell &bs);
-
 void pad_levels(const std::vector<int> &ptr, const std::vector<int> &rows, int w, std::vector<int> &out) {
     out.clear();
     for (size_t l = 0; l + 1 < ptr.size(); l++) {
@@ -219,14 +184,50 @@ static T *upload(cfd_mesh *m, const T *h, size_t n, int *rc, size_t pad = 0) {
     return d;
 }
 
-static int upload_block_sell(cfd_mesh *m, const std::vector<int> &off, const HostArray<int> &col,
-                             const HostArray<int> &src, BlockSell &bs) {
+// A device array that holds an input of the layout kernels until they have run.
+template <class T>
+static T *scratch(cfd_mesh *m, const T *h, size_t n, std::vector<void *> &tmp, int *rc) {
+    T *d = upload(m, h, n, rc);
+    if (d) tmp.push_back(d);
+    return d;
+}
+
+// Waits for the kernels that read them, then frees the scratch arrays.
+static int free_scratch(cfd_mesh *m, std::vector<void *> &tmp, int rc) {
+    hipError_t e;
+    {
+        CfdRuntimeGuard g;
+        e = hipStreamSynchronize(m->stream);
+    }
+    for (void *p : tmp) cfd_dfree(m, p);
+    tmp.clear();
+    return rc || e == hipSuccess ? rc : cfd_set_error(m->ctx, CFD_E_HIP, "layout kernels: %s", hipGetErrorString(e));
+}
+
+// Block-SELL layout (BlockSell) of a part of each row of a BSR pattern: the
+// host sizes the slices, the device fills them.
+static int make_block_sell(cfd_mesh *m, BsrPart part, const int *hia, const int *hiau, const int *ia, const int *iau,
+                           const int *ja, BlockSell &bs) {
+    const int n = m->N, ns = (n + 63) / 64;
+    std::vector<int> off(ns + 1, 0);
+    int64_t tot = 0;
+    for (int sl = 0; sl < ns; sl++) {
+        int w = 0;
+        for (int i = 64 * sl; i < std::min(n, 64 * sl + 64); i++)
+            w = std::max(w, (part == BsrPart::kLower ? hiau[i] : hia[i + 1]) -
+                                (part == BsrPart::kUpper ? hiau[i] + 1 : hia[i]));
+        tot += 64 * (int64_t)w;
+        if (tot > INT32_MAX) return cfd_set_error(m->ctx, CFD_E_OOM, "cfd_mesh_create: block-SELL offsets");
+        off[sl + 1] = (int)tot;
+    }
     int rc = 0;
-    bs.nblk = (int64_t)col.size();
+    bs.nblk = tot;
     bs.off = upload(m, off.data(), off.size(), &rc);
-    if (!rc && col.size()) bs.col = upload(m, col.data(), col.size(), &rc);
-    if (!rc && src.size()) bs.src = upload(m, src.data(), src.size(), &rc);
-    return rc;
+    if (rc || !tot) return rc;
+    bs.col = (int *)cfd_dalloc(m, sizeof(int) * (size_t)tot);
+    bs.src = (int *)cfd_dalloc(m, sizeof(int) * (size_t)tot);
+    if (!bs.col || !bs.src) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
+    return launch_block_sell(m, part, ia, iau, ja, bs);
 }
 
 extern "C" void cfd_mesh_destroy(cfd_mesh *m) {
@@ -404,58 +405,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         });
         for (int b = 0; b < B; b++) ip[iperm[d->bedge[2 * b]] + 1]++;
         for (int i = 0; i < N; i++) ip[i + 1] += ip[i];
-        HostArray<int2> inc(ip[N]);  // every entry written below (checked by the list ends)
-        {
-            // Edges and boundary edges in order, each appended to the lists of
-            // its nodes.  A union's cases hold ascending ranges of nodes, edges
-            // and boundary edges with no edge between cases, so each case's
-            // ranges are filled on their own (in parallel) in the same order.
-            std::vector<int> pos(ip.begin(), ip.end() - 1), ecut{0}, bcut{0};
-            bool ranges = node_case != nullptr;
-            auto ecase = [&](int e) { return node_case[d->edge[2 * e]]; };
-            auto bcase = [&](int b) { return node_case[d->bedge[2 * b]]; };
-            for (int e = 0; ranges && e < E; e++) {
-                if (node_case[d->edge[2 * e + 1]] != ecase(e) || (e && ecase(e) < ecase(e - 1))) ranges = false;
-                else if (e && ecase(e) != ecase(e - 1)) ecut.push_back(e);
-            }
-            for (int b = 1; ranges && b < B; b++) {
-                if (bcase(b) < bcase(b - 1)) ranges = false;
-                else if (bcase(b) != bcase(b - 1)) bcut.push_back(b);
-            }
-            // piece r: edges [ecut[r], ecut[r+1]) and boundary edges [bcut[r], bcut[r+1]) of one case
-            const int ncs = node_case ? node_case[N - 1] + 1 : 1;
-            if (ranges && E && B && (int)ecut.size() == ncs && (int)bcut.size() == ncs && ecase(0) == 0 &&
-                bcase(0) == 0) {
-                ecut.push_back(E);
-                bcut.push_back(B);
-            } else {
-                ecut.assign({0, E});
-                bcut.assign({0, B});
-            }
-            cfd_parallel_for(
-                (int64_t)ecut.size() - 1,
-                [&](int64_t r0, int64_t r1) {
-                    for (int64_t r = r0; r < r1; r++) {
-                        for (int e = ecut[r]; e < ecut[r + 1]; e++) {
-                            // .y = e for the L end of the edge, ~e for the R end (roles follow
-                            // the reference numbering, L < R, not the internal one)
-                            const int l = iperm[d->edge[2 * e]], rr = iperm[d->edge[2 * e + 1]];
-                            inc[pos[l]++] = make_int2(rr, e);
-                            inc[pos[rr]++] = make_int2(l, ~e);
-                        }
-                        for (int b = bcut[r]; b < bcut[r + 1]; b++)
-                            inc[pos[iperm[d->bedge[2 * b]]]++] = make_int2(N + b, E + b);
-                    }
-                },
-                1);
-            for (int i = 0; i < N; i++)
-                if (pos[i] != ip[i + 1]) {
-                    cfd_mesh_destroy(m);
-                    return cfd_set_error(ctx, CFD_E_ARG, "cfd_mesh_create: n2n lists do not match the edges at node %d",
-                                         order[i]);
-                }
-        }
-        phase("incidence lists");
         // SELL-64 copy of the incidence lists with the area vector of each
         // incidence (see cfd_mesh::nbr); padding entries are never read.
         const int nsl = (N + kSlice - 1) / kSlice;
@@ -474,49 +423,51 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             }
         }
         m->nsell = (size_t)sptr[nsl];
-        // uninitialised storage: the per-slice pass below writes every entry
-        // once (padding included), in parallel, instead of a serial zero fill
-        HostArray<int> nbr(m->nsell);
-        HostArray<double> isx(m->nsell), isy(m->nsell), isz(m->nsell);
-        m->h_sell_edge = HostArray<int>(m->nsell);  // every entry written below
-        cfd_parallel_for(
-            nsl,
-            [&](int64_t s0, int64_t s1) {
-                for (int sl = (int)s0; sl < (int)s1; sl++) {
-                    const int w = (sptr[sl + 1] - sptr[sl]) / kSlice;
-                    for (int l = 0; l < kSlice; l++) {
-                        const int i = sl * kSlice + l;
-                        const int cnt = i < N ? ip[i + 1] - ip[i] : 0;
-                        for (int k = 0; k < w; k++) {
-                            const size_t idx = (size_t)sptr[sl] + (size_t)k * kSlice + l;
-                            if (k >= cnt) {  // padding, never read
-                                nbr[idx] = 0;
-                                isx[idx] = isy[idx] = isz[idx] = 0.0;
-                                m->h_sell_edge[idx] = -1;
-                                continue;
-                            }
-                            const int2 en = inc[ip[i] + k];
-                            m->h_sell_edge[idx] = en.y >= 0 ? en.y : ~en.y;  // boundary: E + b
-                            const double *S;
-                            if (en.x >= N) {
-                                nbr[idx] = en.x;
-                                S = d->bedge_area + 3 * (size_t)(en.x - N);
-                            } else if (en.y >= 0) {
-                                nbr[idx] = en.x;
-                                S = d->edge_area + 3 * (size_t)en.y;
-                            } else {
-                                nbr[idx] = ~en.x;
-                                S = d->edge_area + 3 * (size_t)(~en.y);
-                            }
-                            isx[idx] = S[0];
-                            isy[idx] = S[1];
-                            isz[idx] = S[2];
-                        }
-                    }
-                }
-            },
-            64);
-        phase("sell incidences");
+        std::vector<void *> tmp;
+        auto alloc = [&](size_t bytes) {
+            void *const v = rc ? nullptr : cfd_dalloc(m, bytes);
+            if (!rc && !v) rc = cfd_set_error(ctx, CFD_E_OOM, "out of device memory");
+            return v;
+        };
+        // Scratch of the incidence kernels is freed before the other arrays
+        // are made, which are larger: the peak is that of the finished mesh.
+        unsigned long long found[2] = {~0ull, ~0ull};  // list that does not fit its edges, missing neighbour
+        if (!rc) m->order = upload(m, order.data(), order.size(), &rc);
+        if (!rc) m->iperm = upload(m, iperm.data(), iperm.size(), &rc);
+        if (!rc) m->inc_ptr = upload(m, ip.data(), ip.size(), &rc);
+        if (!rc) m->sptr = upload(m, sptr.data(), sptr.size(), &rc);
+        m->nbr = (int *)alloc(sizeof(int) * m->nsell);
+        m->sell_edge = (int *)alloc(sizeof(int) * m->nsell);
+        m->d.isx = (double *)alloc(sizeof(double) * m->nsell);
+        m->d.isy = (double *)alloc(sizeof(double) * m->nsell);
+        m->d.isz = (double *)alloc(sizeof(double) * m->nsell);
+        unsigned long long *dfound = nullptr;
+        if (!rc) dfound = scratch(m, found, 2, tmp, &rc);
+        if (!rc) {
+            IncidenceInput in{};
+            in.edge = scratch(m, d->edge, 2 * (size_t)E, tmp, &rc);
+            if (!rc) in.earea = scratch(m, d->edge_area, 3 * (size_t)E, tmp, &rc);
+            if (!rc) in.bedge = scratch(m, d->bedge, 2 * (size_t)B, tmp, &rc);
+            if (!rc) in.barea = scratch(m, d->bedge_area, 3 * (size_t)B, tmp, &rc);
+            in.fill = (int *)alloc(sizeof(int) * (size_t)N);
+            if (in.fill) tmp.push_back(in.fill);
+            in.bad = dfound;
+            if (!rc && hipMemsetAsync(in.fill, 0, sizeof(int) * (size_t)N, m->stream) != hipSuccess)
+                rc = cfd_set_error(ctx, CFD_E_HIP, "hipMemsetAsync failed");
+            if (!rc) rc = launch_incidences(m, in);
+        }
+        if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = cfd_set_error(ctx, CFD_E_HIP, "incidence lists");
+        if (!rc && cfd_memcpy(found, dfound, sizeof(found[0]), hipMemcpyDeviceToHost) != hipSuccess)
+            rc = cfd_set_error(ctx, CFD_E_HIP, "hipMemcpy failed");
+        rc = free_scratch(m, tmp, rc);
+        if (!rc && found[0] != ~0ull)
+            rc = cfd_set_error(ctx, CFD_E_ARG, "cfd_mesh_create: n2n lists do not match the edges at node %d",
+                               order[found[0]]);
+        if (rc) {
+            cfd_mesh_destroy(m);
+            return rc;
+        }
+        phase("incidence lists");
         // BSR pattern, Create_CRS_SolverBlockMatrix (Euler3D/src/Solver.cpp:612-675):
         // row i holds i and its neighbours in ascending column order.
         m->h_ia.assign(N + 1, 0);
@@ -535,49 +486,24 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             }
         });
         phase("bsr pattern");
-        // BSR block of the off-diagonal (row of the node, column of the neighbour)
-        HostArray<int> off(inc.size());  // every entry written below (unless a neighbour is missing)
-        std::vector<int> missing(N, -1);  // per node: a neighbour missing from its n2n list
-        cfd_parallel_for(N, [&](int64_t i0, int64_t i1) {
-            for (int ii = (int)i0; ii < (int)i1; ii++) {
-                const int i = order[ii];
-                for (int k = ip[ii]; k < ip[ii + 1]; k++) {
-                    if (inc[k].x >= N) {
-                        off[k] = -1;
-                        continue;
-                    }
-                    const int j = order[inc[k].x];
-                    auto b0 = m->h_ja.begin() + m->h_ia[i], b1 = m->h_ja.begin() + m->h_ia[i + 1];
-                    auto it = std::lower_bound(b0, b1, j);
-                    if (it == b1 || *it != j) {
-                        missing[ii] = j;
-                        break;
-                    }
-                    off[k] = (int)(it - m->h_ja.begin());
-                }
-            }
-        });
-        for (int ii = 0; ii < N; ii++)
-            if (missing[ii] >= 0) {
-                const int i = order[ii], j = missing[ii];
-                cfd_mesh_destroy(m);
-                return cfd_set_error(ctx, CFD_E_ARG, "cfd_mesh_create: edge (%d,%d) missing from n2n lists", i, j);
-            }
-        HostArray<int> soff(m->nsell);
-        cfd_parallel_for(
-            nsl,
-            [&](int64_t s0, int64_t s1) {
-                for (int sl = (int)s0; sl < (int)s1; sl++) {
-                    const int w = (sptr[sl + 1] - sptr[sl]) / kSlice;
-                    for (int l = 0; l < kSlice; l++) {
-                        const int i = sl * kSlice + l;
-                        const int cnt = i < N ? ip[i + 1] - ip[i] : 0;
-                        for (int k = 0; k < w; k++)
-                            soff[(size_t)sptr[sl] + (size_t)k * kSlice + l] = k < cnt ? off[ip[i] + k] : -1;
-                    }
-                }
-            },
-            64);
+        // BSR block of each incidence's off-diagonal (row of the node, column of the neighbour)
+        m->ia = upload(m, m->h_ia.data(), m->h_ia.size(), &rc);
+        if (!rc) m->ja = upload(m, m->h_ja.data(), m->h_ja.size(), &rc, kIluPad);
+        if (!rc) m->iau = upload(m, m->h_iau.data(), m->h_iau.size(), &rc);
+        m->soff = (int *)alloc(sizeof(int) * m->nsell);
+        if (!rc) dfound = scratch(m, found + 1, 1, tmp, &rc);
+        if (!rc) rc = launch_off_slots(m, dfound);
+        if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = cfd_set_error(ctx, CFD_E_HIP, "off-diagonal slots");
+        if (!rc && cfd_memcpy(found + 1, dfound, sizeof(found[1]), hipMemcpyDeviceToHost) != hipSuccess)
+            rc = cfd_set_error(ctx, CFD_E_HIP, "hipMemcpy failed");
+        rc = free_scratch(m, tmp, rc);
+        if (!rc && found[1] != ~0ull)
+            rc = cfd_set_error(ctx, CFD_E_ARG, "cfd_mesh_create: edge (%d,%d) missing from n2n lists",
+                               order[(size_t)(found[1] >> 32)], (int)(uint32_t)found[1]);
+        if (rc) {
+            cfd_mesh_destroy(m);
+            return rc;
+        }
         phase("off-diagonal slots");
         std::vector<int> lrows, urows;
         build_levels(m->h_ia, m->h_ja, m->h_iau, N, false, m->lower.ptr, lrows, m->lower.maxwidth);
@@ -677,29 +603,28 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         }
         phase("multicolour: levels");
         // neighbour lists (reference order within each list), internal numbering
-        std::vector<int> nia(N + 1, 0), nja((size_t)d->n2n_ia[N]);
+        std::vector<int> nia(N + 1, 0);
         for (int ii = 0; ii < N; ii++) nia[ii + 1] = nia[ii] + (d->n2n_ia[order[ii] + 1] - d->n2n_ia[order[ii]]);
-        cfd_parallel_for(N, [&](int64_t i0, int64_t i1) {
-            for (int ii = (int)i0; ii < (int)i1; ii++) {
-                const int i = order[ii];
-                int k = nia[ii];
-                for (int q = d->n2n_ia[i]; q < d->n2n_ia[i + 1]; q++) nja[k++] = iperm[d->n2n_ja[q]];
-            }
-        });
+        m->n2n_ia = upload(m, nia.data(), nia.size(), &rc);
+        m->n2n_ja = (int *)alloc(sizeof(int) * (size_t)d->n2n_ia[N]);
+        if (!rc) {
+            const int *const ria = scratch(m, d->n2n_ia, (size_t)N + 1, tmp, &rc);
+            const int *const rja = rc ? nullptr : scratch(m, d->n2n_ja, (size_t)d->n2n_ia[N], tmp, &rc);
+            if (!rc) rc = launch_neighbours(m, ria, rja);
+        }
 
         // packed node records: q (freestream), coordinates
-        HostArray<double> qa((size_t)kQA * m->NT);
-        std::vector<double> sa((size_t)4 * B, 0.0), vol(N);
-        double q5[5];
-        freestream_q(p, q5);
-        cfd_parallel_for(m->NT, [&](int64_t i0, int64_t i1) {
-            for (int i = (int)i0; i < (int)i1; i++) {
-                for (int k = 0; k < 5; k++) qa[(size_t)kQA * i + k] = q5[k];
-                for (int k = 0; k < 3; k++)  // ghost records hold no coordinates
-                    qa[(size_t)kQA * i + 5 + k] = i < N ? d->xyz[3 * (size_t)order[i] + k] : 0.0;
-                if (i < N) vol[i] = d->vol[order[i]];
-            }
-        });
+        m->d.qa = (double *)alloc(sizeof(double) * (size_t)kQA * m->NT);
+        m->d.vol = (double *)alloc(sizeof(double) * (size_t)N);
+        if (!rc) {
+            double q5[5];
+            freestream_q(p, q5);
+            const double *const xyz = scratch(m, d->xyz, 3 * (size_t)N, tmp, &rc);
+            const double *const vol = rc ? nullptr : scratch(m, d->vol, (size_t)N, tmp, &rc);
+            if (!rc) rc = launch_node_records(m, xyz, vol, q5);
+        }
+        rc = free_scratch(m, tmp, rc);
+        std::vector<double> sa((size_t)4 * B, 0.0);
         for (int b = 0; b < B; b++)
             for (int k = 0; k < 3; k++) sa[4 * (size_t)b + k] = d->bedge_area[3 * (size_t)b + k];
         std::vector<int> bnode(B), btag(B, 0);
@@ -709,50 +634,23 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         }
 
         phase("node records");
-        m->order = upload(m, order.data(), order.size(), &rc);
-        if (!rc) m->inc_ptr = upload(m, ip.data(), ip.size(), &rc);
-        if (!rc) m->sptr = upload(m, sptr.data(), sptr.size(), &rc);
-        if (!rc) m->nbr = upload(m, nbr.data(), nbr.size(), &rc);
-        if (!rc) m->soff = upload(m, soff.data(), soff.size(), &rc);
-        if (!rc) m->d.isx = upload(m, isx.data(), isx.size(), &rc);
-        if (!rc) m->d.isy = upload(m, isy.data(), isy.size(), &rc);
-        if (!rc) m->d.isz = upload(m, isz.data(), isz.size(), &rc);
-        if (!rc) m->iperm = upload(m, iperm.data(), iperm.size(), &rc);
-        if (!rc) m->n2n_ia = upload(m, nia.data(), nia.size(), &rc);
-        if (!rc) m->n2n_ja = upload(m, nja.data(), nja.size(), &rc);
         if (!rc) m->bnode = upload(m, bnode.data(), bnode.size(), &rc);
         if (!rc) m->btype = upload(m, d->bedge_type, (size_t)B, &rc);
         if (!rc) m->btag = upload(m, btag.data(), btag.size(), &rc);
-        if (!rc) m->d.qa = upload(m, qa.data(), qa.size(), &rc);
         if (!rc) m->d.sa = upload(m, sa.data(), sa.size(), &rc);
-        if (!rc) m->d.vol = upload(m, vol.data(), vol.size(), &rc);
-        if (!rc) m->ia = upload(m, m->h_ia.data(), m->h_ia.size(), &rc);
-        if (!rc) m->ja = upload(m, m->h_ja.data(), m->h_ja.size(), &rc, kIluPad);
-        if (!rc) m->iau = upload(m, m->h_iau.data(), m->h_iau.size(), &rc);
         if (!rc) m->mc_perm = upload(m, mperm.data(), mperm.size(), &rc);
         if (!rc) m->mc_ia = upload(m, mia.data(), mia.size(), &rc);
         if (!rc) m->mc_ja = upload(m, mja.data(), mja.size(), &rc, kIluPad);
         if (!rc) m->mc_iau = upload(m, miau.data(), miau.size(), &rc);
         if (!rc) m->mc_src = upload(m, msrc.data(), msrc.size(), &rc);
         phase("uploads");
-        if (!rc) {  // block-SELL patterns of A and of the multicolour factors
-            std::vector<int> off;
-            HostArray<int> col(0), src(0);
-            const std::vector<int> &hia = m->h_ia;
-            build_block_sell(N, [&](int i) { return hia[i]; }, [&](int i) { return hia[i + 1]; }, m->h_ja.data(), off, col,
-                             src);
-            rc = upload_block_sell(m, off, col, src, m->a_sell);
-            if (!rc) {
-                build_block_sell(N, [&](int t) { return mia[t]; }, [&](int t) { return miau[t]; }, mja.data(), off, col,
-                                 src);
-                rc = upload_block_sell(m, off, col, src, m->mcl_sell);
-            }
-            if (!rc) {
-                build_block_sell(N, [&](int t) { return miau[t] + 1; }, [&](int t) { return mia[t + 1]; }, mja.data(), off,
-                                 col, src);
-                rc = upload_block_sell(m, off, col, src, m->mcu_sell);
-            }
-        }
+        // block-SELL patterns of A and of the multicolour factors
+        if (!rc)
+            rc = make_block_sell(m, BsrPart::kAll, m->h_ia.data(), m->h_iau.data(), m->ia, m->iau, m->ja, m->a_sell);
+        if (!rc)
+            rc = make_block_sell(m, BsrPart::kLower, mia.data(), miau.data(), m->mc_ia, m->mc_iau, m->mc_ja, m->mcl_sell);
+        if (!rc)
+            rc = make_block_sell(m, BsrPart::kUpper, mia.data(), miau.data(), m->mc_ia, m->mc_iau, m->mc_ja, m->mcu_sell);
         phase("block-sell");
         if (!rc) m->mc_lower.rows = upload(m, mlrows.data(), mlrows.size(), &rc);
         if (!rc) m->mc_upper.rows = upload(m, murows.data(), murows.size(), &rc);
@@ -841,7 +739,7 @@ extern "C" int64_t cfd_footprint_bytes(int32_t N, int32_t E, int32_t B, int32_t 
     // order, inverse order, inc_ptr, sptr, n2n lists, boundary node/type/tag, Roe-pass candidates and block
     // flags, risk
     bytes += 4 * (n + n + (n + 1) + (n / kSlice + 2) + (n + 1) + 2 * e + 3 * b + 2 * n + (n / 4096 + 1) + 1);
-    bytes += nsell * (4 + 4 + 3 * 8);                       // nbr, soff, isx, isy, isz
+    bytes += nsell * (4 + 4 + 4 + 3 * 8);                   // nbr, soff, edge index, isx, isy, isz
     bytes += 4 * ((n + 1) + nnz + n);                       // BSR ia, ja, iau
     bytes += 4 * (n + (n + 1) + 2 * nnz + n + 2 * n);       // multicolour pattern, slot map, levels
     bytes += s * 6 * 5 * n;                                 // work vectors of the sweeps
@@ -948,6 +846,9 @@ int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order) {
         CFD_HIP(m, cfd_memcpy(ip.data(), m->inc_ptr, sizeof(int) * ip.size(), hipMemcpyDeviceToHost));
         CFD_HIP(m, cfd_memcpy(sptr.data(), m->sptr, sizeof(int) * sptr.size(), hipMemcpyDeviceToHost));
         CFD_HIP(m, cfd_memcpy(nbr.data(), m->nbr, sizeof(int) * nbr.size(), hipMemcpyDeviceToHost));
+        const bool by_edge = order == kPatchEdgeOrder;
+        HostArray<int> edge(by_edge ? m->nsell : 0);
+        if (by_edge) CFD_HIP(m, cfd_memcpy(edge.data(), m->sell_edge, sizeof(int) * edge.size(), hipMemcpyDeviceToHost));
         CFD_HIP(m, cfd_memcpy(sx.data(), m->d.isx, sizeof(double) * sx.size(), hipMemcpyDeviceToHost));
         CFD_HIP(m, cfd_memcpy(sy.data(), m->d.isy, sizeof(double) * sy.size(), hipMemcpyDeviceToHost));
         CFD_HIP(m, cfd_memcpy(sz.data(), m->d.isz, sizeof(double) * sz.size(), hipMemcpyDeviceToHost));
@@ -957,7 +858,6 @@ int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order) {
         // index (edge order: interior edges by index, then boundary edges by
         // index, the order of each node's incidence list, along which its
         // slots then ascend)
-        const bool by_edge = order == kPatchEdgeOrder;
         struct Work {
             int key, l, r;
             size_t inc;
@@ -974,14 +874,14 @@ int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order) {
                             const size_t x = sell(i, k);
                             const int jr = nbr[x];
                             if (jr >= N) {
-                                w.push_back({by_edge ? m->h_sell_edge[x] : i - n0, i, jr, x});
+                                w.push_back({by_edge ? edge[x] : i - n0, i, jr, x});
                                 continue;
                             }
                             const bool isL = jr >= 0;
                             const int j = isL ? jr : ~jr;
                             const bool inside = j >= n0 && j < n1;
                             if (inside && !isL) continue;  // taken from its L end
-                            const int key = by_edge ? m->h_sell_edge[x] : (inside ? std::min(i, j) : i) - n0;
+                            const int key = by_edge ? edge[x] : (inside ? std::min(i, j) : i) - n0;
                             w.push_back({key, isL ? i : j, isL ? j : i, x});
                         }
                     }

@@ -238,9 +238,9 @@ struct cfd_mesh {
     // set per work-edge order (kPatchNodeOrder for the fast build,
     // kPatchEdgeOrder for the exact build)
     PatchSet patch[2];
-    // host, SELL as nbr: the reference edge index of each incidence (E + b for
+    // SELL as nbr: the reference edge index of each incidence (E + b for
     // boundary edge b; -1 for padding), which orders kPatchEdgeOrder's work edges
-    HostArray<int> h_sell_edge{0};
+    int *sell_edge = nullptr;
 
     ResidualBufs<double> d;   // FP64
     ResidualBufs<float> f;    // FP32 (allocated on first use)
@@ -433,6 +433,21 @@ CFD_RES_LAUNCHERS
 }  // namespace res_fast
 #undef CFD_RES_LAUNCHERS
 using namespace res_exact;
+
+// Layouts of a new mesh (layout.hip), filled on its stream from lists that the
+// host put on the device.
+struct IncidenceInput {
+    const int *edge, *bedge;       // node pairs in the caller's numbering
+    const double *earea, *barea;   // area vectors
+    int *fill;                     // [N] zeros
+    unsigned long long *bad;       // ~0: the smallest internal node whose list does not fit the edges
+};
+int launch_incidences(cfd_mesh *m, const IncidenceInput &in);   // nbr, d.isx.., sell_edge
+int launch_off_slots(cfd_mesh *m, unsigned long long *miss);    // soff; miss ~0: first (node << 32 | neighbour) missing
+enum class BsrPart { kAll, kLower, kUpper };                    // slots of a row: all, before and after the diagonal
+int launch_block_sell(cfd_mesh *m, BsrPart part, const int *ia, const int *iau, const int *ja, const BlockSell &bs);
+int launch_neighbours(cfd_mesh *m, const int *ref_ia, const int *ref_ja);  // n2n_ja
+int launch_node_records(cfd_mesh *m, const double *xyz, const double *vol, const double *q5);  // d.qa, d.vol
 
 int launch_jacobian(cfd_mesh *m, const cfd_params *p, int rhs_mode, int mixed);
 // The Jacobian of one step of the steady loop (cfd_solve_steady, batches).

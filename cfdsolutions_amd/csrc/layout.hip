@@ -1,0 +1,264 @@
+// Device side of mesh creation: the sliced and blocked layouts that the
+// kernels read are filled on the GPU from the caller's lists, which cross to
+// the device once and as they are.  The host keeps what is sequential (orders,
+// row offsets, colours, levels).
+//
+// Every kernel here moves each entry once and is bound by memory.  What they
+// replace was bound by the host: for 16 cases of 48k nodes (763k nodes, 5.1M
+// edges) cfd_mesh_create took 192 ms, with host passes over fresh pages and
+// 0.75 GB of uploads, and takes 96 ms, with 0.39 GB of uploads and 1.6 ms in
+// the kernels of this file.
+#include "cfd_internal.h"
+
+namespace {
+
+constexpr int kBlock = 256;
+
+// An incidence while its node's list is put in order: twice the index of the
+// edge (E + b for boundary edge b), plus one at the R end of an interior edge.
+__device__ __forceinline__ uint32_t inc_key(int e, int side) { return 2 * (uint32_t)e + (uint32_t)side; }
+
+struct IncArgs {
+    int N, E, B;
+    const int *edge, *bedge;       // caller's numbering
+    const double *earea, *barea;
+    const int *iperm, *ip, *sptr;
+    int *fill;                     // [N] incidences found (starts at zero)
+    uint32_t *key;                 // SELL, becomes the edge indices
+    int *nbr;
+    double *sx, *sy, *sz;
+    unsigned long long *bad;       // smallest internal node whose list does not fit its edges (starts at ~0)
+};
+
+// Each edge enters itself in the lists of its nodes, in any order.
+__global__ __launch_bounds__(kBlock) void k_inc_edges(IncArgs a) {
+    const int t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= a.E + a.B) return;
+    const bool inner = t < a.E;
+    for (int side = 0; side < (inner ? 2 : 1); side++) {
+        const int i = a.iperm[inner ? a.edge[2 * (size_t)t + side] : a.bedge[2 * (size_t)(t - a.E)]];
+        const int k = atomicAdd(&a.fill[i], 1);
+        if (k < a.ip[i + 1] - a.ip[i])
+            a.key[(size_t)a.sptr[i / kSlice] + (size_t)kSlice * k + i % kSlice] = inc_key(t, side);
+    }
+}
+
+// Lists up to this length are sorted in LDS (one column a lane: tetrahedral
+// meshes have 14 neighbours a node), longer ones by the whole wavefront where
+// they are.
+constexpr int kSortLds = 32;
+
+// Ascending sort of v[kSlice * k], k < n, by a workgroup of one wavefront:
+// bitonic merges whose comparators all put the larger word behind, so words
+// past n (larger than any) stay where they are and need not exist.
+__device__ void wave_sort(uint32_t *v, uint32_t n) {
+    auto order2 = [&](uint32_t lo, uint32_t hi) {
+        if (hi >= n) return;
+        uint32_t &a = v[(size_t)kSlice * lo], &b = v[(size_t)kSlice * hi];
+        const uint32_t x = a, y = b;
+        if (y < x) {
+            a = y;
+            b = x;
+        }
+    };
+    uint32_t n2 = 1;
+    while (n2 < n) n2 *= 2;
+    for (uint32_t size = 2; size <= n2; size *= 2) {
+        const uint32_t half = size / 2;
+        for (uint32_t p = threadIdx.x; p < n2 / 2; p += kSlice) {
+            const uint32_t g = p / half * size, j = p % half;
+            order2(g + j, g + size - 1 - j);
+        }
+        __syncthreads();
+        for (uint32_t stride = half / 2; stride; stride /= 2) {
+            for (uint32_t p = threadIdx.x; p < n2 / 2; p += kSlice) {
+                const uint32_t lo = p / stride * 2 * stride + p % stride;
+                order2(lo, lo + stride);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// One wavefront a slice, one lane a node, so the layout is written in full
+// lines: the node's list in edge order with neighbour and area vector.
+__global__ __launch_bounds__(kSlice) void k_inc_lists(IncArgs a) {
+    __shared__ uint32_t col[kSortLds][kSlice];
+    const int sl = blockIdx.x, i = sl * kSlice + threadIdx.x;
+    const size_t base = (size_t)a.sptr[sl] + threadIdx.x;
+    const int w = (a.sptr[sl + 1] - a.sptr[sl]) / kSlice;
+    int cnt = i < a.N ? a.ip[i + 1] - a.ip[i] : 0;
+    if (i < a.N && a.fill[i] != cnt) {
+        atomicMin(a.bad, (unsigned long long)i);
+        cnt = 0;
+    }
+    const bool lds = cnt <= kSortLds;
+    if (lds) {
+        for (int k = 0; k < cnt; k++) {
+            const uint32_t x = a.key[base + (size_t)kSlice * k];
+            int q = k;
+            for (; q > 0 && col[q - 1][threadIdx.x] > x; q--) col[q][threadIdx.x] = col[q - 1][threadIdx.x];
+            col[q][threadIdx.x] = x;
+        }
+    }
+    for (uint64_t hubs = __ballot(!lds); hubs; hubs &= hubs - 1) {
+        const int l = __ffsll((unsigned long long)hubs) - 1;
+        wave_sort(a.key + a.sptr[sl] + l, (uint32_t)__shfl(cnt, l));
+    }
+    for (int k = 0; k < w; k++) {
+        const size_t x = base + (size_t)kSlice * k;
+        int nb = 0, e = -1;  // padding, never read
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+        if (k < cnt) {
+            const uint32_t key = lds ? col[k][threadIdx.x] : a.key[x];
+            e = (int)(key >> 1);
+            const double *S;
+            if (e >= a.E) {
+                nb = a.N + (e - a.E);
+                S = a.barea + 3 * (size_t)(e - a.E);
+            } else {
+                const int side = key & 1, j = a.iperm[a.edge[2 * (size_t)e + 1 - side]];
+                nb = side ? ~j : j;
+                S = a.earea + 3 * (size_t)e;
+            }
+            s0 = S[0];
+            s1 = S[1];
+            s2 = S[2];
+        }
+        a.key[x] = (uint32_t)e;
+        a.nbr[x] = nb;
+        a.sx[x] = s0;
+        a.sy[x] = s1;
+        a.sz[x] = s2;
+    }
+}
+
+// BSR block (row of the node, column of the neighbour) of each incidence.
+// miss: (node << 32 | neighbour) of the first node, and of its first
+// neighbour, without one (starts at ~0).
+__global__ __launch_bounds__(kBlock) void k_off_slots(int N, const int *__restrict__ ip, const int *__restrict__ sptr,
+                                                      const int *__restrict__ nbr, const int *__restrict__ order,
+                                                      const int *__restrict__ ia, const int *__restrict__ ja,
+                                                      int *__restrict__ soff, unsigned long long *miss) {
+    const int ii = blockIdx.x * kBlock + threadIdx.x, sl = ii / kSlice;
+    if (sl >= (N + kSlice - 1) / kSlice) return;
+    const size_t base = (size_t)sptr[sl] + ii % kSlice;
+    const int w = (sptr[sl + 1] - sptr[sl]) / kSlice;
+    const int cnt = ii < N ? ip[ii + 1] - ip[ii] : 0;
+    const int i = ii < N ? order[ii] : 0;
+    const int b0 = ia[i], b1 = ia[i + 1];
+    bool whole = true;
+    for (int k = 0; k < w; k++) {
+        const size_t x = base + (size_t)kSlice * k;
+        int slot = -1;
+        if (k < cnt && nbr[x] < N) {
+            const int j = order[nbr[x] < 0 ? ~nbr[x] : nbr[x]];
+            int lo = b0, hi = b1;
+            while (lo < hi) {
+                const int mid = lo + (hi - lo) / 2;
+                if (ja[mid] < j) lo = mid + 1;
+                else hi = mid;
+            }
+            if (lo < b1 && ja[lo] == j) {
+                slot = lo;
+            } else if (whole) {
+                atomicMin(miss, (unsigned long long)ii << 32 | (unsigned)j);
+                whole = false;
+            }
+        }
+        soff[x] = slot;
+    }
+}
+
+// Block-SELL pattern of the slots first(i) .. last(i)-1 of each row: column 0
+// and source -1 in padding.
+__global__ __launch_bounds__(kBlock) void k_block_sell(int n, BsrPart part, const int *__restrict__ ia,
+                                                       const int *__restrict__ iau, const int *__restrict__ ja,
+                                                       const int *__restrict__ off, int *__restrict__ col,
+                                                       int *__restrict__ src) {
+    const int i = blockIdx.x * kBlock + threadIdx.x, sl = i / 64;
+    if (sl >= (n + 63) / 64) return;
+    const int w = (off[sl + 1] - off[sl]) / 64;
+    int b = 0, e = 0;
+    if (i < n) {
+        b = part == BsrPart::kUpper ? iau[i] + 1 : ia[i];
+        e = part == BsrPart::kLower ? iau[i] : ia[i + 1];
+    }
+    for (int k = 0; k < w; k++) {
+        const size_t q = (size_t)off[sl] + 64 * (size_t)k + i % 64;
+        const bool in = k < e - b;
+        col[q] = in ? ja[b + k] : 0;
+        src[q] = in ? b + k : -1;
+    }
+}
+
+// Neighbour lists in internal numbering, the order within a list unchanged.
+__global__ __launch_bounds__(kBlock) void k_neighbours(int N, const int *__restrict__ order,
+                                                       const int *__restrict__ iperm, const int *__restrict__ ria,
+                                                       const int *__restrict__ rja, const int *__restrict__ nia,
+                                                       int *__restrict__ nja) {
+    const int ii = blockIdx.x * kBlock + threadIdx.x;
+    if (ii >= N) return;
+    const int r = ria[order[ii]], b = nia[ii], n = nia[ii + 1] - b;
+    for (int k = 0; k < n; k++) nja[b + k] = iperm[rja[r + k]];
+}
+
+struct Five {
+    double v[5];
+};
+
+// Node records: freestream state, coordinates (none in ghosts), and volumes.
+__global__ __launch_bounds__(kBlock) void k_node_records(int N, int NT, const int *__restrict__ order,
+                                                         const double *__restrict__ xyz,
+                                                         const double *__restrict__ vref, Five q,
+                                                         double *__restrict__ qa, double *__restrict__ vol) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= NT) return;
+    const int r = i < N ? order[i] : 0;
+    for (int k = 0; k < 5; k++) qa[(size_t)kQA * i + k] = q.v[k];
+    for (int k = 0; k < 3; k++) qa[(size_t)kQA * i + 5 + k] = i < N ? xyz[3 * (size_t)r + k] : 0.0;
+    if (i < N) vol[i] = vref[r];
+}
+
+inline dim3 blocks(int64_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
+
+}  // namespace
+
+int launch_incidences(cfd_mesh *m, const IncidenceInput &in) {
+    IncArgs a{m->N, m->E, m->B, in.edge, in.bedge, in.earea, in.barea, m->iperm, m->inc_ptr, m->sptr, in.fill,
+              (uint32_t *)m->sell_edge, m->nbr, m->d.isx, m->d.isy, m->d.isz, in.bad};
+    if (m->E + m->B) hipLaunchKernelGGL(k_inc_edges, blocks((int64_t)m->E + m->B), dim3(kBlock), 0, m->stream, a);
+    hipLaunchKernelGGL(k_inc_lists, dim3((m->N + kSlice - 1) / kSlice), dim3(kSlice), 0, m->stream, a);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}
+
+int launch_off_slots(cfd_mesh *m, unsigned long long *miss) {
+    hipLaunchKernelGGL(k_off_slots, blocks(m->N), dim3(kBlock), 0, m->stream, m->N, m->inc_ptr, m->sptr, m->nbr,
+                       m->order, m->ia, m->ja, m->soff, miss);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}
+
+int launch_block_sell(cfd_mesh *m, BsrPart part, const int *ia, const int *iau, const int *ja, const BlockSell &bs) {
+    hipLaunchKernelGGL(k_block_sell, blocks(m->N), dim3(kBlock), 0, m->stream, m->N, part, ia, iau, ja, bs.off, bs.col,
+                       bs.src);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}
+
+int launch_neighbours(cfd_mesh *m, const int *ref_ia, const int *ref_ja) {
+    hipLaunchKernelGGL(k_neighbours, blocks(m->N), dim3(kBlock), 0, m->stream, m->N, m->order, m->iperm, ref_ia, ref_ja,
+                       m->n2n_ia, m->n2n_ja);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}
+
+int launch_node_records(cfd_mesh *m, const double *xyz, const double *vol, const double *q5) {
+    Five q;
+    for (int k = 0; k < 5; k++) q.v[k] = q5[k];
+    hipLaunchKernelGGL(k_node_records, blocks(m->NT), dim3(kBlock), 0, m->stream, m->N, m->NT, m->order, xyz, vol, q,
+                       m->d.qa, m->d.vol);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}

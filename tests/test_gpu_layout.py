@@ -1,0 +1,98 @@
+"""Layouts that mesh creation fills on the device, on node graphs at the edges of its kernels: fewer nodes than a slice,
+slices that are not full, lists that are empty, of the longest length sorted by one lane (32), just above it, of a
+power of two and far above, edges in arbitrary order, several boundary edges on a node.
+
+The incidence lists are seen through the Green-Gauss gradient, which sums over them in edge order, the neighbour lists
+and node records through the least-squares gradient: both follow the oracle's operation order, so they are equal bit
+for bit.
+"""
+import types
+
+import numpy as np
+import pytest
+
+from cfdsolutions_amd import cfd
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = cfd.Context(0)
+    yield c
+    c.close()
+
+
+def star_mesh(n, degrees, seed=3):
+    """A chain of n nodes; degrees[k]: incidences of the k-th hub, five of them boundary edges; edges shuffled."""
+    rng = np.random.default_rng(seed)
+    e = {(i, i + 1) for i in range(n - 1)}
+    hubs = [(k + 1) * n // (len(degrees) + 1) for k in range(len(degrees))]
+    for h, deg in zip(hubs, degrees):
+        mine = {x for x in e if h in x}
+        for j in rng.permutation(n):
+            if len(mine) >= deg - 5:
+                break
+            if j != h and j not in hubs:
+                mine.add((int(min(h, j)), int(max(h, j))))
+        e |= mine
+    e = np.array(sorted(e), np.int32).reshape(-1, 2)
+    rng.shuffle(e)
+    both = np.concatenate([e, e[:, ::-1]])
+    both = both[np.lexsort((both[:, 1], both[:, 0]))]
+    ia = np.concatenate([[0], np.cumsum(np.bincount(both[:, 0], minlength=n))]).astype(np.int32)
+    bn = np.repeat(np.array(hubs or [0], np.int32), 5)
+    rng.shuffle(bn)
+    return types.SimpleNamespace(
+        n_node=n, edge=e, edge_area=rng.standard_normal((len(e), 3)),
+        bedge=np.stack([bn, n + np.arange(bn.size, dtype=np.int32)], 1), bedge_area=rng.standard_normal((bn.size, 3)),
+        bedge_type=np.zeros(bn.size, np.int32), bedge_tag=np.ones(bn.size, np.int32),
+        xyz=rng.standard_normal((n, 3)), vol=rng.uniform(0.5, 2.0, n), n2n_ia=ia, n2n_ja=both[:, 1].astype(np.int32))
+
+
+CASES = [(1, []), (2, []), (63, [7]), (64, [32]), (65, [33]), (300, [31, 32, 33, 64, 65]), (3000, [127, 128, 129, 2500])]
+
+
+def same(a, b, what):  # (NaN where a node's neighbours do not span space)
+    assert np.array_equal(a, b, equal_nan=True), what
+
+
+@pytest.mark.parametrize("n,degrees", CASES, ids=[f"{n}-{max(d, default=0)}" for n, d in CASES])
+def test_layouts_match_oracle(ctx, n, degrees):
+    print("layouts", n, degrees, flush=True)
+    m = star_mesh(n, degrees)
+    om = orc.Mesh(m.xyz, m.edge, m.edge_area, m.bedge, m.bedge_area, m.bedge_type, m.vol, m.n2n_ia, m.n2n_ja)
+    dm = cfd.DeviceMesh(ctx, m, cfd.make_params())
+    try:
+        if degrees:
+            counts = np.diff(m.n2n_ia) + np.bincount(m.bedge[:, 0], minlength=n)
+            assert sorted(counts)[-len(degrees):] == sorted(degrees)
+        rng = np.random.default_rng(n)
+        q = dm.get(cfd.FIELD_Q)
+        q *= 1.0 + 0.1 * rng.standard_normal(q.shape)
+        dm.set(cfd.FIELD_Q, q)
+        for gradient, ref in ((cfd.GRAD_GG, orc.gg_gradient), (cfd.GRAD_LSQ, orc.lsq_gradient)):
+            dm.gradient(cfd.make_params(order=2, gradient=gradient))
+            same(dm.get(cfd.FIELD_GRAD), ref(om, q), ref.__name__)
+        ia, ja, iau = dm.bsr_structure()
+        oia, oja, oiau = orc.bsr_structure(om)
+        assert np.array_equal(ia, oia) and np.array_equal(ja, oja) and np.array_equal(iau, oiau)
+    finally:
+        dm.close()
+
+
+def test_lists_that_do_not_fit_are_refused(ctx):
+    """An edge whose end has no room in its node's list, and one whose nodes do not list each other."""
+    m = star_mesh(300, [40])
+    m.edge = m.edge.copy()
+    k = int(np.flatnonzero((m.edge == [10, 11]).all(1))[0])
+    m.edge[k] = (10, 12)  # node 11 is one short, node 12 one over
+    with pytest.raises(cfd.CfdError, match="do not match the edges at node 1[12]"):
+        cfd.DeviceMesh(ctx, m, cfd.make_params())
+    m = star_mesh(300, [40])
+    a, b = (int(np.flatnonzero((m.edge == x).all(1))[0]) for x in ([10, 11], [20, 21]))
+    m.edge = m.edge.copy()
+    m.edge[a], m.edge[b] = (10, 20), (11, 21)  # every count fits, the neighbours do not
+    with pytest.raises(cfd.CfdError, match="missing from n2n lists"):
+        cfd.DeviceMesh(ctx, m, cfd.make_params())
