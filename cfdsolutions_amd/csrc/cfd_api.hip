@@ -414,6 +414,7 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             for (int sl = 0; sl < nsl; sl++) {
                 int w = 0;
                 for (int i = sl * kSlice; i < std::min(N, (sl + 1) * kSlice); i++) w = std::max(w, ip[i + 1] - ip[i]);
+                m->widest = std::max(m->widest, w);
                 tot += (int64_t)kSlice * w;
                 if (tot > INT32_MAX) {
                     cfd_mesh_destroy(m);
@@ -803,9 +804,11 @@ int cfd_ensure_fp32(cfd_mesh *m) {
 // bit: the node is R), which is the order of its incidence list: each node
 // adds its fluxes in the reference's order.  Patches hold kPatch consecutive
 // nodes, restarting at every case of a union.
+//
+// Work edges in node order are placed by kernels (4.17M nodes: 6 ms, host:
+// 800 ms); edge order needs a sort of each patch, and meshes with a list too
+// long for the kernels are rare: both stay on the host.
 // ---------------------------------------------------------------------------
-constexpr int kPatch = 256;  // nodes per patch: one per thread of the patch kernel's workgroup
-
 // The fast build runs the flux-once patch kernel at second order; the exact
 // build runs the node-centred kernel, since its patches (whose work edges go
 // in the reference's edge order, giving the same bits) cost a host build of
@@ -825,11 +828,167 @@ int64_t cfd_patch_footprint_bytes(int64_t n, int64_t e, int64_t b, int64_t cases
     return inc * (4 + 4 + 24 + 12) + 4 * nsell + 8 * (n / kPatch + cases + 2);
 }
 
+static int patches_on_device(cfd_mesh *m, PatchSet &ps, const std::vector<int> &pstart) {
+    const int P = (int)pstart.size() - 1;
+    std::vector<void *> tmp;
+    std::vector<int> wptr(P + 1, 0);
+    int rc = 0;
+    PatchBuild a{m->N, P, m->inc_ptr, m->sptr, m->nbr, nullptr, m->d.isx, m->d.isy, m->d.isz};
+    auto alloc = [&](size_t bytes) {
+        void *const v = rc ? nullptr : cfd_dalloc(m, bytes);
+        if (!rc && !v) rc = cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
+        return v;
+    };
+    ps.pn_start = upload(m, pstart.data(), pstart.size(), &rc);
+    a.pstart = ps.pn_start;
+    a.own = (int *)alloc(sizeof(int) * (size_t)m->N);
+    if (a.own) tmp.push_back(a.own);
+    a.cnt = (int *)alloc(sizeof(int) * (size_t)P);
+    if (a.cnt) tmp.push_back(a.cnt);
+    if (!rc) rc = launch_patch_own(m, a);
+    if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = cfd_set_error(m->ctx, CFD_E_HIP, "patch sizes");
+    if (!rc && cfd_memcpy(wptr.data() + 1, a.cnt, sizeof(int) * (size_t)P, hipMemcpyDeviceToHost) != hipSuccess)
+        rc = cfd_set_error(m->ctx, CFD_E_HIP, "hipMemcpy failed");
+    for (int p = 0; p < P; p++) wptr[p + 1] += wptr[p];
+    const size_t W = (size_t)wptr[P];
+    if (!rc) ps.pw_ptr = upload(m, wptr.data(), wptr.size(), &rc);
+    ps.pw_l = (int *)alloc(sizeof(int) * W);
+    ps.pw_r = (int *)alloc(sizeof(int) * W);
+    ps.pn_slot = (int *)alloc(sizeof(int) * m->nsell);
+    ps.ws = (double *)alloc(sizeof(double) * 3 * W);
+    a.wptr = ps.pw_ptr;
+    a.wl = ps.pw_l;
+    a.wr = ps.pw_r;
+    a.slot = ps.pn_slot;
+    a.ws = ps.ws;
+    if (!rc) rc = launch_patch_edges(m, a);
+    rc = free_scratch(m, tmp, rc);
+    if (rc) {  // nothing half made stays
+        for (void *p : {(void *)ps.pn_start, (void *)ps.pw_ptr, (void *)ps.pw_l, (void *)ps.pw_r, (void *)ps.pn_slot,
+                        (void *)ps.ws})
+            cfd_dfree(m, p);
+        ps = PatchSet{};
+        return rc;
+    }
+    ps.npatch = P;
+    ps.npw = (int64_t)W;
+    return CFD_OK;
+}
+
+static int patches_on_host(cfd_mesh *m, PatchSet &ps, const std::vector<int> &pstart, bool by_edge) {
+    const int N = m->N, nsl = (N + kSlice - 1) / kSlice, P = (int)pstart.size() - 1;
+    std::vector<int> ip(N + 1), sptr(nsl + 1);
+    HostArray<int> nbr(m->nsell);  // (downloaded in full)
+    HostArray<double> sx(m->nsell), sy(m->nsell), sz(m->nsell);
+    CFD_HIP(m, hipStreamSynchronize(m->stream));
+    CFD_HIP(m, cfd_memcpy(ip.data(), m->inc_ptr, sizeof(int) * ip.size(), hipMemcpyDeviceToHost));
+    CFD_HIP(m, cfd_memcpy(sptr.data(), m->sptr, sizeof(int) * sptr.size(), hipMemcpyDeviceToHost));
+    CFD_HIP(m, cfd_memcpy(nbr.data(), m->nbr, sizeof(int) * nbr.size(), hipMemcpyDeviceToHost));
+    HostArray<int> edge(by_edge ? m->nsell : 0);
+    if (by_edge) CFD_HIP(m, cfd_memcpy(edge.data(), m->sell_edge, sizeof(int) * edge.size(), hipMemcpyDeviceToHost));
+    CFD_HIP(m, cfd_memcpy(sx.data(), m->d.isx, sizeof(double) * sx.size(), hipMemcpyDeviceToHost));
+    CFD_HIP(m, cfd_memcpy(sy.data(), m->d.isy, sizeof(double) * sy.size(), hipMemcpyDeviceToHost));
+    CFD_HIP(m, cfd_memcpy(sz.data(), m->d.isz, sizeof(double) * sz.size(), hipMemcpyDeviceToHost));
+    auto sell = [&](int i, int k) { return (size_t)sptr[i / kSlice] + (size_t)kSlice * k + i % kSlice; };
+    // work edges of each patch: (key, l, r, incidence of the area vector);
+    // key: the first end in the patch (node order) or the reference edge
+    // index (edge order: interior edges by index, then boundary edges by
+    // index, the order of each node's incidence list, along which its
+    // slots then ascend)
+    struct Work {
+        int key, l, r;
+        size_t inc;
+    };
+    std::vector<std::vector<Work>> pw(P);
+    cfd_parallel_for(
+        P,
+        [&](int64_t p0, int64_t p1) {
+            for (int p = (int)p0; p < (int)p1; p++) {
+                const int n0 = pstart[p], n1 = pstart[p + 1];
+                std::vector<Work> &w = pw[p];
+                for (int i = n0; i < n1; i++) {
+                    for (int k = 0; k < ip[i + 1] - ip[i]; k++) {
+                        const size_t x = sell(i, k);
+                        const int jr = nbr[x];
+                        if (jr >= N) {
+                            w.push_back({by_edge ? edge[x] : i - n0, i, jr, x});
+                            continue;
+                        }
+                        const bool isL = jr >= 0;
+                        const int j = isL ? jr : ~jr;
+                        const bool inside = j >= n0 && j < n1;
+                        if (inside && !isL) continue;  // taken from its L end
+                        const int key = by_edge ? edge[x] : (inside ? std::min(i, j) : i) - n0;
+                        w.push_back({key, isL ? i : j, isL ? j : i, x});
+                    }
+                }
+                // (edge order: the keys are distinct; node order: ties by L, then R)
+                std::sort(w.begin(), w.end(), [](const Work &a, const Work &b) {
+                    return a.key != b.key ? a.key < b.key : (a.l != b.l ? a.l < b.l : a.r < b.r);
+                });
+            }
+        },
+        1);
+    std::vector<int> wptr(P + 1, 0);
+    for (int p = 0; p < P; p++) wptr[p + 1] = wptr[p] + (int)pw[p].size();
+    const int64_t W = wptr[P];
+    HostArray<int> wl(W), wr(W);  // every entry written below
+    HostArray<double> ws(3 * (size_t)W);
+    std::vector<int> slot(m->nsell, 0);
+    bool ok = true;
+    std::vector<char> bad(P, 0);
+    cfd_parallel_for(
+        P,
+        [&](int64_t p0, int64_t p1) {
+            std::vector<int> cnt;
+            for (int p = (int)p0; p < (int)p1; p++) {
+                const int n0 = pstart[p], n1 = pstart[p + 1];
+                // each node's slots, ascending as the work edges are visited in order
+                cnt.assign(n1 - n0, 0);
+                auto add = [&](int i, int v) {
+                    int &c = cnt[i - n0];
+                    if (c < ip[i + 1] - ip[i]) slot[sell(i, c)] = v;
+                    c++;
+                };
+                for (int q = 0; q < (int)pw[p].size(); q++) {
+                    const Work &u = pw[p][q];
+                    const size_t o = (size_t)wptr[p] + q;
+                    wl[o] = u.l;
+                    wr[o] = u.r;
+                    ws[3 * o] = sx[u.inc];
+                    ws[3 * o + 1] = sy[u.inc];
+                    ws[3 * o + 2] = sz[u.inc];
+                    if (u.l >= n0 && u.l < n1) add(u.l, q);
+                    if (u.r >= n0 && u.r < n1) add(u.r, q | (int)0x80000000u);
+                }
+                for (int i = n0; i < n1; i++)
+                    if (cnt[i - n0] != ip[i + 1] - ip[i]) bad[p] = 1;
+            }
+        },
+        1);
+    for (char b : bad) ok = ok && !b;
+    if (!ok) return cfd_set_error(m->ctx, CFD_E_STATE, "work-edge patches do not cover the incidence lists");
+    int rc = 0;
+    ps.pw_ptr = upload(m, wptr.data(), wptr.size(), &rc);
+    if (!rc) ps.pn_start = upload(m, pstart.data(), pstart.size(), &rc);
+    if (!rc) ps.pw_l = upload(m, wl.data(), wl.size(), &rc);
+    if (!rc) ps.pw_r = upload(m, wr.data(), wr.size(), &rc);
+    if (!rc) ps.pn_slot = upload(m, slot.data(), slot.size(), &rc);
+    if (!rc) ps.ws = upload(m, ws.data(), ws.size(), &rc);
+    if (rc) {
+        ps.pw_ptr = nullptr;
+        return rc;
+    }
+    ps.npatch = P;
+    ps.npw = W;
+    return CFD_OK;
+}
+
 int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order) {
     PatchSet &ps = m->patch[order];
     if (!ps.pw_ptr) {
         const auto t0 = std::chrono::steady_clock::now();
-        const int N = m->N, nsl = (N + kSlice - 1) / kSlice;
+        const int N = m->N;
         // patches of kPatch nodes from the start of the mesh, or of each case
         // of a union (so a case's patches, and its sums, are those it has alone)
         std::vector<int> pstart;
@@ -838,125 +997,24 @@ int cfd_ensure_patches(cfd_mesh *m, bool fp32, int order) {
         for (size_t c = 0; c + 1 < cut.size(); c++)
             for (int n = cut[c]; n < cut[c + 1]; n += kPatch) pstart.push_back(n);
         pstart.push_back(N);
-        const int P = (int)pstart.size() - 1;
-        std::vector<int> ip(N + 1), sptr(nsl + 1);
-        HostArray<int> nbr(m->nsell);  // (downloaded in full)
-        HostArray<double> sx(m->nsell), sy(m->nsell), sz(m->nsell);
-        CFD_HIP(m, hipStreamSynchronize(m->stream));
-        CFD_HIP(m, cfd_memcpy(ip.data(), m->inc_ptr, sizeof(int) * ip.size(), hipMemcpyDeviceToHost));
-        CFD_HIP(m, cfd_memcpy(sptr.data(), m->sptr, sizeof(int) * sptr.size(), hipMemcpyDeviceToHost));
-        CFD_HIP(m, cfd_memcpy(nbr.data(), m->nbr, sizeof(int) * nbr.size(), hipMemcpyDeviceToHost));
-        const bool by_edge = order == kPatchEdgeOrder;
-        HostArray<int> edge(by_edge ? m->nsell : 0);
-        if (by_edge) CFD_HIP(m, cfd_memcpy(edge.data(), m->sell_edge, sizeof(int) * edge.size(), hipMemcpyDeviceToHost));
-        CFD_HIP(m, cfd_memcpy(sx.data(), m->d.isx, sizeof(double) * sx.size(), hipMemcpyDeviceToHost));
-        CFD_HIP(m, cfd_memcpy(sy.data(), m->d.isy, sizeof(double) * sy.size(), hipMemcpyDeviceToHost));
-        CFD_HIP(m, cfd_memcpy(sz.data(), m->d.isz, sizeof(double) * sz.size(), hipMemcpyDeviceToHost));
-        auto sell = [&](int i, int k) { return (size_t)sptr[i / kSlice] + (size_t)kSlice * k + i % kSlice; };
-        // work edges of each patch: (key, l, r, incidence of the area vector);
-        // key: the first end in the patch (node order) or the reference edge
-        // index (edge order: interior edges by index, then boundary edges by
-        // index, the order of each node's incidence list, along which its
-        // slots then ascend)
-        struct Work {
-            int key, l, r;
-            size_t inc;
-        };
-        std::vector<std::vector<Work>> pw(P);
-        cfd_parallel_for(
-            P,
-            [&](int64_t p0, int64_t p1) {
-                for (int p = (int)p0; p < (int)p1; p++) {
-                    const int n0 = pstart[p], n1 = pstart[p + 1];
-                    std::vector<Work> &w = pw[p];
-                    for (int i = n0; i < n1; i++) {
-                        for (int k = 0; k < ip[i + 1] - ip[i]; k++) {
-                            const size_t x = sell(i, k);
-                            const int jr = nbr[x];
-                            if (jr >= N) {
-                                w.push_back({by_edge ? edge[x] : i - n0, i, jr, x});
-                                continue;
-                            }
-                            const bool isL = jr >= 0;
-                            const int j = isL ? jr : ~jr;
-                            const bool inside = j >= n0 && j < n1;
-                            if (inside && !isL) continue;  // taken from its L end
-                            const int key = by_edge ? edge[x] : (inside ? std::min(i, j) : i) - n0;
-                            w.push_back({key, isL ? i : j, isL ? j : i, x});
-                        }
-                    }
-                    // (edge order: the keys are distinct; node order: ties by L, then R)
-                    std::sort(w.begin(), w.end(), [](const Work &a, const Work &b) {
-                        return a.key != b.key ? a.key < b.key : (a.l != b.l ? a.l < b.l : a.r < b.r);
-                    });
-                }
-            },
-            1);
-        std::vector<int> wptr(P + 1, 0);
-        for (int p = 0; p < P; p++) wptr[p + 1] = wptr[p] + (int)pw[p].size();
-        const int64_t W = wptr[P];
-        HostArray<int> wl(W), wr(W);  // every entry written below
-        HostArray<double> ws(3 * (size_t)W);
-        std::vector<int> slot(m->nsell, 0);
-        bool ok = true;
-        std::vector<char> bad(P, 0);
-        cfd_parallel_for(
-            P,
-            [&](int64_t p0, int64_t p1) {
-                std::vector<int> cnt;
-                for (int p = (int)p0; p < (int)p1; p++) {
-                    const int n0 = pstart[p], n1 = pstart[p + 1];
-                    // each node's slots, ascending as the work edges are visited in order
-                    cnt.assign(n1 - n0, 0);
-                    auto add = [&](int i, int v) {
-                        int &c = cnt[i - n0];
-                        if (c < ip[i + 1] - ip[i]) slot[sell(i, c)] = v;
-                        c++;
-                    };
-                    for (int q = 0; q < (int)pw[p].size(); q++) {
-                        const Work &u = pw[p][q];
-                        const size_t o = (size_t)wptr[p] + q;
-                        wl[o] = u.l;
-                        wr[o] = u.r;
-                        ws[3 * o] = sx[u.inc];
-                        ws[3 * o + 1] = sy[u.inc];
-                        ws[3 * o + 2] = sz[u.inc];
-                        if (u.l >= n0 && u.l < n1) add(u.l, q);
-                        if (u.r >= n0 && u.r < n1) add(u.r, q | (int)0x80000000u);
-                    }
-                    for (int i = n0; i < n1; i++)
-                        if (cnt[i - n0] != ip[i + 1] - ip[i]) bad[p] = 1;
-                }
-            },
-            1);
-        for (char b : bad) ok = ok && !b;
-        if (!ok) return cfd_set_error(m->ctx, CFD_E_STATE, "work-edge patches do not cover the incidence lists");
-        int rc = 0;
-        ps.pw_ptr = upload(m, wptr.data(), wptr.size(), &rc);
-        if (!rc) ps.pn_start = upload(m, pstart.data(), pstart.size(), &rc);
-        if (!rc) ps.pw_l = upload(m, wl.data(), wl.size(), &rc);
-        if (!rc) ps.pw_r = upload(m, wr.data(), wr.size(), &rc);
-        if (!rc) ps.pn_slot = upload(m, slot.data(), slot.size(), &rc);
-        if (!rc) ps.ws = upload(m, ws.data(), ws.size(), &rc);
-        if (rc) {
-            ps.pw_ptr = nullptr;
-            return rc;
-        }
-        ps.npatch = P;
-        ps.npw = W;
+        const bool dev = order == kPatchNodeOrder && m->widest <= kPatchDeviceList;
+        const int rc = dev ? patches_on_device(m, ps, pstart) : patches_on_host(m, ps, pstart, order == kPatchEdgeOrder);
+        if (rc) return rc;
         if (cfd_progress())
-            fprintf(stderr, "cfd_ensure_patches: %d patches, %lld work edges (%s order) %8.3f s\n", P, (long long)W,
+            fprintf(stderr, "cfd_ensure_patches: %d patches, %lld work edges (%s order) %8.3f s\n", ps.npatch,
+                    (long long)ps.npw,
                     order == kPatchEdgeOrder ? "edge" : "node",
                     std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
     }
     if (fp32 && !ps.ws_f) {
-        std::vector<double> ws(3 * (size_t)ps.npw);
-        CFD_HIP(m, hipStreamSynchronize(m->stream));
-        CFD_HIP(m, cfd_memcpy(ws.data(), ps.ws, sizeof(double) * ws.size(), hipMemcpyDeviceToHost));
-        std::vector<float> wf(ws.begin(), ws.end());
-        int rc = 0;
-        ps.ws_f = upload(m, wf.data(), wf.size(), &rc);
-        if (rc) return rc;
+        float *const wf = (float *)cfd_dalloc(m, sizeof(float) * 3 * (size_t)ps.npw);
+        if (!wf) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
+        const int rc = launch_to_float(m, 3 * (size_t)ps.npw, ps.ws, wf);
+        if (rc) {
+            cfd_dfree(m, wf);
+            return rc;
+        }
+        ps.ws_f = wf;
     }
     return CFD_OK;
 }

@@ -187,6 +187,7 @@ struct BlockSell {
 //   kPatchEdgeOrder: by reference edge index, boundary edges last, so each
 //     node adds its fluxes in the reference's order (the exact build).
 constexpr int kPatchNodeOrder = 0, kPatchEdgeOrder = 1;
+constexpr int kPatch = 256;  // nodes per patch: one per thread of the patch kernel's workgroup
 struct PatchSet {
     int npatch = 0;
     int64_t npw = 0;
@@ -222,6 +223,7 @@ struct cfd_mesh {
     int *nbr = nullptr;       // [sptr[last]]
     int *soff = nullptr;      // [sptr[last]] BSR block (row of the node, column of the neighbour), -1 for ghosts
     size_t nsell = 0;
+    int widest = 0;           // longest incidence list
     int *n2n_ia = nullptr, *n2n_ja = nullptr;
     int *bnode = nullptr, *btype = nullptr, *btag = nullptr;  // [B]
     // Roe pressure correction: bit n of roe_cand[a] set where node a's test
@@ -447,6 +449,25 @@ int launch_off_slots(cfd_mesh *m, unsigned long long *miss);    // soff; miss ~0
 enum class BsrPart { kAll, kLower, kUpper };                    // slots of a row: all, before and after the diagonal
 int launch_block_sell(cfd_mesh *m, BsrPart part, const int *ia, const int *iau, const int *ja, const BlockSell &bs);
 int launch_neighbours(cfd_mesh *m, const int *ref_ia, const int *ref_ja);  // n2n_ja
+// Work-edge patches in node order, built in two passes: own and cnt from the
+// incidence lists, then (wptr: offsets from cnt) the arrays of the PatchSet.
+struct PatchBuild {
+    int N, P;
+    const int *ip, *sptr, *nbr, *pstart;
+    const double *sx, *sy, *sz;
+    int *own, *cnt;  // [N], [P]
+    const int *wptr;
+    int *wl, *wr, *slot;
+    double *ws;
+};
+int launch_patch_own(cfd_mesh *m, const PatchBuild &a);
+int launch_patch_edges(cfd_mesh *m, const PatchBuild &a);  // lists of at most kPatchDeviceList incidences
+int launch_to_float(cfd_mesh *m, size_t n, const double *in, float *out);
+// A lane keeps its node's slots in LDS and counts through its neighbours'
+// lists, which takes the square of a list's length; 128 slots a lane fill
+// 32 KB.  Meshes of tetrahedra and hexahedra have lists of 14 to 40; one with
+// a longer list is left to the host, whose sort does not mind.
+constexpr int kPatchDeviceList = 128;
 int launch_node_records(cfd_mesh *m, const double *xyz, const double *vol, const double *q5);  // d.qa, d.vol
 
 int launch_jacobian(cfd_mesh *m, const cfd_params *p, int rhs_mode, int mixed);

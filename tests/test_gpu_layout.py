@@ -96,3 +96,36 @@ def test_lists_that_do_not_fit_are_refused(ctx):
     m.edge[a], m.edge[b] = (10, 20), (11, 21)  # every count fits, the neighbours do not
     with pytest.raises(cfd.CfdError, match="missing from n2n lists"):
         cfd.DeviceMesh(ctx, m, cfd.make_params())
+
+
+@pytest.mark.parametrize("n,degrees", [(5, []), (300, [31, 33, 65]), (1500, [127, 128]), (1500, [129, 200])],
+                         ids=["5", "300", "device-widest", "host"])
+def test_patches_match_node_kernel(ctx, n, degrees, monkeypatch):
+    """Work-edge patches in node order, whose lists are made on the device up to 128 incidences: each flux once against
+    each node's own fluxes.  The two sum the same terms in different orders and round each flux differently: of d
+    incidences, within (64 + d) 2^-52 of the sum of |area| times the largest flux (below 16 for these states)."""
+    print("patches", n, degrees, flush=True)
+    m = star_mesh(n, degrees)
+    p = cfd.make_params(mach=0.5, flux="roe", order=2, limiter=cfd.LIM_NONE, arith=cfd.ARITH_FAST)
+    dm = cfd.DeviceMesh(ctx, m, p)
+    try:
+        rng = np.random.default_rng(n)
+        q = dm.get(cfd.FIELD_Q)
+        q *= 1.0 + 0.02 * rng.uniform(-1.0, 1.0, q.shape)
+        dm.set(cfd.FIELD_Q, q)
+        dm.set(cfd.FIELD_GRAD, np.zeros((15, n)))
+        out = {}
+        for once in ("0", "1"):
+            monkeypatch.setenv("CFD_FLUX_ONCE", once)
+            dm.residual(p)
+            out[once] = [dm.get(f) for f in (cfd.FIELD_RES_CONV, cfd.FIELD_RES_DISS)]
+    finally:
+        dm.close()
+    area, deg = np.zeros(n), np.zeros(n)
+    for ends, s in ((m.edge[:, 0], m.edge_area), (m.edge[:, 1], m.edge_area), (m.bedge[:, 0], m.bedge_area)):
+        np.add.at(area, ends, np.linalg.norm(s, axis=1))
+        np.add.at(deg, ends, 1)
+    tol = (64 + deg) * 2.0**-52 * area * 16
+    for a, b in zip(out["1"], out["0"]):
+        assert np.all(np.isfinite(b)) and np.any(b != 0.0)
+        assert np.all(np.abs(a - b) <= tol)
