@@ -515,7 +515,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         // multicolour ordering for ILU(0): greedy colouring of the node graph in
         // reference order; rows sorted by (colour, index)
         std::vector<int> mperm(N), mia(N + 1, 0), miau(N), mlrows, murows;
-        HostArray<int> mja(m->nnz), msrc(m->nnz);  // filled in full below
         {
             // Greedy colouring in reference order.  The cases of a union hold
             // ascending node ranges with no edge between them, so each range
@@ -578,27 +577,33 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             for (int c = 0; c < nc; c++) m->mc_cstart[c + 1] = cnt[c];  // cnt[c] now ends colour c
             for (int t = 0; t < N; t++) miperm[mperm[t]] = t;
             for (int t = 0; t < N; t++) mia[t + 1] = mia[t] + (m->h_ia[mperm[t] + 1] - m->h_ia[mperm[t]]);
-            cfd_parallel_for(N, [&](int64_t t0, int64_t t1) {
-                std::vector<std::pair<int, int>> row;
-                for (int t = (int)t0; t < (int)t1; t++) {
-                    const int oi = mperm[t];
-                    row.clear();
-                    for (int k = m->h_ia[oi]; k < m->h_ia[oi + 1]; k++) row.push_back({miperm[m->h_ja[k]], k});
-                    std::sort(row.begin(), row.end());
-                    int k2 = mia[t];
-                    for (auto &e : row) {
-                        if (e.first == t) miau[t] = k2;
-                        mja[k2] = e.first;
-                        msrc[k2] = e.second;
-                        k2++;
-                    }
-                }
-            });
+            m->mc_perm = upload(m, mperm.data(), mperm.size(), &rc);
+            if (!rc) m->mc_ia = upload(m, mia.data(), mia.size(), &rc);
+            m->mc_ja = (int *)alloc(sizeof(int) * ((size_t)m->nnz + kIluPad));
+            m->mc_src = (int *)alloc(sizeof(int) * (size_t)m->nnz);
+            m->mc_iau = (int *)alloc(sizeof(int) * (size_t)N);
+            // a row's lower neighbours hold every earlier colour (it took the
+            // first one free), so the lower sweep's levels are the colours
+            m->mc_lower.ptr = m->mc_cstart;
+            mlrows.resize(N);
+            for (int t = 0; t < N; t++) mlrows[t] = t;
+            for (int c = 0; c < nc; c++)
+                m->mc_lower.maxwidth = std::max(m->mc_lower.maxwidth, m->mc_cstart[c + 1] - m->mc_cstart[c]);
+            std::vector<int> lev(N);
+            int *const dperm = rc ? nullptr : scratch(m, miperm.data(), miperm.size(), tmp, &rc);
+            int *const dlev = rc ? nullptr : scratch(m, lev.data(), lev.size(), tmp, &rc);
+            if (!rc) rc = launch_mc_pattern(m, dperm, dlev);
+            if (!rc && hipStreamSynchronize(m->stream) != hipSuccess) rc = cfd_set_error(ctx, CFD_E_HIP, "colours");
+            if (!rc && (cfd_memcpy(lev.data(), dlev, sizeof(int) * (size_t)N, hipMemcpyDeviceToHost) != hipSuccess ||
+                        cfd_memcpy(miau.data(), m->mc_iau, sizeof(int) * (size_t)N, hipMemcpyDeviceToHost) != hipSuccess))
+                rc = cfd_set_error(ctx, CFD_E_HIP, "hipMemcpy failed");
+            rc = free_scratch(m, tmp, rc);
+            if (rc) {
+                cfd_mesh_destroy(m);
+                return rc;
+            }
             phase("multicolour: pattern");
-            build_levels_by_colour(mia.data(), mja.data(), miau.data(), N, false, m->mc_cstart, m->mc_lower.ptr, mlrows,
-                                   m->mc_lower.maxwidth);
-            build_levels_by_colour(mia.data(), mja.data(), miau.data(), N, true, m->mc_cstart, m->mc_upper.ptr, murows,
-                                   m->mc_upper.maxwidth);
+            group_by_level(lev, N, m->mc_upper.ptr, murows, m->mc_upper.maxwidth);
             m->mc_lower.nlevels = (int)m->mc_lower.ptr.size() - 1;
             m->mc_upper.nlevels = (int)m->mc_upper.ptr.size() - 1;
         }
@@ -639,11 +644,6 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         if (!rc) m->btype = upload(m, d->bedge_type, (size_t)B, &rc);
         if (!rc) m->btag = upload(m, btag.data(), btag.size(), &rc);
         if (!rc) m->d.sa = upload(m, sa.data(), sa.size(), &rc);
-        if (!rc) m->mc_perm = upload(m, mperm.data(), mperm.size(), &rc);
-        if (!rc) m->mc_ia = upload(m, mia.data(), mia.size(), &rc);
-        if (!rc) m->mc_ja = upload(m, mja.data(), mja.size(), &rc, kIluPad);
-        if (!rc) m->mc_iau = upload(m, miau.data(), miau.size(), &rc);
-        if (!rc) m->mc_src = upload(m, msrc.data(), msrc.size(), &rc);
         phase("uploads");
         // block-SELL patterns of A and of the multicolour factors
         if (!rc)

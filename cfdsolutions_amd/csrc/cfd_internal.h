@@ -448,6 +448,8 @@ int launch_incidences(cfd_mesh *m, const IncidenceInput &in);   // nbr, d.isx..,
 int launch_off_slots(cfd_mesh *m, unsigned long long *miss);    // soff; miss ~0: first (node << 32 | neighbour) missing
 enum class BsrPart { kAll, kLower, kUpper };                    // slots of a row: all, before and after the diagonal
 int launch_block_sell(cfd_mesh *m, BsrPart part, const int *ia, const int *iau, const int *ja, const BlockSell &bs);
+// mc_ja, mc_iau, mc_src from mc_perm (iperm: its inverse) and mc_ia; lev [N]: levels of the upper sweep
+int launch_mc_pattern(cfd_mesh *m, const int *iperm, int *lev);
 int launch_neighbours(cfd_mesh *m, const int *ref_ia, const int *ref_ja);  // n2n_ja
 // Work-edge patches in node order, built in two passes: own and cnt from the
 // incidence lists, then (wptr: offsets from cnt) the arrays of the PatchSet.

@@ -6,7 +6,7 @@
 // Every kernel here moves each entry once and is bound by memory.  What they
 // replace was bound by the host: for 16 cases of 48k nodes (763k nodes, 5.1M
 // edges) cfd_mesh_create took 192 ms, with host passes over fresh pages and
-// 0.75 GB of uploads, and takes 96 ms, with 0.39 GB of uploads and 1.6 ms in
+// 0.75 GB of uploads, and takes 80 ms, with 0.30 GB of uploads and 2 ms in
 // the kernels of this file.
 #include "cfd_internal.h"
 
@@ -192,6 +192,64 @@ __global__ __launch_bounds__(kBlock) void k_block_sell(int n, BsrPart part, cons
     }
 }
 
+// Multicolour pattern: row t is row perm[t] with its blocks in ascending new
+// column (src: the slot a block comes from; equal columns keep their order).
+// A block's place is the number of blocks before it, counted in LDS by the
+// row's lane, or by the whole wavefront for rows that do not fit.
+__global__ __launch_bounds__(kSlice) void k_mc_pattern(int N, const int *__restrict__ perm,
+                                                       const int *__restrict__ iperm, const int *__restrict__ ia,
+                                                       const int *__restrict__ ja, const int *__restrict__ mia,
+                                                       int *__restrict__ mja, int *__restrict__ miau,
+                                                       int *__restrict__ src) {
+    __shared__ int col[kSortLds][kSlice];
+    const int lane = threadIdx.x, t = blockIdx.x * kSlice + lane;
+    int from = 0, to = 0, n = 0;
+    if (t < N) {
+        from = ia[perm[t]];
+        n = ia[perm[t] + 1] - from;
+        to = mia[t];
+    }
+    const bool lds = n <= kSortLds;
+    if (lds) {
+        for (int k = 0; k < n; k++) col[k][lane] = iperm[ja[from + k]];
+        for (int k = 0; k < n; k++) {
+            const int c = col[k][lane];
+            int q = to;
+            for (int u = 0; u < n; u++) q += col[u][lane] < c || (col[u][lane] == c && u < k);
+            mja[q] = c;
+            src[q] = from + k;
+            if (c == t) miau[t] = q;
+        }
+    }
+    for (uint64_t big = __ballot(!lds); big; big &= big - 1) {
+        const int l = __ffsll((unsigned long long)big) - 1;
+        const int f = __shfl(from, l), m = __shfl(n, l), o = __shfl(to, l), row = blockIdx.x * kSlice + l;
+        for (int k = lane; k < m; k += kSlice) {
+            const int c = iperm[ja[f + k]];
+            int q = o;
+            for (int u = 0; u < m; u++) {
+                const int d = iperm[ja[f + u]];
+                q += d < c || (d == c && u < k);
+            }
+            mja[q] = c;
+            src[q] = f + k;
+            if (c == row) miau[row] = q;
+        }
+    }
+}
+
+// Levels of the upper sweep of the rows [r0, r1) of one colour, the later
+// colours' being there: one more than the largest of the rows it needs.
+__global__ __launch_bounds__(kBlock) void k_mc_levels(int r0, int r1, const int *__restrict__ mia,
+                                                      const int *__restrict__ miau, const int *__restrict__ mja,
+                                                      int *lev) {
+    const int t = r0 + blockIdx.x * kBlock + threadIdx.x;
+    if (t >= r1) return;
+    int l = 0;
+    for (int k = miau[t] + 1; k < mia[t + 1]; k++) l = max(l, lev[mja[k]] + 1);
+    lev[t] = l;
+}
+
 // Neighbour lists in internal numbering, the order within a list unchanged.
 __global__ __launch_bounds__(kBlock) void k_neighbours(int N, const int *__restrict__ order,
                                                        const int *__restrict__ iperm, const int *__restrict__ ria,
@@ -343,6 +401,19 @@ int launch_off_slots(cfd_mesh *m, unsigned long long *miss) {
 int launch_block_sell(cfd_mesh *m, BsrPart part, const int *ia, const int *iau, const int *ja, const BlockSell &bs) {
     hipLaunchKernelGGL(k_block_sell, blocks(m->N), dim3(kBlock), 0, m->stream, m->N, part, ia, iau, ja, bs.off, bs.col,
                        bs.src);
+    CFD_HIP(m, hipGetLastError());
+    return CFD_OK;
+}
+
+int launch_mc_pattern(cfd_mesh *m, const int *iperm, int *lev) {
+    hipLaunchKernelGGL(k_mc_pattern, dim3((m->N + kSlice - 1) / kSlice), dim3(kSlice), 0, m->stream, m->N, m->mc_perm,
+                       iperm, m->ia, m->ja, m->mc_ia, m->mc_ja, m->mc_iau, m->mc_src);
+    for (int c = m->ncolor - 1; c >= 0; c--) {
+        const int r0 = m->mc_cstart[c], r1 = m->mc_cstart[c + 1];
+        if (r1 > r0)
+            hipLaunchKernelGGL(k_mc_levels, blocks(r1 - r0), dim3(kBlock), 0, m->stream, r0, r1, m->mc_ia, m->mc_iau,
+                               m->mc_ja, lev);
+    }
     CFD_HIP(m, hipGetLastError());
     return CFD_OK;
 }

@@ -58,6 +58,24 @@ inline bool build_merge_map_par(const int *ia, const int *ja, const int *iau, in
     return true;
 }
 
+// Rows 0..N-1 by level (ascending row within a level): ptr[l]..ptr[l+1] index
+// rows; maxw is the widest level.
+inline void group_by_level(const std::vector<int> &lev, int N, std::vector<int> &ptr, std::vector<int> &rows,
+                           int &maxw) {
+    int nl = 0;
+    for (int i = 0; i < N; i++) nl = std::max(nl, lev[i] + 1);
+    ptr.assign((size_t)nl + 1, 0);
+    for (int i = 0; i < N; i++) ptr[lev[i] + 1]++;
+    maxw = 0;
+    for (int l = 0; l < nl; l++) {
+        maxw = std::max(maxw, ptr[l + 1]);
+        ptr[l + 1] += ptr[l];
+    }
+    rows.assign((size_t)N, 0);
+    std::vector<int> pos(ptr.begin(), ptr.end() - 1);
+    for (int i = 0; i < N; i++) rows[pos[lev[i]]++] = i;
+}
+
 // Level schedule of the lower (or upper) triangular sweep of a multicolour
 // ordered pattern: rows [cstart[c], cstart[c+1]) have colour c and no block
 // couples two rows of one colour, so a row's lower neighbours all have
@@ -81,16 +99,5 @@ inline void build_levels_by_colour(const int *ia, const int *ja, const int *iau,
             }
         });
     }
-    int nl = 0;
-    for (int i = 0; i < N; i++) nl = std::max(nl, lev[i] + 1);
-    ptr.assign((size_t)nl + 1, 0);
-    for (int i = 0; i < N; i++) ptr[lev[i] + 1]++;
-    maxw = 0;
-    for (int l = 0; l < nl; l++) {
-        maxw = std::max(maxw, ptr[l + 1]);
-        ptr[l + 1] += ptr[l];
-    }
-    rows.assign((size_t)N, 0);
-    std::vector<int> pos(ptr.begin(), ptr.end() - 1);
-    for (int i = 0; i < N; i++) rows[pos[lev[i]]++] = i;
+    group_by_level(lev, N, ptr, rows, maxw);
 }
