@@ -3,7 +3,8 @@
 // block Gauss-Seidel and LU-SGS sweeps, and restarted FGMRES.
 //
 // Row-sequential algorithms (ILU(0), Gauss-Seidel, LU-SGS, triangular solves)
-// run level by level over the dependency DAG of the BSR pattern: rows of one
+// follow the dependency DAG of the BSR pattern, a launch per level or rows
+// handed over inside one launch (see "Row-to-row handover"): rows of one
 // level do not depend on each other and every row performs the same
 // operations in the same order as the sequential CPU code, so factors and
 // sweeps are bit-identical to it.
@@ -504,24 +505,30 @@ __device__ bool inv5(const double *A, double *Ai) {
 // operations of orc_ilu0 on every entry in its order.  Factors in TM; the
 // pivot inverse is computed in FP64.
 //
-// G groups of five lanes share a block row, 12 / G rows to a wavefront: lane r of
-// group g holds row r of the row's blocks g, g + G, ... in registers from the
-// first load to the store (blocks past the kSets of a lane stay in lu, read and
-// written by the lane that owns them).  For the lower block (i, k) every group
-// forms L_ik = A_ik D_k^-1 for itself, finds which of row k's upper columns its own
-// blocks have, and subtracts L_ik U_kj; the updates of one k run side by side.
-// A level's time is that of one row's chain over its lower blocks (narrow
-// levels) or instructions and reads of row k's blocks (wide ones), so narrow
-// levels take one row per wavefront and wide ones three.  With a row's blocks in
+// Up to kIluFewRows rows (k_ilu0_level) G groups of five lanes share a block
+// row, 12 / G rows to a wavefront: lane r of group g holds row r of the row's
+// blocks g, g + G, ... in registers from the first load to the store (blocks
+// past the kSets of a lane stay in lu, read and written by the lane that owns
+// them).  For the lower block (i, k) every group forms L_ik = A_ik D_k^-1 for
+// itself, finds which of row k's upper columns its own blocks have, and
+// subtracts L_ik U_kj; the updates of one k run side by side.  Such a level's
+// time is that of one row's chain over its lower blocks.  With a row's blocks in
 // memory and one group per row, a level of the 48x16x16 mesh took 46 us (FP64,
-// natural order) and 72 us (FP32, multicolour), now 16.6 and 24 us; a colour of
-// 45,625 rows 74 us, now 35; of 815,425 rows 441 us (FP32), now 433, without
-// the pass that copied A into the pattern's order (0.89 ms a factorisation).
+// natural order) and 72 us (FP32, multicolour), now 16.6 and 24 us.
+//
+// Wider levels (k_ilu0_rows) are bound by instructions and by the reads of row
+// k's blocks: five lanes to a row, 12 rows to a wavefront, each lane's row of
+// the blocks in an LDS column of its own.  Colours of 95,000 rows on average:
+// 401 us with three rows to a wavefront as above, now 253 (FP32, 763k rows in 8
+// colours); of 102,000 rows 739, now 523 us (FP64).  A row's blocks are read in
+// flights of five: waiting for each cost 30 us a colour.  Reading the next
+// pivot's blocks and the next update's ahead spilled and lost (384 us).
 // ---------------------------------------------------------------------------
-// One row per wavefront up to this many rows (four wavefronts per SIMD): at
+// One row per wavefront up to kIluNarrowRows (four wavefronts per SIMD): at
 // 1,770 rows of a level 24 us against 30 us with three rows, at 5,700 44 us
-// against 35 us (FP32).
-constexpr int kIluNarrowRows = 4096;
+// against 35 us (FP32).  Three rows up to kIluFewRows: at 6,800 rows 33 us
+// against 37 us with 12 rows, at 13,300 65 us against 53 us.
+constexpr int kIluNarrowRows = 4096, kIluFewRows = 8192;
 template <int G>
 constexpr int kIluSets = (16 + G - 1) / G;
 
@@ -710,6 +717,202 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
     if (in >= 5 && in < 10)
 #pragma unroll
         for (int q = 0; q < 5; q++) dinv[25 * (size_t)i + 5 * q + in - 5] = singular ? TM(0.0) : (TM)m[q];
+}
+
+// The same factorisation with five lanes to a block row, 12 rows to a
+// wavefront: lane r keeps row r of the blocks in its own LDS column, where the
+// block that an update meets can be looked up, so L_ik is formed once, the rows'
+// searches are shared out (lane r compares the columns of blocks r, r + 5, ...)
+// and a row's updates follow each other without idle lanes.
+constexpr int kIluCols = 3, kIluKeep = 5 * kIluCols;  // blocks of a row kept in LDS, the rest stay in lu
+
+template <class TM>
+__global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restrict__ rows, const int *__restrict__ ia,
+                                                  const int *__restrict__ ja, const int *__restrict__ iau,
+                                                  const int *__restrict__ src, const TM *__restrict__ a, TM *lu,
+                                                  TM *dinv, const TM *__restrict__ luk, const TM *__restrict__ dinvk,
+                                                  int *flag) {
+    __shared__ TM keep[kIluKeep][5][60];
+    __shared__ double diag[12][25];
+    const int lane = threadIdx.x, rs = lane / 5, base = 5 * rs, r = lane - base;
+    const int t = blockIdx.x * 12 + rs;
+    const bool active = rs < 12 && t < nrows;
+    const int i = active ? rows[t] : 0;
+    const int b0 = active ? ia[i] : 0, n = active ? ia[i + 1] - b0 : 0, nl = active ? iau[i] - b0 : 0;
+    int col[kIluCols], up[kIluCols], nu[kIluCols];  // of blocks r, r + 5, ..; for lower ones the upper blocks of that row
+#pragma unroll
+    for (int s = 0; s < kIluCols; s++) {
+        const int b = 5 * s + r;
+        col[s] = -1;
+        up[s] = nu[s] = 0;
+        if (b < n) {
+            col[s] = ja[b0 + b];
+            if (b < nl) {
+                up[s] = iau[col[s]] + 1;
+                nu[s] = ia[col[s] + 1] - up[s];
+            }
+        }
+    }
+    // all reads in flight at once: past the row's end its last block again
+    int sl[kIluKeep];
+#pragma unroll
+    for (int b = 0; b < kIluKeep; b++) {
+        const int q = b0 + max(0, min(b, n - 1));
+        sl[b] = src ? src[q] : q;
+    }
+    for (int h = 0; h < kIluCols; h++) {
+        TM A[5][5];
+#pragma unroll
+        for (int b = 0; b < 5; b++)
+#pragma unroll
+            for (int c = 0; c < 5; c++)
+                A[b][c] = a[25 * (size_t)(h == 0 ? sl[b] : h == 1 ? sl[b + 5] : sl[b + 10]) + 5 * r + c];
+        if (lane < 60)
+#pragma unroll
+            for (int b = 0; b < 5; b++)
+#pragma unroll
+                for (int c = 0; c < 5; c++) keep[5 * h + b][c][lane] = A[b][c];
+    }
+    for (int b = kIluKeep; b < n; b++) {
+        const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
+        for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+    }
+    for (int l = 0; l < nl; l++) {  // (the lanes of a row stay together)
+        int k, p0, np;
+        TM Ar[5], L[5], D[25];
+        if (l < kIluKeep) {
+            const int so = l / 5, from = base + l - 5 * so;
+            k = __shfl(so == 0 ? col[0] : so == 1 ? col[1] : col[2], from, 64);
+            p0 = __shfl(so == 0 ? up[0] : so == 1 ? up[1] : up[2], from, 64);
+            np = __shfl(so == 0 ? nu[0] : so == 1 ? nu[1] : nu[2], from, 64);
+#pragma unroll
+            for (int c = 0; c < 5; c++) Ar[c] = keep[l][c][lane];
+        } else {
+            k = ja[b0 + l];
+            p0 = iau[k] + 1;
+            np = ia[k + 1] - p0;
+            for (int c = 0; c < 5; c++) Ar[c] = lu[25 * (size_t)(b0 + l) + 5 * r + c];
+        }
+#pragma unroll
+        for (int q = 0; q < 25; q++) D[q] = dinvk[25 * (size_t)k + q];
+        int hit[kIluCols];
+#pragma unroll
+        for (int s = 0; s < kIluCols; s++) hit[s] = -1;
+        for (int c0 = 0; c0 < np; c0 += kIluPad) {  // (ja is padded by kIluPad entries)
+            int cq[kIluPad];
+#pragma unroll
+            for (int q = 0; q < kIluPad; q++) cq[q] = ja[p0 + c0 + q];
+#pragma unroll
+            for (int q = 0; q < kIluPad; q++)
+#pragma unroll
+                for (int s = 0; s < kIluCols; s++) hit[s] = ((cq[q] == col[s]) & (c0 + q < np)) ? c0 + q : hit[s];
+        }
+        unsigned mask = 0;  // blocks of the row that row k's upper blocks meet
+#pragma unroll
+        for (int s = 0; s < kIluCols; s++) mask |= (unsigned)(__ballot(hit[s] >= 0) >> base & 31) << (5 * s);
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+            TM v = TM(0.0);
+#pragma unroll
+            for (int q = 0; q < 5; q++) v += Ar[q] * D[5 * q + c];
+            L[c] = v;
+        }
+        if (l < kIluKeep) {
+#pragma unroll
+            for (int c = 0; c < 5; c++) keep[l][c][lane] = L[c];
+        } else {
+            for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + l) + 5 * r + c] = L[c];
+        }
+        for (; mask; mask &= mask - 1) {
+            const int b = __ffs(mask) - 1, so = b / 5;
+            const int q = __shfl(so == 0 ? hit[0] : so == 1 ? hit[1] : hit[2], base + b - 5 * so, 64);
+            const TM *U = luk + 25 * (size_t)(p0 + q);
+            TM u[25];
+#pragma unroll
+            for (int z = 0; z < 25; z++) u[z] = U[z];
+#pragma unroll
+            for (int c = 0; c < 5; c++) {
+                TM v = TM(0.0);
+#pragma unroll
+                for (int z = 0; z < 5; z++) v += L[z] * u[5 * z + c];
+                keep[b][c][lane] = keep[b][c][lane] - v;
+            }
+        }
+        for (int b = max(kIluKeep, l + 1); b < n; b++) {
+            TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
+            const int cb = ja[b0 + b];
+            for (int q = 0; q < np; q++) {
+                if (ja[p0 + q] != cb) continue;
+                const TM *U = luk + 25 * (size_t)(p0 + q);
+                for (int c = 0; c < 5; c++) {
+                    TM v = TM(0.0);
+                    for (int z = 0; z < 5; z++) v += L[z] * U[5 * z + c];
+                    B[c] = B[c] - v;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < kIluKeep; b++)
+        if (b < n) {
+            TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
+#pragma unroll
+            for (int c = 0; c < 5; c++) B[c] = keep[b][c][lane];
+        }
+    if (active)
+        for (int c = 0; c < 5; c++)
+            diag[rs][5 * r + c] =
+                (double)(nl < kIluKeep ? keep[nl][c][lane] : lu[25 * (size_t)(b0 + nl) + 5 * r + c]);
+    __syncthreads();
+    // Gauss-Jordan inverse of inv5, columns r of D and of I to a lane: the same
+    // operations on every entry
+    double m[5], w[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        m[q] = active ? diag[rs][5 * q + r] : 0.0;
+        w[q] = r == q ? 1.0 : 0.0;
+    }
+    bool singular = false;
+#pragma unroll
+    for (int c = 0; c < 5; c++) {
+        double p[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) p[q] = __shfl(m[q], base + c, 64);
+        int piv = c;
+        double best = fabs(p[c]);
+#pragma unroll
+        for (int q = c + 1; q < 5; q++) {
+            const double v = fabs(p[q]);
+            if (v > best) {
+                piv = q;
+                best = v;
+            }
+        }
+#pragma unroll
+        for (int q = c + 1; q < 5; q++) {
+            const bool sw = piv == q;
+            const double x = m[c], y = p[c], z = w[c];
+            m[c] = sw ? m[q] : x;
+            m[q] = sw ? x : m[q];
+            p[c] = sw ? p[q] : y;
+            p[q] = sw ? y : p[q];
+            w[c] = sw ? w[q] : z;
+            w[q] = sw ? z : w[q];
+        }
+        singular = singular || p[c] == 0.0;
+        m[c] = m[c] / p[c];
+        w[c] = w[c] / p[c];
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+            if (q != c) {
+                m[q] = m[q] - p[q] * m[c];
+                w[q] = w[q] - p[q] * w[c];
+            }
+    }
+    if (!active) return;
+    if (singular && r == 0) atomicAdd(flag + 2, 1);
+#pragma unroll
+    for (int q = 0; q < 5; q++) dinv[25 * (size_t)i + 5 * q + r] = singular ? TM(0.0) : (TM)w[q];
 }
 
 // Inverse diagonal blocks (block-Jacobi).
@@ -2094,7 +2297,10 @@ void ilu0_levels(cfd_mesh *m, const LevelSchedule &ls, const int *ia, const int 
                        m->stream, nr, ls.rows + b0, ia, ja, iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, \
                        m->flag)
         if (nr <= kIluNarrowRows) CFD_ILU(12);
-        else CFD_ILU(4);
+        else if (nr <= kIluFewRows) CFD_ILU(4);
+        else
+            hipLaunchKernelGGL(k_ilu0_rows<TM>, dim3((nr + 11) / 12), dim3(64), 0, m->stream, nr, ls.rows + b0, ia, ja,
+                               iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, m->flag);
 #undef CFD_ILU
     }
 }

@@ -160,7 +160,8 @@ def multicolour(ia, ja, iau, a, b):
     ("hub", 173, cfd.PREC_ILU0),  # a row of 81 blocks, 40 of them lower: more than a lane group keeps in registers
     ("hub", 173, cfd.PREC_ILU0_MC),
     ("hub", 30000, cfd.PREC_ILU0_MC),  # colours of more rows than the one-row-per-wavefront kernel takes
-    ("random", 30000, cfd.PREC_ILU0_MC)])
+    ("random", 30000, cfd.PREC_ILU0_MC),
+    ("random", 50000, cfd.PREC_ILU0_MC)])  # wide colours, rows of up to 20 blocks with the diagonal anywhere among them
 def test_ilu_factors_equal_oracle(ctx, kind, n, precond):
     """One FGMRES step without restarts gives x = y M^-1 b: its direction is the oracle's preconditioned b.  Each entry
     of b / ||b|| is rounded once, and the systems' inverses amplify that little (dominance 3 per neighbour against row
