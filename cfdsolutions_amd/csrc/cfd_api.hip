@@ -474,6 +474,9 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         m->h_ia.assign(N + 1, 0);
         for (int i = 0; i < N; i++) m->h_ia[i + 1] = m->h_ia[i] + (d->n2n_ia[i + 1] - d->n2n_ia[i]) + 1;
         m->nnz = m->h_ia[N];
+        int over = 0;
+        for (int i = 0; i < N; i++) over += m->h_ia[i + 1] - m->h_ia[i] > kIluKeep;
+        m->ilu_long = over >= std::max(1, N / 16);
         m->h_ja.resize(m->nnz);
         m->h_iau.resize(N);
         cfd_parallel_for(N, [&](int64_t i0, int64_t i1) {

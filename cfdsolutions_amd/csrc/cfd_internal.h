@@ -80,6 +80,7 @@ struct LevelSchedule {
 };
 
 constexpr int kIluPad = 8;       // column entries of the ILU(0) that are read together; ja and mc_ja are padded by as many
+constexpr int kIluKeep = 15;     // blocks of a row that the ILU(0) of wide levels keeps in LDS
 constexpr int kMaxKrylov = 64;   // largest FGMRES restart length
 constexpr int kDotParts = 512;   // partial sums of one Krylov dot product, at most
 // Blocks of 256 threads for a Krylov dot product over n entries: one entry per
@@ -252,6 +253,7 @@ struct cfd_mesh {
     double *dt = nullptr;     // [N]
     int nnz = 0;
     std::vector<int> h_ia, h_ja, h_iau;
+    bool ilu_long = false;    // one row in 16 or more has over kIluKeep blocks
     int *ia = nullptr, *ja = nullptr, *iau = nullptr;
     double *a = nullptr, *b = nullptr, *x = nullptr;
     float *af = nullptr;      // FP32 Jacobian (mixed)

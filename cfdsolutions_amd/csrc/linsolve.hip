@@ -508,8 +508,9 @@ __device__ bool inv5(const double *A, double *Ai) {
 // Up to kIluFewRows rows (k_ilu0_level) G groups of five lanes share a block
 // row, 12 / G rows to a wavefront: lane r of group g holds row r of the row's
 // blocks g, g + G, ... in registers from the first load to the store (blocks
-// past the kSets of a lane stay in lu, read and written by the lane that owns
-// them).  For the lower block (i, k) every group forms L_ik = A_ik D_k^-1 for
+// past the kIluSets of a lane stay in lu, read and written by the lane that owns
+// them; the columns of the next NX are in registers, a row still longer is
+// searched for each of row k's columns).  For the lower block (i, k) every group forms L_ik = A_ik D_k^-1 for
 // itself, finds which of row k's upper columns its own blocks have, and
 // subtracts L_ik U_kj; the updates of one k run side by side.  Such a level's
 // time is that of one row's chain over its lower blocks.  With a row's blocks in
@@ -528,9 +529,45 @@ __device__ bool inv5(const double *A, double *Ai) {
 // 1,770 rows of a level 24 us against 30 us with three rows, at 5,700 44 us
 // against 35 us (FP32).  Three rows up to kIluFewRows: at 6,800 rows 33 us
 // against 37 us with 12 rows, at 13,300 65 us against 53 us.
-constexpr int kIluNarrowRows = 4096, kIluFewRows = 8192;
+//
+// Rows of unstructured meshes are longer and differ in length (Delaunay meshes:
+// 16.5 blocks on average, up to 70), so rows that share a wavefront wait for
+// the longest, and blocks past 15 stay in memory in k_ilu0_rows.  There
+// (cfd_mesh::ilu_long) one row per wavefront is ahead at every width in FP32
+// and up to kIluLongRows rows in FP64.  Delaunay meshes, multicolour, whole
+// factorisation, ms in FP64 / FP32, with the lines of short rows and as it is:
+// 60,000 rows 3.45 / 3.05 and 2.7 / 2.2; 200,000 rows 9.1 / 7.3 and 7.9 / 5.7;
+// 500,000 rows 14.7 / 11.1 and 14.6 / 10.1.
+constexpr int kIluNarrowRows = 4096, kIluFewRows = 8192, kIluLongRows = 32768;
 template <int G>
 constexpr int kIluSets = (16 + G - 1) / G;
+
+// The slot of the row's blocks [b0, b1) that has column c, or -1 (ascending
+// columns).
+__device__ __forceinline__ int find_col(const int *__restrict__ ja, int b0, int b1, int c) {
+    const int end = b1;
+    while (b0 < b1) {
+        const int mid = b0 + (b1 - b0) / 2;
+        if (ja[mid] < c) b0 = mid + 1;
+        else b1 = mid;
+    }
+    return b0 < end && ja[b0] == c ? b0 : -1;
+}
+
+// Row r of a block in memory loses L U (r: row of L).
+template <class TM>
+__device__ __forceinline__ void block_update(TM *B, const TM *L, const TM *__restrict__ U) {
+    TM u[25];
+#pragma unroll
+    for (int z = 0; z < 25; z++) u[z] = U[z];
+#pragma unroll
+    for (int c = 0; c < 5; c++) {
+        TM v = TM(0.0);
+#pragma unroll
+        for (int z = 0; z < 5; z++) v += L[z] * u[5 * z + c];
+        B[c] = B[c] - v;
+    }
+}
 
 template <class TM, int G>
 __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__restrict__ rows,
@@ -542,7 +579,7 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
     // luk / dinvk view the blocks and inverse pivots of rows of earlier
     // levels, which this launch only reads (it writes rows of one level).
     // src: slot of A for each slot of the pattern (NULL: the same).
-    constexpr int NS = kIluSets<G>, RW = 12 / G, W = 5 * G;
+    constexpr int NS = kIluSets<G>, NX = 24 / G, RW = 12 / G, W = 5 * G;
     __shared__ double diag[kBlock / 64][RW][25];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int rs = lane / W, base = rs * W, in = lane - base, g = in / 5, r = in - 5 * g;
@@ -568,9 +605,18 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
             }
         }
     }
-    for (int b = NS * G + g; b < n; b += G) {
-        const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
-        for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+    const bool more = __any(n > NS * G);  // a row has blocks that stay in lu: the columns of the next NX per lane
+    int xcol[NX];
+    if (more) {
+#pragma unroll
+        for (int x = 0; x < NX; x++) {
+            const int b = (NS + x) * G + g;
+            xcol[x] = b < n ? ja[b0 + b] : -1;
+        }
+        for (int b = NS * G + g; b < n; b += G) {
+            const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
+            for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+        }
     }
     for (int l = 0; __any(l < nl); l++) {
         const int so = l / G, from = base + 5 * (l - so * G);
@@ -602,9 +648,11 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
         for (int q = 0; q < 25; q++) D[q] = dinvk[25 * (size_t)k + q];
         // which of row k's upper blocks meets each of this lane's blocks; eight
         // columns at a time (ja is padded by kIluPad entries)
-        int hit[NS];
+        int hit[NS], xhit[NX];
 #pragma unroll
         for (int s = 0; s < NS; s++) hit[s] = -1;
+#pragma unroll
+        for (int x = 0; x < NX; x++) xhit[x] = -1;
         for (int c0 = 0; c0 < np; c0 += kIluPad) {
             int cq[kIluPad];
 #pragma unroll
@@ -613,6 +661,11 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
             for (int q = 0; q < kIluPad; q++)
 #pragma unroll
                 for (int s = 0; s < NS; s++) hit[s] = ((cq[q] == col[s]) & (c0 + q < np)) ? c0 + q : hit[s];
+            if (more)
+#pragma unroll
+                for (int q = 0; q < kIluPad; q++)
+#pragma unroll
+                    for (int x = 0; x < NX; x++) xhit[x] = ((cq[q] == xcol[x]) & (c0 + q < np)) ? c0 + q : xhit[x];
         }
 #pragma unroll
         for (int c = 0; c < 5; c++) {
@@ -640,22 +693,17 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
                 }
             }
         }
-        for (int b = NS * G + g; b < n; b += G) {
-            TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
-            if (b == l) {
-                for (int c = 0; c < 5; c++) B[c] = L[c];
-            } else if (b > l) {
-                const int cb = ja[b0 + b];
-                for (int q = 0; q < np; q++) {
-                    if (ja[p0 + q] != cb) continue;
-                    const TM *U = luk + 25 * (size_t)(p0 + q);
-                    for (int c = 0; c < 5; c++) {
-                        TM v = TM(0.0);
-                        for (int z = 0; z < 5; z++) v += L[z] * U[5 * z + c];
-                        B[c] = B[c] - v;
-                    }
-                }
-            }
+        if (!more) continue;
+        TM *const row = lu + 25 * (size_t)b0 + 5 * r;
+        if (l >= NS * G && l % G == g)
+            for (int c = 0; c < 5; c++) row[25 * (size_t)l + c] = L[c];
+#pragma unroll
+        for (int x = 0; x < NX; x++)
+            if (xhit[x] >= 0) block_update(row + 25 * (size_t)((NS + x) * G + g), L, luk + 25 * (size_t)(p0 + xhit[x]));
+        const int t0 = max((NS + NX) * G, l + 1);  // the blocks past those, sought from row k's side
+        for (int q = 0; t0 < n && q < np; q++) {
+            const int b = find_col(ja, b0 + t0, b0 + n, ja[p0 + q]) - b0;
+            if (b >= t0 && b % G == g) block_update(row + 25 * (size_t)b, L, luk + 25 * (size_t)(p0 + q));
         }
     }
 #pragma unroll
@@ -724,7 +772,8 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
 // block that an update meets can be looked up, so L_ik is formed once, the rows'
 // searches are shared out (lane r compares the columns of blocks r, r + 5, ...)
 // and a row's updates follow each other without idle lanes.
-constexpr int kIluCols = 3, kIluKeep = 5 * kIluCols;  // blocks of a row kept in LDS, the rest stay in lu
+constexpr int kIluCols = kIluKeep / 5;                           // blocks of a row kept in LDS, the rest stay in lu:
+constexpr int kIluMore = 4, kIluSeen = kIluKeep + 5 * kIluMore;  // of these so many have their columns in registers
 
 template <class TM>
 __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restrict__ rows, const int *__restrict__ ia,
@@ -773,9 +822,18 @@ __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restri
 #pragma unroll
                 for (int c = 0; c < 5; c++) keep[5 * h + b][c][lane] = A[b][c];
     }
-    for (int b = kIluKeep; b < n; b++) {
-        const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
-        for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+    const bool more = __any(n > kIluKeep);
+    int xcol[kIluMore];
+    if (more) {
+#pragma unroll
+        for (int x = 0; x < kIluMore; x++) {
+            const int b = kIluKeep + 5 * x + r;
+            xcol[x] = b < n ? ja[b0 + b] : -1;
+        }
+        for (int b = kIluKeep; b < n; b++) {
+            const TM *A = a + 25 * (size_t)(src ? src[b0 + b] : b0 + b) + 5 * r;
+            for (int c = 0; c < 5; c++) lu[25 * (size_t)(b0 + b) + 5 * r + c] = A[c];
+        }
     }
     for (int l = 0; l < nl; l++) {  // (the lanes of a row stay together)
         int k, p0, np;
@@ -795,9 +853,11 @@ __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restri
         }
 #pragma unroll
         for (int q = 0; q < 25; q++) D[q] = dinvk[25 * (size_t)k + q];
-        int hit[kIluCols];
+        int hit[kIluCols], xhit[kIluMore];
 #pragma unroll
         for (int s = 0; s < kIluCols; s++) hit[s] = -1;
+#pragma unroll
+        for (int x = 0; x < kIluMore; x++) xhit[x] = -1;
         for (int c0 = 0; c0 < np; c0 += kIluPad) {  // (ja is padded by kIluPad entries)
             int cq[kIluPad];
 #pragma unroll
@@ -806,6 +866,12 @@ __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restri
             for (int q = 0; q < kIluPad; q++)
 #pragma unroll
                 for (int s = 0; s < kIluCols; s++) hit[s] = ((cq[q] == col[s]) & (c0 + q < np)) ? c0 + q : hit[s];
+            if (more)
+#pragma unroll
+                for (int q = 0; q < kIluPad; q++)
+#pragma unroll
+                    for (int x = 0; x < kIluMore; x++)
+                        xhit[x] = ((cq[q] == xcol[x]) & (c0 + q < np)) ? c0 + q : xhit[x];
         }
         unsigned mask = 0;  // blocks of the row that row k's upper blocks meet
 #pragma unroll
@@ -838,18 +904,20 @@ __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restri
                 keep[b][c][lane] = keep[b][c][lane] - v;
             }
         }
-        for (int b = max(kIluKeep, l + 1); b < n; b++) {
-            TM *B = lu + 25 * (size_t)(b0 + b) + 5 * r;
-            const int cb = ja[b0 + b];
-            for (int q = 0; q < np; q++) {
-                if (ja[p0 + q] != cb) continue;
-                const TM *U = luk + 25 * (size_t)(p0 + q);
-                for (int c = 0; c < 5; c++) {
-                    TM v = TM(0.0);
-                    for (int z = 0; z < 5; z++) v += L[z] * U[5 * z + c];
-                    B[c] = B[c] - v;
-                }
-            }
+        if (!more) continue;
+        TM *const row = lu + 25 * (size_t)b0 + 5 * r;
+        unsigned xmask = 0;  // the same of the blocks in lu
+#pragma unroll
+        for (int x = 0; x < kIluMore; x++) xmask |= (unsigned)(__ballot(xhit[x] >= 0) >> base & 31) << (5 * x);
+        for (; xmask; xmask &= xmask - 1) {
+            const int b = __ffs(xmask) - 1, so = b / 5;
+            const int q = __shfl(so == 0 ? xhit[0] : so == 1 ? xhit[1] : so == 2 ? xhit[2] : xhit[3], base + b - 5 * so, 64);
+            block_update(row + 25 * (size_t)(kIluKeep + b), L, luk + 25 * (size_t)(p0 + q));
+        }
+        const int t0 = max(kIluSeen, l + 1);  // the blocks past those, sought from row k's side
+        for (int q = 0; t0 < n && q < np; q++) {
+            const int b = find_col(ja, b0 + t0, b0 + n, ja[p0 + q]) - b0;
+            if (b >= t0) block_update(row + 25 * (size_t)b, L, luk + 25 * (size_t)(p0 + q));
         }
     }
 #pragma unroll
@@ -2290,13 +2358,14 @@ const float *bsr_a<float>(cfd_mesh *m) { return m->af; }
 template <class TM>
 void ilu0_levels(cfd_mesh *m, const LevelSchedule &ls, const int *ia, const int *ja, const int *iau, const int *src,
                  const TM *a, TM *lu, TM *dinv) {
+    const int narrow = !m->ilu_long ? kIluNarrowRows : sizeof(TM) == 4 ? INT_MAX : kIluLongRows;
     for (int l = 0; l < ls.nlevels; l++) {
         const int b0 = ls.ptr[l], nr = ls.ptr[l + 1] - b0;
 #define CFD_ILU(G)                                                                                                    \
     hipLaunchKernelGGL((k_ilu0_level<TM, G>), dim3((nr + 4 * (12 / G) - 1) / (4 * (12 / G))), dim3(kBlock), 0,         \
                        m->stream, nr, ls.rows + b0, ia, ja, iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, \
                        m->flag)
-        if (nr <= kIluNarrowRows) CFD_ILU(12);
+        if (nr <= narrow) CFD_ILU(12);
         else if (nr <= kIluFewRows) CFD_ILU(4);
         else
             hipLaunchKernelGGL(k_ilu0_rows<TM>, dim3((nr + 11) / 12), dim3(64), 0, m->stream, nr, ls.rows + b0, ia, ja,
