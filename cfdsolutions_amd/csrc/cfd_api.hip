@@ -670,6 +670,9 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             if (!rc) m->upper.slots12 = upload(m, s12.data(), s12.size(), &rc);
             const char *sf = getenv("CFD_SYNC_FREE");
             m->sync_free = !(sf && sf[0] == '0');
+            // any number of workgroups gives the same bits: CFD_FLOW_BLOCKS is for measuring and tests
+            const char *fb = getenv("CFD_FLOW_BLOCKS");
+            m->flow_blocks = fb ? std::max(0, atoi(fb)) : 0;
             const char *gr = getenv("CFD_GRAPHS");
             m->use_graphs = !(gr && gr[0] == '0');
             // one row per lane fills the GPU only with enough rows; smaller
@@ -693,7 +696,7 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         m->risk = (int *)cfd_dalloc(m, sizeof(int));
         m->red = (double *)cfd_dalloc(m, sizeof(double) * 1024 * 65);
         m->redout = (double *)cfd_dalloc(m, sizeof(double) * 4 * 65);
-        m->flag = (int *)cfd_dalloc(m, sizeof(int) * 4);
+        m->flag = (int *)cfd_dalloc(m, sizeof(int) * kFlagWords);
         m->eigbits = (unsigned long long *)cfd_dalloc(m, sizeof(unsigned long long) * 6);
         if (!m->d.qb || !m->d.lsq || !m->d.res || !m->dt || !m->b || !m->x || !m->roe_cand || !m->roe_blk ||
             !m->risk || !m->red || !m->redout || !m->flag || !m->eigbits) {
@@ -707,7 +710,7 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         }
         hipMemsetAsync(m->d.qb, 0, sizeof(double) * kQB * (size_t)N, m->stream);
         hipMemsetAsync(m->roe_blk, 0, sizeof(int) * (size_t)((N + 4095) / 4096), m->stream);
-        hipMemsetAsync(m->flag, 0, sizeof(int) * 4, m->stream);
+        hipMemsetAsync(m->flag, 0, sizeof(int) * kFlagWords, m->stream);
         hipMemsetAsync(m->d.res, 0, sizeof(double) * kRES * (size_t)N, m->stream);
         phase("workspaces");
         rc = launch_lsq_coef(m);
@@ -748,7 +751,7 @@ extern "C" int64_t cfd_footprint_bytes(int32_t N, int32_t E, int32_t B, int32_t 
     bytes += 4 * (n + (n + 1) + 2 * nnz + n + 2 * n);       // multicolour pattern, slot map, levels
     bytes += s * 6 * 5 * n;                                 // work vectors of the sweeps
     bytes += 4 * (2 * n + 4 * n + 4 * 11 * lvl);           // level rows and padded slot lists
-    bytes += 8 * (1024 * 65 + 4 * 65 + 6) + 4 * 4;         // reduction scratch, eigenvalue bits, flags
+    bytes += 8 * (1024 * 65 + 4 * 65 + 6) + 4 * kFlagWords;  // reduction scratch, eigenvalue bits, flags
     bytes += 25 * s * nnz * 2 + 25 * s * n;                 // Jacobian, ILU(0) factors, inverse pivots
     bytes += s * 5 * n * (2 * (int64_t)km + 2) + 8 * 5 * n; // Krylov V, Z, w; FP64 true residual
     // block-SELL copies: A, and the multicolour factors (strict lower + upper

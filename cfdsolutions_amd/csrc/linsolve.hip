@@ -1067,19 +1067,28 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int nrows, const int *__r
 // one word per value: 354 us.)  A result that is itself a NaN is stored as the
 // default NaN, so no result can look unset.
 //
-// Waves take their rows in level order, chunk w, w + W, ... of W waves, and a
-// row reads only rows of earlier chunks (levels are padded to whole chunks), so
-// the earliest unfinished chunk is always being worked on once its wave runs.
-// All waves of a launch have to be resident: a grid is at most a quarter of the
-// workgroups that the GPU holds at the kernel's registers (flow_blocks of the
-// workgroups per CU that its launch bounds ask for), for the four hardware
-// queues that can run sweeps of different streams at a time.  A wait over kSpinMax polls raises flag[3],
-// and every waiter gives up once it is set: a sweep always ends, and the solve
-// reports it.
+// Rows go in chunks of 12 in level order (levels are padded to whole chunks),
+// so a chunk reads only earlier ones.  A running workgroup draws the next four
+// chunks by a ticket when it is done with the last: the earliest unfinished
+// chunk is always held by a wave that runs, whatever else the GPU holds and
+// however many of the launch's workgroups it holds, so a wait always ends.  (A
+// fixed share of the chunks to each workgroup needs every workgroup resident.)
+// A wait over kSpinMax polls raises flag[3], and every waiter gives up once it
+// is set: a sweep ends even where a store is lost, and the solve reports it.
+//
+// flow_blocks: how many workgroups pay depends on how many chunks can run at a
+// time (a level's).  Too few leave loads unissued, too many poll more than they
+// work.  Twenty Arnoldi steps, ms at 128, 256 and 512 workgroups: 6 chunks
+// (48x16x16, natural order, FP64) 15.0, 15.6, 17.2; 33 (120x40x40) 41.8, 42.8,
+// 50.0; 81 (192x64x64) 82.2, 79.8, 97.3; 147 (48x16x16, colours) 2.06, 1.96,
+// 2.16; 333 (Delaunay mesh of 60,000, colours) -, 7.2, 7.8; 475 (72x24x24,
+// colours) 4.80, 3.24, 3.18; 1,088 (95x33x31, colours) -, 6.3, 5.5.
 // ---------------------------------------------------------------------------
 constexpr int kSpinMax = 1 << 22;
-constexpr int kFlowShare = 64;  // a quarter of the 256 CUs
-constexpr int flow_blocks(int per_cu) { return kFlowShare * per_cu; }
+inline int flow_blocks(const cfd_mesh *m, int64_t chunks, int64_t width) {
+    const int64_t n = m->flow_blocks ? m->flow_blocks : width < 60 ? 128 : width < 400 ? 256 : 512;
+    return (int)std::min((chunks + 3) / 4, n);
+}
 
 template <class T>
 struct FlowWord;
@@ -1115,21 +1124,43 @@ template <class T>
 __device__ __forceinline__ void flow_unset(T *p) {
     st_coh(reinterpret_cast<typename FlowWord<T>::U *>(p), FlowWord<T>::unset);
 }
+// Whether poll `it` of a wait was its last: the bound is reached or another
+// wait's was.
+__device__ __forceinline__ bool flow_give_up(int it, int *flag) {
+    if ((it & 255) != 255 || (it < kSpinMax && ld_coh(flag + 3) == 0)) return false;
+    atomicOr(flag + 3, 1);
+    return true;
+}
 // The value of word p, of which v has been read already.
 template <class T>
 __device__ __forceinline__ T flow_wait(const T *p, typename FlowWord<T>::U v, int *flag) {
-    for (int it = 0; v == FlowWord<T>::unset; it++) {
-        if (it >= kSpinMax || ((it & 255) == 255 && ld_coh(flag + 3) != 0)) {
-            atomicOr(flag + 3, 1);
-            break;
-        }
-        v = flow_load(p);
-    }
+    for (int it = 0; v == FlowWord<T>::unset && !flow_give_up(it, flag); it++) v = flow_load(p);
     return __builtin_bit_cast(T, v);
 }
 
+// Chunk tickets of a launch, one to a workgroup for a chunk to each of its
+// wavefronts: for (w = next(); more(total); w = next()), with nothing to do for
+// a wave whose chunk w is not below total.  (Drawn when the chunks are done: the
+// answer of a ticket drawn ahead is waited for with the chunk's own loads, 2.4
+// against 1.7 ms for 20 Gauss-Seidel sweeps of the 48x16x16 mesh.)
+struct FlowTicket {
+    int *const count, *const shared;  // the counter, two words of LDS
+    int n = 0;
+    __device__ __forceinline__ FlowTicket(int *c, int *s) : count(c), shared(s) {}
+    __device__ __forceinline__ int next() {
+        n ^= 1;
+        if (threadIdx.x == 0)
+            shared[n] = (kBlock / 64) * __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        return __builtin_amdgcn_readfirstlane(shared[n] + (int)(threadIdx.x >> 6));
+    }
+    __device__ __forceinline__ bool more(int total) const { return __builtin_amdgcn_readfirstlane(shared[n]) < total; }
+};
+
+// Also sets a launch's ticket counter back (NULL: none).
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_flow_unset(size_t n, T *x) {
+__global__ __launch_bounds__(kBlock) void k_flow_unset(size_t n, T *x, int *ticket) {
+    if (ticket && blockIdx.x == 0 && threadIdx.x == 0) st_coh(ticket, 0);
     for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) flow_unset(x + i);
 }
 
@@ -1176,10 +1207,7 @@ struct FlowBlocks {
 #pragma unroll
             for (int u = 0; u < U; u++) all = all & (v[u] != FlowWord<TV>::unset);
             if (all) return;
-            if (it >= kSpinMax || ((it & 255) == 255 && ld_coh(flag + 3) != 0)) {
-                atomicOr(flag + 3, 1);
-                return;
-            }
+            if (flow_give_up(it, flag)) return;
 #pragma unroll
             for (int u = 0; u < U; u++)
                 if (v[u] == FlowWord<TV>::unset) v[u] = flow_load(x + 5 * (size_t)j[u]);
@@ -1231,9 +1259,7 @@ struct FlowBlocks {
 // sweep and (where P is given) of z in the reference's order.  The other set of
 // words is left unset for the next launch, so nothing is cleared while it is
 // read.  A backward row starts when its own neighbours are done, a product
-// while the last rows still run, and four launches are saved: ten mixed steps on
-// 45,625 rows 36.6 -> 34.3 ms, a step on 14,161 rows 2% (the chain of the
-// colours, 57 us, bounds it).
+// while the last rows still run, and four launches are saved.
 template <class TM, class TV>
 struct FlowStep {
     int nf, nb, np;          // padded rows of the sweeps' schedules, rows of the product (0: none)
@@ -1247,7 +1273,7 @@ struct FlowStep {
     const TM *a;
     TV *words, *other;       // this launch's set of handover words and the next one's
     size_t L;
-    int *flag;
+    int *flag, *ticket, *next_ticket;  // this launch's counter and the next one's, set back here
 };
 
 template <class TM>
@@ -1260,8 +1286,12 @@ __global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_arnoldi_flow(FlowSte
     TV *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<TV>::slot;
     const double denom = f.norm2 ? sqrt(f.norm2[0]) : 1.0;
     const int cf = (f.nf + 11) / 12, cb = (f.nb + 11) / 12, cp = (f.np + 11) / 12;
-    const int nw = gridDim.x * (kBlock / 64);
-    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); w < cf + cb + cp; w += nw) {
+    __shared__ int tickets[2];
+    FlowTicket q(f.ticket, tickets);
+    const int total = cf + cb + cp;
+    for (int w = q.next(); q.more(total); w = q.next()) {
+        if (w == 0 && lane == 0) st_coh(f.next_ticket, 0);
+        if (w >= total) continue;
         FlowBlocks<8, TM, TV> g;
         if (w >= cf + cb) {
             const int i = 12 * (w - cf - cb) + slot;
@@ -1730,12 +1760,11 @@ __device__ __forceinline__ const double *flow_lu(double *sh, int r, const double
 // and sweep s follows `reach` + 1 chunks behind sweep s - 1 instead of waiting
 // for its end (reach: how many chunks ahead an upper neighbour can be,
 // ensure_gs_schedule).  Items (chunk c, sweep s) go in ascending
-// c + s (reach + 1), so each needs only earlier ones.  The chain is about
+// c + s (reach + 1), then s, so each needs only earlier ones.  The chain is about
 // levels + 8 S rows long instead of levels * S: 20 sweeps of the 48x16x16 mesh
-// (205 levels) took 64.3 ms with a launch per level, 2.07 ms so.
+// (205 levels) took 64.3 ms with a launch per level, 1.71 ms so.
 // x0: x before the first sweep.  rowrms[s][i]: row i's sum of sweep s.
-constexpr int kGsPerCu = 2;
-__global__ __launch_bounds__(kBlock, kGsPerCu) void k_gs_flow(int N, int nchunk, int reach, int S, const int *__restrict__ slots,
+__global__ __launch_bounds__(kBlock, 2) void k_gs_flow(int N, int nchunk, int reach, int S, const int *__restrict__ slots,
                                                     const int *__restrict__ ia, const int *__restrict__ ja,
                                                     const int *__restrict__ iau, const double *__restrict__ a,
                                                     const double *__restrict__ b, const double *__restrict__ lu,
@@ -1743,12 +1772,20 @@ __global__ __launch_bounds__(kBlock, kGsPerCu) void k_gs_flow(int N, int nchunk,
     const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
     __shared__ __align__(16) FlowLds<double> lds;
     double *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<double>::slot;
-    const int64_t items = ((int64_t)nchunk + (int64_t)(S - 1) * (reach + 1)) * S;
-    const int nw = gridDim.x * (kBlock / 64);
-    for (int64_t w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); w < items; w += nw) {
-        const int s = (int)(w % S);
-        const int64_t c = w / S - (int64_t)s * (reach + 1);
-        if (c < 0 || c >= nchunk) continue;
+    // step t holds the items (t - s lag, s), lo <= s <= hi; first: the number of items before it
+    const int lag = reach + 1, items = nchunk * S;
+    int t = 0, first = 0, lo = 0, hi = 0;
+    __shared__ int tickets[2];
+    FlowTicket q(flag + kFlagTicket, tickets);
+    for (int w = q.next(); q.more(items); w = q.next()) {
+        if (w >= items) continue;
+        while (w - first > hi - lo) {
+            first += hi - lo + 1;
+            t++;
+            if (hi + 1 < S && t >= (hi + 1) * lag) hi++;
+            if (t >= nchunk + lo * lag) lo++;
+        }
+        const int s = lo + w - first, c = t - s * lag;
         const int i = slot < 12 ? slots[12 * c + slot] : -1;
         const double *prev = s ? ver + (size_t)(s - 1) * 5 * N : x0;
         double *cur = ver + (size_t)s * 5 * N;
@@ -1857,17 +1894,22 @@ __global__ __launch_bounds__(kBlock) void k_lusgs_lu(int N, const int *iau, cons
 // from prev, the result of the half sweep before.  next is left unset for the
 // half sweep after this one.  Half sweeps run in opposite directions, so they
 // do not overlap.
-__global__ __launch_bounds__(kBlock, kGsPerCu) void k_lusgs_flow(int nslots, const int *__restrict__ slots,
+__global__ __launch_bounds__(kBlock, 2) void k_lusgs_flow(int nslots, const int *__restrict__ slots,
                                                        const int *__restrict__ ia, const int *__restrict__ ja,
                                                        const int *__restrict__ iau, const double *__restrict__ a,
                                                        const double *__restrict__ b, const double *__restrict__ lu,
                                                        const int *__restrict__ piv, const double *prev, double *cur,
-                                                       double *next, int backward, int *flag) {
+                                                       double *next, int backward, int *flag, int *ticket,
+                                                       int *next_ticket) {
     const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
     __shared__ __align__(16) FlowLds<double> lds;
     double *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<double>::slot;
-    const int nw = gridDim.x * (kBlock / 64);
-    for (int w = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); 12 * w < nslots; w += nw) {
+    __shared__ int drawn[2];
+    FlowTicket q(ticket, drawn);
+    const int total = (nslots + 11) / 12;
+    for (int w = q.next(); q.more(total); w = q.next()) {
+        if (w == 0 && lane == 0) st_coh(next_ticket, 0);
+        if (w >= total) continue;
         const int t = 12 * w + slot;
         const int i = slot < 12 && t < nslots ? slots[t] : -1;
         const size_t ri = 5 * (size_t)(i >= 0 ? i : 0) + r;
@@ -2063,10 +2105,12 @@ struct GsSums {
 // Block b of the P of a partition: the pass over its entries, then its partial
 // sums (a butterfly within each wavefront, the four wavefront sums in order)
 // into the words of dot k, and in the wavefronts of the last blocks the final
-// sums: lane l adds partials l, l + 64, ... in order, then the butterfly.  They
-// wait only for blocks dispatched before them or with them.  (A launch of its
+// sums: lane l adds partials l, l + 64, ... in order, then the butterfly.  These
+// kGsTail blocks wait for the others, which wait for nothing, so a launch ends
+// on any GPU that holds more than kGsTail blocks of every launch under way.  (A launch of its
 // own for the final sums took 4-5 us, three times per Arnoldi step, and a copy
 // of the sums to the host 3 us.)
+constexpr int kGsTail = 8;
 template <class TV, int NVMAX, GsMode M, int U>
 __device__ __forceinline__ void gs_block(size_t o, int b, int P, size_t n, int nv, const TV *__restrict__ V, size_t ld,
                                          const double *__restrict__ h, TV *__restrict__ w, const GsSums &g,
@@ -2101,7 +2145,9 @@ __device__ __forceinline__ void gs_block(size_t o, int b, int P, size_t n, int n
     __syncthreads();
     for (int k = threadIdx.x; k < nd; k += kBlock)
         flow_store(g.words + (size_t)k * P + b, ((wsum[k][0] + wsum[k][1]) + wsum[k][2]) + wsum[k][3]);
-    for (int k = (P - 1 - b) * (kBlock / 64) + wave; k < nd; k += P * (kBlock / 64)) {
+    const int tail = min(P, kGsTail);
+    if (b < P - tail) return;
+    for (int k = (P - 1 - b) * (kBlock / 64) + wave; k < nd; k += tail * (kBlock / 64)) {
         double *p = g.words + (size_t)k * P;
         double s = 0.0;
         for (int q = lane; q < P; q += 64 * 8) {
@@ -2422,18 +2468,14 @@ void spmv(cfd_mesh *m, const TX *x, TY *y, const double *bsub) {
                            0, m->stream, m->N, m->ia, m->ja, bsr_a<TM>(m), x, y, bsub);
 }
 
-// Whether the sweeps of this preconditioner run in one launch each: always in
-// the natural order (hundreds of levels), in the multicolour order (8 colours
-// on the bump channels) up to kFlowMcRows rows.  There a launch per colour
-// costs more than the handovers; above, all waves of a colour together keep
-// more loads in flight than the resident waves of one launch.  With nothing
-// else changed, whole mixed steps took 4.74 ms against 5.96 ms with a launch
-// per colour at 14,161 rows, 43.1 against 48.7 ms (ten steps) at 45,625 rows,
-// 21.4 against 19.8 ms at 104,448 rows.
-constexpr int kFlowMcRows = 65536;
+// Whether the sweeps of this preconditioner run in one launch: in the natural
+// order (hundreds of levels), and in the multicolour order on the BSR arrays,
+// which meshes below kSellMinRows use.  20 Arnoldi steps with a launch per
+// colour and in one launch, ms in FP64 and FP32: 63,504 rows 5.0 and 3.9, 3.5
+// and 2.7; 104,448 rows 6.6 and 5.5, 5.1 and 4.2; 126,175 rows 7.1 and 6.2, 5.5
+// and 4.9; Delaunay mesh of 100,000 11.2 and 9.0, 9.3 and 7.5.
 bool flow_sweeps(const cfd_mesh *m, int kind) {
-    return m->sync_free &&
-           (kind == CFD_PREC_ILU0 || (kind == CFD_PREC_ILU0_MC && !m->use_sell && m->N <= kFlowMcRows));
+    return m->sync_free && (kind == CFD_PREC_ILU0 || (kind == CFD_PREC_ILU0_MC && !m->use_sell));
 }
 
 template <class TV>
@@ -2640,9 +2682,11 @@ bool flow_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *vj, T
     f.other = set + (1 - (j & 1)) * kFlowWords * L;
     f.L = L;
     f.flag = m->flag;
+    f.ticket = m->flag + kFlagTicket + (j & 1);
+    f.next_ticket = m->flag + kFlagTicket + 1 - (j & 1);
     const int chunks = (f.nf + 11) / 12 + (f.nb + 11) / 12 + (f.np + 11) / 12;
-    hipLaunchKernelGGL((k_arnoldi_flow<TM, TV>), dim3(std::min((chunks + 3) / 4, flow_blocks(kTrsvPerCu<TM>))),
-                       dim3(kBlock), 0, m->stream, f);
+    const int64_t width = m->N / 12 / std::max(1, std::max(lo.nlevels, up.nlevels));
+    hipLaunchKernelGGL((k_arnoldi_flow<TM, TV>), dim3(flow_blocks(m, chunks, width)), dim3(kBlock), 0, m->stream, f);
     return f.np > 0;
 }
 
@@ -2650,7 +2694,8 @@ bool flow_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *vj, T
 template <class TV>
 void flow_begin(cfd_mesh *m) {
     const size_t n = kFlowWords * 5 * (size_t)m->N;
-    hipLaunchKernelGGL(k_flow_unset<TV>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, mc_work<TV>(m));
+    hipLaunchKernelGGL(k_flow_unset<TV>, dim3(grid_cap(n, 4096)), dim3(kBlock), 0, m->stream, n, mc_work<TV>(m),
+                       m->flag + kFlagTicket);
 }
 
 // One Arnoldi step j of FGMRES: V_j = w / ||w|| (j > 0, norm of the previous
@@ -3123,9 +3168,14 @@ static int gs_sweeps(cfd_mesh *m, int sweeps, const LevelSchedule &ls, int reach
     int it = 0;
     for (bool done = false; it < sweeps && !done;) {
         const int S = std::min(g.nver, sweeps - it);
-        hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(S * L, 4096)), dim3(kBlock), 0, m->stream, S * L, g.ver);
-        hipLaunchKernelGGL(k_gs_flow, dim3((int)std::min<int64_t>(((int64_t)nchunk * S + 3) / 4, flow_blocks(kGsPerCu))),
-                           dim3(kBlock), 0, m->stream, m->N, nchunk, reach, S, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, g.lu,
+        // a step's chunks of every sweep under way, five times over for the
+        // longer work on a row: 2.42, 1.93 and 1.71 ms at 128, 256 and 512
+        // workgroups (48x16x16 mesh, 100 chunks), 0.82, 0.86 and 0.97 (24x8x8, 17)
+        const int64_t under = std::min<int64_t>(S, nchunk / (reach + 1) + 1);
+        const int64_t width = 5 * nchunk * under / ls.nlevels;
+        hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(S * L, 4096)), dim3(kBlock), 0, m->stream, S * L, g.ver,
+                           m->flag + kFlagTicket);
+        hipLaunchKernelGGL(k_gs_flow, dim3(flow_blocks(m, (int64_t)nchunk * S, width)), dim3(kBlock), 0, m->stream, m->N, nchunk, reach, S, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, g.lu,
                            m->x, g.ver, g.rows, m->flag);
         // row RMS of each sweep: ordered reduction of the per-row sums
         hipLaunchKernelGGL(k_vsum_partial, dim3(np, S), dim3(kBlock), 0, m->stream, (size_t)m->N, g.rows, m->red);
@@ -3223,14 +3273,15 @@ int run_linsolve(cfd_mesh *m, const cfd_linsolve_opts *o, cfd_linsolve_stats *st
                                m->b, m->x);
             hipLaunchKernelGGL(k_lusgs_lu, dim3((m->N + kBlock - 1) / kBlock), dim3(kBlock), 0, m->stream, m->N, m->iau,
                                m->a, m->gslu, piv);
-            hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(L, 4096)), dim3(kBlock), 0, m->stream, L, ver);
+            hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(L, 4096)), dim3(kBlock), 0, m->stream, L, ver,
+                               m->flag + kFlagTicket);
             // half sweep h writes version h % 3, reads h - 1 and clears h + 1
             for (int h = 0; h < 2 * sweeps; h++) {
                 const LevelSchedule &ls = h % 2 ? m->upper : m->lower;
-                hipLaunchKernelGGL(k_lusgs_flow, dim3(std::min((ls.n12 + 47) / 48, flow_blocks(kGsPerCu))), dim3(kBlock),
-                                   0, m->stream, ls.n12, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, m->gslu, piv,
+                hipLaunchKernelGGL(k_lusgs_flow, dim3(flow_blocks(m, ls.n12 / 12, m->N / 12 / ls.nlevels)),
+                                   dim3(kBlock), 0, m->stream, ls.n12, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, m->gslu, piv,
                                    h ? ver + (h + 2) % 3 * L : m->x, ver + h % 3 * L, ver + (h + 1) % 3 * L, h % 2,
-                                   m->flag);
+                                   m->flag, m->flag + kFlagTicket + h % 2, m->flag + kFlagTicket + 1 - h % 2);
             }
             CFD_HIP(m, hipMemcpyAsync(m->x, ver + (2 * sweeps - 1) % 3 * L, sizeof(double) * L,
                                       hipMemcpyDeviceToDevice, m->stream));
@@ -3341,7 +3392,7 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
     // reductions between linear solves)
     const size_t nw = (size_t)(kMaxKrylov + 1) * (m->ncase ? m->seg_dot.nblocks : dot_parts(5 * (size_t)m->N));
     hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(nw, 4096)), dim3(kBlock), 0, m->stream, nw,
-                       m->ncase ? m->bpart : m->red);
+                       m->ncase ? m->bpart : m->red, (int *)nullptr);
     if (flow_sweeps(m, o->precond)) {
         rc = ensure_slots12(m, m->mc_lower);
         if (!rc) rc = ensure_slots12(m, m->mc_upper);
