@@ -673,6 +673,9 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
             // any number of workgroups gives the same bits: CFD_FLOW_BLOCKS is for measuring and tests
             const char *fb = getenv("CFD_FLOW_BLOCKS");
             m->flow_blocks = fb ? std::max(0, atoi(fb)) : 0;
+            // CFD_SPIN_MAX: lets a test see a wait given up
+            const char *sm = getenv("CFD_SPIN_MAX");
+            if (sm) m->spin_max = std::max(1, atoi(sm));
             const char *gr = getenv("CFD_GRAPHS");
             m->use_graphs = !(gr && gr[0] == '0');
             // one row per lane fills the GPU only with enough rows; smaller
@@ -711,6 +714,7 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         hipMemsetAsync(m->d.qb, 0, sizeof(double) * kQB * (size_t)N, m->stream);
         hipMemsetAsync(m->roe_blk, 0, sizeof(int) * (size_t)((N + 4095) / 4096), m->stream);
         hipMemsetAsync(m->flag, 0, sizeof(int) * kFlagWords, m->stream);
+        hipMemcpyAsync(m->flag + kFlagSpin, &m->spin_max, sizeof(int), hipMemcpyHostToDevice, m->stream);
         hipMemsetAsync(m->d.res, 0, sizeof(double) * kRES * (size_t)N, m->stream);
         phase("workspaces");
         rc = launch_lsq_coef(m);

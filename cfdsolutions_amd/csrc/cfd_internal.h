@@ -81,9 +81,9 @@ struct LevelSchedule {
 
 constexpr int kIluPad = 8;       // column entries of the ILU(0) that are read together; ja and mc_ja are padded by as many
 constexpr int kIluKeep = 15;     // blocks of a row that the ILU(0) of wide levels keeps in LDS
-// Words of cfd_mesh::flag: four error flags, then two chunk tickets of the
-// single-launch sweeps.
-constexpr int kFlagTicket = 4, kFlagWords = 6;
+// Words of cfd_mesh::flag: four error flags, then two chunk tickets and the bound
+// of a wait, in polls, of the single-launch sweeps.
+constexpr int kFlagTicket = 4, kFlagSpin = 6, kFlagWords = 8;
 constexpr int kMaxKrylov = 64;   // largest FGMRES restart length
 constexpr int kDotParts = 512;   // partial sums of one Krylov dot product, at most
 // Blocks of 256 threads for a Krylov dot product over n entries: one entry per
@@ -279,6 +279,7 @@ struct cfd_mesh {
     double *zp = nullptr;  // nzp64 x [N][5] work vectors of the sweeps (single-launch: handover words)
     int nzp64 = 0, nzp32 = 0;
     float *zpf = nullptr;
+    int spin_max = 1 << 22;   // polls after which a wait of the single-launch sweeps is given up
     int flow_blocks = 0;      // workgroups of the single-launch sweeps, 0: by the rule
     bool sync_free = true;    // single-launch triangular sweeps (else one launch per level)
     // block-SELL copies for the Krylov loop: A (SpMV), and the multicolour

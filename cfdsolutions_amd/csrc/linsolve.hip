@@ -1073,8 +1073,9 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int nrows, const int *__r
 // chunk is always held by a wave that runs, whatever else the GPU holds and
 // however many of the launch's workgroups it holds, so a wait always ends.  (A
 // fixed share of the chunks to each workgroup needs every workgroup resident.)
-// A wait over kSpinMax polls raises flag[3], and every waiter gives up once it
-// is set: a sweep ends even where a store is lost, and the solve reports it.
+// A wait over cfd_mesh::spin_max polls (a word beside the flags) raises flag[3],
+// and every waiter gives up once it is set: a sweep ends even where a store is
+// lost, and the solve reports it.
 //
 // flow_blocks: how many workgroups pay depends on how many chunks can run at a
 // time (a level's).  Too few leave loads unissued, too many poll more than they
@@ -1084,7 +1085,6 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int nrows, const int *__r
 // 2.16; 333 (Delaunay mesh of 60,000, colours) -, 7.2, 7.8; 475 (72x24x24,
 // colours) 4.80, 3.24, 3.18; 1,088 (95x33x31, colours) -, 6.3, 5.5.
 // ---------------------------------------------------------------------------
-constexpr int kSpinMax = 1 << 22;
 inline int flow_blocks(const cfd_mesh *m, int64_t chunks, int64_t width) {
     const int64_t n = m->flow_blocks ? m->flow_blocks : width < 60 ? 128 : width < 400 ? 256 : 512;
     return (int)std::min((chunks + 3) / 4, n);
@@ -1127,7 +1127,7 @@ __device__ __forceinline__ void flow_unset(T *p) {
 // Whether poll `it` of a wait was its last: the bound is reached or another
 // wait's was.
 __device__ __forceinline__ bool flow_give_up(int it, int *flag) {
-    if ((it & 255) != 255 || (it < kSpinMax && ld_coh(flag + 3) == 0)) return false;
+    if ((it & 255) != 255 || (it < ld_coh(flag + kFlagSpin) && ld_coh(flag + 3) == 0)) return false;
     atomicOr(flag + 3, 1);
     return true;
 }
@@ -2871,6 +2871,15 @@ int enqueue_step_batch(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, T
     return CFD_OK;
 }
 
+// The solve's error flags to m->hflag; an error if a single-launch sweep gave up
+// a wait.
+int sweep_gave_up(cfd_mesh *m) {
+    m->hflag[2] = m->hflag[3] = 0;
+    CFD_HIP(m, hipMemcpyAsync(m->hflag, m->flag, 4 * sizeof(int), hipMemcpyDeviceToHost, m->stream));
+    CFD_HIP(m, hipStreamSynchronize(m->stream));
+    return m->hflag[3] ? cfd_set_error(m->ctx, CFD_E_HIP, "a single-launch sweep exceeded its wait bound") : CFD_OK;
+}
+
 // Batched restarted FGMRES(m): every case of the union runs the algorithm of
 // fgmres() on its own rows, in lockstep; a case that has converged (or is
 // not being solved) keeps riding along but its results are not used.
@@ -2947,6 +2956,8 @@ int fgmres_batch(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM 
                 kdim[c] = j + 1;
                 res[c] = fabs(gvc[j + 1]);
                 if (!(res[c] == res[c])) {
+                    rc = sweep_gave_up(m);
+                    if (rc) return rc;
                     // this case fails on its own (as its solve alone would);
                     // its correction is dropped and the other cases go on
                     status[c] = CFD_E_NONFINITE;
@@ -3049,7 +3060,11 @@ int fgmres(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM *lu, c
             total++;
             kdim = j + 1;
             res = fabs(gv[j + 1]);
-            if (!(res == res)) return cfd_set_error(m->ctx, CFD_E_NONFINITE, "FGMRES: non-finite residual");
+            if (!(res == res)) {
+                // a wait that was given up leaves NaNs: that is the failure then
+                rc = sweep_gave_up(m);
+                return rc ? rc : cfd_set_error(m->ctx, CFD_E_NONFINITE, "FGMRES: non-finite residual");
+            }
             // the next step starts with V_{j+1} = w / hn (k_scale_dev)
             if (res <= tol || hn == 0.0) break;
         }
@@ -3181,9 +3196,8 @@ static int gs_sweeps(cfd_mesh *m, int sweeps, const LevelSchedule &ls, int reach
         hipLaunchKernelGGL(k_vsum_partial, dim3(np, S), dim3(kBlock), 0, m->stream, (size_t)m->N, g.rows, m->red);
         hipLaunchKernelGGL(k_mdot_final, dim3(S), dim3(64), 0, m->stream, np, S, m->red, m->redout);
         CFD_HIP(m, hipMemcpyAsync(m->hred, m->redout, sizeof(double) * S, hipMemcpyDeviceToHost, m->stream));
-        CFD_HIP(m, hipMemcpyAsync(m->hflag, m->flag, 4 * sizeof(int), hipMemcpyDeviceToHost, m->stream));
-        CFD_HIP(m, hipStreamSynchronize(m->stream));
-        if (m->hflag[3]) return cfd_set_error(m->ctx, CFD_E_HIP, "Gauss-Seidel sweep exceeded its wait bound");
+        const int rc = sweep_gave_up(m);
+        if (rc) return rc;
         int last = S;
         for (int s = 0; s < S && !done; s++) {
             rms = sqrt(m->hred[s] / (double)m->N);
@@ -3440,11 +3454,9 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
 
 // Error flags raised by the preconditioner and the sweeps.
 int read_solve_flags(cfd_mesh *m) {
-    CFD_HIP(m, hipMemcpyAsync(m->hflag, m->flag, 4 * sizeof(int), hipMemcpyDeviceToHost, m->stream));
-    CFD_HIP(m, hipStreamSynchronize(m->stream));
+    const int rc = sweep_gave_up(m);
     if (m->hflag[2]) return cfd_set_error(m->ctx, CFD_E_SINGULAR, "zero pivot in %d diagonal blocks", m->hflag[2]);
-    if (m->hflag[3]) return cfd_set_error(m->ctx, CFD_E_HIP, "sync-free triangular sweep exceeded its wait bound");
-    return CFD_OK;
+    return rc;
 }
 
 }  // namespace
