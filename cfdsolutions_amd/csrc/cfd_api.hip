@@ -63,6 +63,7 @@ hipError_t cfd_host_alloc(void **p, size_t bytes) {
 void *cfd_dalloc(cfd_mesh *m, size_t bytes) {
     void *p = nullptr;
     if (bytes == 0) bytes = 8;
+    if ((int64_t)bytes > m->bytes_max - m->bytes) return nullptr;
     CfdRuntimeGuard g;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -305,6 +306,7 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
     m->E = E;
     m->B = B;
     m->NT = N + B;
+    if (const char *bm = getenv("CFD_MESH_BYTES_MAX")) m->bytes_max = strtoll(bm, nullptr, 10);
     int rc = CFD_OK;
     auto tph = std::chrono::steady_clock::now();
     auto phase = [&](const char *what) {

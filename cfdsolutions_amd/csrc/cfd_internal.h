@@ -209,6 +209,7 @@ struct cfd_mesh {
     hipStream_t stream = nullptr;
     int N = 0, E = 0, B = 0, NT = 0;
     int64_t bytes = 0;
+    int64_t bytes_max = INT64_MAX;  // allocations past it fail (CFD_MESH_BYTES_MAX: lets a test see memory run short)
     std::vector<std::pair<void *, size_t>> allocs;  // device allocations and their sizes
 
     // topology
@@ -265,6 +266,7 @@ struct cfd_mesh {
     double *gslu = nullptr;   // [N][25] LU of the diagonal blocks (block GS, LU-SGS)
     double *gsver = nullptr;  // [gs_nver][6 N] versions of x and row sums of the sweeps of one launch
     int gs_nver = 0;
+    bool gs_short = false;    // the device had no room for more of them
     LevelSchedule lower, upper;
     LevelSchedule gs;         // schedule of pipelined Gauss-Seidel sweeps (made on first use)
     int gs_reach = 0;         // and how many of its chunks an upper neighbour can be ahead

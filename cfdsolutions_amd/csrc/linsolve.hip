@@ -3252,10 +3252,29 @@ int run_gs_noalloc(cfd_mesh *m, int sweeps, cfd_linsolve_stats *st) {
 // Gauss-Seidel sweeps per launch: each keeps a version of x (48 bytes per node
 // with its row sums).  A further sweep in a launch costs reach + 1 chunks of
 // the chain, a further launch the whole chain, so as many as fit 512 MB, 32 at
-// most.
+// most, and fewer where the device has less left: one will do.
 static int gs_versions(const cfd_mesh *m, int sweeps) {
     const int64_t fit = (512LL << 20) / (48 * (int64_t)m->N);
     return (int)std::max<int64_t>(1, std::min<int64_t>({fit, 32, sweeps}));
+}
+
+// Room for `want` versions in m->gsver, at least `need`; how many there are.
+static int ensure_gs_room(cfd_mesh *m, int want, int need) {
+    if (m->gs_nver >= want) return want;
+    if (m->gs_short && m->gs_nver >= need) return m->gs_nver;
+    if (m->gs_nver) {
+        CfdRuntimeGuard g;
+        if (hipStreamSynchronize(m->stream) != hipSuccess) return 0;
+    }
+    cfd_dfree(m, m->gsver);
+    m->gsver = nullptr;
+    m->gs_nver = 0;
+    for (int v = want; v >= need && !m->gsver; v = v > need ? std::max(need, v / 2) : 0) {
+        m->gsver = (double *)cfd_dalloc(m, sizeof(double) * 6 * (size_t)m->N * v);
+        if (m->gsver) m->gs_nver = v;
+        else m->gs_short = true;
+    }
+    return m->gs_nver;
 }
 
 int run_linsolve(cfd_mesh *m, const cfd_linsolve_opts *o, cfd_linsolve_stats *st) {
@@ -3266,20 +3285,18 @@ int run_linsolve(cfd_mesh *m, const cfd_linsolve_opts *o, cfd_linsolve_stats *st
         if (m->jac_mixed) return cfd_set_error(m->ctx, CFD_E_ARG, "reference sweeps need an FP64 Jacobian");
         const int sweeps = o->sweeps > 0 ? o->sweeps : (o->solver == CFD_SOLVER_BLOCK_GS ? 10000 : 100);
         const bool gs = o->solver == CFD_SOLVER_BLOCK_GS;
-        const int nver = gs ? gs_versions(m, sweeps) : 3;
         if (!m->gslu) m->gslu = (double *)cfd_dalloc(m, sizeof(double) * 25 * (size_t)m->N);
-        if (m->gs_nver < nver) {
-            if (m->gs_nver) CFD_HIP(m, hipStreamSynchronize(m->stream));
-            cfd_dfree(m, m->gsver);
-            m->gsver = (double *)cfd_dalloc(m, sizeof(double) * 6 * (size_t)m->N * nver);
-            m->gs_nver = m->gsver ? nver : 0;
-        }
-        if (!m->gslu || !m->gsver) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory");
+        const int nver = m->gslu ? ensure_gs_room(m, gs ? gs_versions(m, sweeps) : 3, gs ? 1 : 3) : 0;
+        if (!nver) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (sweeps)");
         const size_t L = 5 * (size_t)m->N;
         double *ver = m->gsver;  // [nver][N][5], then [nver][N] row sums (GS) or the pivot orders (LU-SGS)
         if (gs) {
-            int rc = ensure_gs_schedule(m);
-            if (!rc) rc = gs_sweeps(m, sweeps, m->gs, m->gs_reach, GsScratch{m->gslu, ver + L * nver, ver, nver}, st);
+            // one sweep to a launch where there is no room for more, or for their schedule
+            int rc = nver > 1 ? ensure_gs_schedule(m) : CFD_OK;
+            const bool one = nver == 1 || rc == CFD_E_OOM;
+            if (rc && !one) return rc;
+            rc = gs_sweeps(m, sweeps, one ? m->lower : m->gs, one ? 0 : m->gs_reach,
+                           GsScratch{m->gslu, ver + L * nver, ver, one ? 1 : nver}, st);
             if (rc) return rc;
         } else {
             int *piv = (int *)(ver + 3 * L);
