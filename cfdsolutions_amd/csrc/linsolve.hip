@@ -8,6 +8,7 @@
 // level do not depend on each other and every row performs the same
 // operations in the same order as the sequential CPU code, so factors and
 // sweeps are bit-identical to it.
+#include <atomic>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -3111,32 +3112,54 @@ void drop_krylov_graphs(cfd_mesh *m) {
 }
 
 // The schedule of k_gs_flow (host, on the mesh's first Gauss-Seidel solve).
-// Row i of sweep s takes step p_i + lag s: p_i is the least number above the
-// p of every lower neighbour and at least p_k + 1 - lag for every upper
-// neighbour k.  The passes below raise p to that; they end for every lag from
-// the number of levels on, and in three passes for lag 8 on the bump channels
-// (lag 7 is the least there; the levels by themselves jump by up to 50 from a
-// row to an upper neighbour).  reach: the largest number of chunks from a row
-// to an upper neighbour.
+// Row i of sweep s takes step p_i + lag s: p_i is above the p of every lower
+// neighbour and at least p_k + 1 - lag for every upper neighbour k.  The levels
+// do with a lag one above their largest jump from a row to an upper neighbour
+// (50 on the bump channels of 200 levels).  A smaller lag is sought by raising
+// p: three passes settle lag 8 on the channels, where 7 is the least there is.
+// On unstructured meshes hardly any lag is below the jumps, and p rises without
+// end: a lag is given up when p passes twice the levels.  (Lags tried in turn
+// up to the levels, sixteen passes each, took 600 ms for 200,000 rows of a
+// Delaunay mesh, this 30.)  reach: the largest number of chunks from a row to
+// an upper neighbour.
 static int ensure_gs_schedule(cfd_mesh *m) {
     if (m->gs.slots12) return CFD_OK;
-    const int N = m->N;
-    std::vector<int> p(N), chunk(N), s12, rows(N);
-    for (int lag = 8;; lag *= 2) {
-        std::fill(p.begin(), p.end(), 0);
-        bool raised = true;
-        for (int pass = 0; pass < 16 && raised; pass++) {
+    const int N = m->N, nl = m->lower.nlevels;
+    std::vector<int> lev(N), p, chunk(N), s12, rows(N);
+    CFD_HIP(m, cfd_memcpy(rows.data(), m->lower.rows, sizeof(int) * rows.size(), hipMemcpyDeviceToHost));
+    for (int l = 0; l < nl; l++)
+        for (int t = m->lower.ptr[l]; t < m->lower.ptr[l + 1]; t++) lev[rows[t]] = l;
+    // largest of of(row, upper neighbour) over the pattern
+    auto most_over_upper = [&](const std::vector<int> &of) {
+        std::atomic<int> most{0};
+        cfd_parallel_for(N, [&](int64_t i0, int64_t i1) {
+            int d = 0;
+            for (int i = (int)i0; i < (int)i1; i++)
+                for (int k = m->h_iau[i] + 1; k < m->h_ia[i + 1]; k++) d = std::max(d, of[m->h_ja[k]] - of[i]);
+            for (int v = most; d > v && !most.compare_exchange_weak(v, d);) {
+            }
+        });
+        return most.load();
+    };
+    const int jump = most_over_upper(lev);
+    bool settled = false;
+    for (int lag = 8; lag <= jump && !settled; lag *= 4) {
+        p = lev;
+        bool raised = true, high = false;
+        for (int pass = 0; pass < 8 && raised && !high; pass++) {
             raised = false;
-            for (int i = 0; i < N; i++) {
+            for (int i = 0; i < N && !high; i++) {
                 int t = p[i];
                 for (int k = m->h_ia[i]; k < m->h_iau[i]; k++) t = std::max(t, p[m->h_ja[k]] + 1);
                 for (int k = m->h_iau[i] + 1; k < m->h_ia[i + 1]; k++) t = std::max(t, p[m->h_ja[k]] + 1 - lag);
                 raised = raised || t > p[i];
+                high = t > 2 * nl;
                 p[i] = t;
             }
         }
-        if (!raised) break;
+        settled = !raised && !high;
     }
+    if (!settled) p = lev;
     LevelSchedule &ls = m->gs;
     ls.nlevels = *std::max_element(p.begin(), p.end()) + 1;
     ls.ptr.assign(ls.nlevels + 1, 0);
@@ -3147,10 +3170,7 @@ static int ensure_gs_schedule(cfd_mesh *m) {
     pad_levels(ls.ptr, rows, 12, s12);
     for (size_t t = 0; t < s12.size(); t++)
         if (s12[t] >= 0) chunk[s12[t]] = (int)(t / 12);
-    m->gs_reach = 0;
-    for (int i = 0; i < N; i++)
-        for (int k = m->h_iau[i] + 1; k < m->h_ia[i + 1]; k++)
-            m->gs_reach = std::max(m->gs_reach, chunk[m->h_ja[k]] - chunk[i]);
+    m->gs_reach = most_over_upper(chunk);
     int *d = (int *)cfd_dalloc(m, sizeof(int) * s12.size());
     if (!d) return cfd_set_error(m->ctx, CFD_E_OOM, "out of device memory (sweep schedule)");
     CFD_HIP(m, cfd_memcpy(d, s12.data(), sizeof(int) * s12.size(), hipMemcpyHostToDevice));
