@@ -1069,7 +1069,7 @@ __global__ __launch_bounds__(kBlock) void k_trsv_level(int nrows, const int *__r
 // default NaN, so no result can look unset.
 //
 // Rows go in chunks of 12 in level order (levels are padded to whole chunks),
-// so a chunk reads only earlier ones.  A running workgroup draws the next four
+// so a chunk reads only earlier ones.  A running wave or workgroup draws its next
 // chunks by a ticket when it is done with the last: the earliest unfinished
 // chunk is always held by a wave that runs, whatever else the GPU holds and
 // however many of the launch's workgroups it holds, so a wait always ends.  (A
@@ -1139,15 +1139,25 @@ __device__ __forceinline__ T flow_wait(const T *p, typename FlowWord<T>::U v, in
     return __builtin_bit_cast(T, v);
 }
 
-// Chunk tickets of a launch, one to a workgroup for a chunk to each of its
-// wavefronts: for (w = next(); more(total); w = next()), with nothing to do for
-// a wave whose chunk w is not below total.  (Drawn when the chunks are done: the
-// answer of a ticket drawn ahead is waited for with the chunk's own loads, 2.4
-// against 1.7 ms for 20 Gauss-Seidel sweeps of the 48x16x16 mesh.)
-struct FlowTicket {
+// A wave's next chunk, from the launch's counter.  It is drawn when the last
+// chunk is done: the answer to a ticket drawn ahead is waited for with the
+// chunk's own loads, which are answered in order (20 Gauss-Seidel sweeps of the
+// 48x16x16 mesh 2.4 against 1.7 ms).
+__device__ __forceinline__ int flow_ticket(int *count) {
+    int w = 0;
+    if ((threadIdx.x & 63) == 0) w = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_amdgcn_readfirstlane(w);
+}
+// The same for a workgroup's four waves at once, where a launch's many short
+// chunks would crowd the counter (colours of 104,448 rows: 20 Arnoldi steps 5.5
+// ms, 8.3 with a ticket to a wave; Gauss-Seidel sweeps, with more work to a
+// chunk, lose by the barrier: 1.7 against 1.4 ms): for (w = next();
+// more(total); w = next()), with nothing to do for a wave whose w is not below
+// total.
+struct FlowGroup {
     int *const count, *const shared;  // the counter, two words of LDS
     int n = 0;
-    __device__ __forceinline__ FlowTicket(int *c, int *s) : count(c), shared(s) {}
+    __device__ __forceinline__ FlowGroup(int *c, int *s) : count(c), shared(s) {}
     __device__ __forceinline__ int next() {
         n ^= 1;
         if (threadIdx.x == 0)
@@ -1288,7 +1298,7 @@ __global__ __launch_bounds__(kBlock, kTrsvPerCu<TM>) void k_arnoldi_flow(FlowSte
     const double denom = f.norm2 ? sqrt(f.norm2[0]) : 1.0;
     const int cf = (f.nf + 11) / 12, cb = (f.nb + 11) / 12, cp = (f.np + 11) / 12;
     __shared__ int tickets[2];
-    FlowTicket q(f.ticket, tickets);
+    FlowGroup q(f.ticket, tickets);
     const int total = cf + cb + cp;
     for (int w = q.next(); q.more(total); w = q.next()) {
         if (w == 0 && lane == 0) st_coh(f.next_ticket, 0);
@@ -1763,7 +1773,7 @@ __device__ __forceinline__ const double *flow_lu(double *sh, int r, const double
 // ensure_gs_schedule).  Items (chunk c, sweep s) go in ascending
 // c + s (reach + 1), then s, so each needs only earlier ones.  The chain is about
 // levels + 8 S rows long instead of levels * S: 20 sweeps of the 48x16x16 mesh
-// (205 levels) took 64.3 ms with a launch per level, 1.71 ms so.
+// (205 levels) took 64.3 ms with a launch per level, 1.39 ms so.
 // x0: x before the first sweep.  rowrms[s][i]: row i's sum of sweep s.
 __global__ __launch_bounds__(kBlock, 2) void k_gs_flow(int N, int nchunk, int reach, int S, const int *__restrict__ slots,
                                                     const int *__restrict__ ia, const int *__restrict__ ja,
@@ -1776,10 +1786,8 @@ __global__ __launch_bounds__(kBlock, 2) void k_gs_flow(int N, int nchunk, int re
     // step t holds the items (t - s lag, s), lo <= s <= hi; first: the number of items before it
     const int lag = reach + 1, items = nchunk * S;
     int t = 0, first = 0, lo = 0, hi = 0;
-    __shared__ int tickets[2];
-    FlowTicket q(flag + kFlagTicket, tickets);
-    for (int w = q.next(); q.more(items); w = q.next()) {
-        if (w >= items) continue;
+    int *const ticket = flag + kFlagTicket;
+    for (int w = flow_ticket(ticket); w < items; w = flow_ticket(ticket)) {
         while (w - first > hi - lo) {
             first += hi - lo + 1;
             t++;
@@ -1905,12 +1913,9 @@ __global__ __launch_bounds__(kBlock, 2) void k_lusgs_flow(int nslots, const int 
     const int lane = threadIdx.x & 63, slot = lane / 5, r = lane - 5 * slot, base = lane - r;
     __shared__ __align__(16) FlowLds<double> lds;
     double *sh = lds.v[threadIdx.x >> 6] + slot * FlowLds<double>::slot;
-    __shared__ int drawn[2];
-    FlowTicket q(ticket, drawn);
     const int total = (nslots + 11) / 12;
-    for (int w = q.next(); q.more(total); w = q.next()) {
+    for (int w = flow_ticket(ticket); w < total; w = flow_ticket(ticket)) {
         if (w == 0 && lane == 0) st_coh(next_ticket, 0);
-        if (w >= total) continue;
         const int t = 12 * w + slot;
         const int i = slot < 12 && t < nslots ? slots[t] : -1;
         const size_t ri = 5 * (size_t)(i >= 0 ? i : 0) + r;
@@ -3203,11 +3208,13 @@ static int gs_sweeps(cfd_mesh *m, int sweeps, const LevelSchedule &ls, int reach
     int it = 0;
     for (bool done = false; it < sweeps && !done;) {
         const int S = std::min(g.nver, sweeps - it);
-        // a step's chunks of every sweep under way, five times over for the
-        // longer work on a row: 2.42, 1.93 and 1.71 ms at 128, 256 and 512
-        // workgroups (48x16x16 mesh, 100 chunks), 0.82, 0.86 and 0.97 (24x8x8, 17)
+        // a step's chunks of every sweep under way; more than 256 workgroups lose
+        // where sweeps hardly overlap (Delaunay meshes) and gain little elsewhere:
+        // 1.53, 1.39, 1.54 ms at 128, 256 and 512 (48x16x16 mesh), 0.79, 0.82, 0.94
+        // (24x8x8), 27.7, 21.3, 31.3 (Delaunay, 200,000 rows), 24.4, 16.1, 14.1
+        // (192x64x64, ten sweeps)
         const int64_t under = std::min<int64_t>(S, nchunk / (reach + 1) + 1);
-        const int64_t width = 5 * nchunk * under / ls.nlevels;
+        const int64_t width = std::min<int64_t>(nchunk * under / ls.nlevels, 399);
         hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(S * L, 4096)), dim3(kBlock), 0, m->stream, S * L, g.ver,
                            m->flag + kFlagTicket);
         hipLaunchKernelGGL(k_gs_flow, dim3(flow_blocks(m, (int64_t)nchunk * S, width)), dim3(kBlock), 0, m->stream, m->N, nchunk, reach, S, ls.slots12, m->ia, m->ja, m->iau, m->a, m->b, g.lu,
