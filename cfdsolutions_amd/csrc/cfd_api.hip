@@ -1067,8 +1067,7 @@ extern "C" int cfd_mesh_reset(cfd_mesh *m, const cfd_params *p) {
 // ---------------------------------------------------------------------------
 // fields
 // ---------------------------------------------------------------------------
-// reference (API) index of internal node record i (ghosts are not renumbered)
-constexpr size_t kFieldSmall = 128u << 10;
+constexpr size_t kFieldSmall = 64u << 10;
 // A field on the device: component f of node (or entry) i, in the caller's
 // numbering, is p[rec * i' + off + f] with i' = perm[i] below nperm, else i.
 struct FieldView {
@@ -1114,7 +1113,7 @@ __global__ __launch_bounds__(256) void k_field(FieldView v, size_t i0, size_t cn
 // One field between the device and the caller's array h [nf][n] (IN: to the
 // device), chunk by chunk through the two pinned slots: while the kernel moves
 // one chunk over PCIe, host threads copy the other from or to the caller's
-// pages.  The kernel puts the records into the caller's order, so only the
+// pages (a field up to kFieldSlot is a single chunk, one after the other).  The kernel puts the records into the caller's order, so only the
 // field itself crosses.  A whole record array copied to pageable memory, with
 // the host picking the components out on one thread, took 163 ms for one
 // set of residual components of the 160^3 cube (167 MB), this 5.5 ms.
@@ -1130,12 +1129,14 @@ static int field_transfer(cfd_mesh *m, const FieldView &v, double *h) {
         return CFD_OK;
     }
     // small records: the runtime's copy of a few kB is quicker than a kernel and
-    // an event (325 nodes: 12 us against 20)
+    // an event (time steps of 3,751 nodes, 30 kB, 14 us against 24; of 14,161,
+    // 113 kB, 28 against 20)
     const size_t nrec = v.n * v.rec;
     if (sizeof(double) * nrec <= kFieldSmall) {
         double buf[kFieldSmall / sizeof(double)];
         CFD_HIP(m, hipStreamSynchronize(m->stream));
-        CFD_HIP(m, cfd_memcpy(buf, v.p, sizeof(double) * nrec, hipMemcpyDeviceToHost));
+        if (!IN || v.nf < v.rec)  // (a whole record is written over)
+            CFD_HIP(m, cfd_memcpy(buf, v.p, sizeof(double) * nrec, hipMemcpyDeviceToHost));
         for (size_t ii = 0; ii < v.n; ii++) {
             const size_t i = ii < v.nperm ? (size_t)m->h_order[ii] : ii;
             for (int f = 0; f < v.nf; f++) {
