@@ -2036,43 +2036,61 @@ __device__ __forceinline__ double wave_sum4(double v0, double v1, double v2, dou
 // kUpdateDots keeps the entries' V values in registers between the update and
 // the products: a grid has at most kDotParts blocks, two wavefronts per SIMD,
 // so registers are free (rereading them from the caches took 166 us at 24
-// vectors of 4.08M FP32 entries, this 130 us with the final sums).
+// vectors of 4.08M FP32 entries, this 130 us with the final sums).  More than 41
+// values of FP64 do not fit beside their sums: there V is read again, two
+// entries at a time (gs_hold; steps 42 to 64 of the 192x64x64 mesh took 2.50 ms
+// each with values spilled, 2.35 so; up to 41 five spilled words lose less).
 enum GsMode { kDots, kUpdateDots, kUpdateNorm };
+
+template <class TV, int NVMAX, GsMode M>
+constexpr bool gs_hold = M == kUpdateDots && (sizeof(TV) == 4 || NVMAX <= 41);
 
 template <class TV, int NVMAX, GsMode M, int U>
 __device__ __forceinline__ void gs_entries(size_t o, size_t i, size_t stride, int nv, const TV *__restrict__ V,
                                            size_t ld, const double *__restrict__ h, TV *__restrict__ w, double *acc) {
-    constexpr int NC = (NVMAX + 7) / 8, HOLD = M == kUpdateDots ? NVMAX : 8;
+    constexpr int NC = (NVMAX + 7) / 8;
+    constexpr bool HOLD = gs_hold<TV, NVMAX, M>;
     double wi[U];
-    TV vv[U][HOLD];
+    TV vv[U][HOLD ? NVMAX : 8];
 #pragma unroll
     for (int u = 0; u < U; u++) wi[u] = (double)w[o + i + u * stride];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
+                if (k < nv) vv[u][HOLD ? k : k - 8 * c] = V[ld * k + o + i + u * stride];
+    };
+    auto dots = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
+                if (k < nv) acc[k] += (double)vv[u][HOLD ? k : k - 8 * c] * wi[u];
+    };
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         if (8 * c >= nv) continue;
+        load(c);
+        if (HOLD) continue;
+        if (M == kDots) {
+            dots(c);
+            continue;
+        }
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
             for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
-                if (k < nv) vv[u][M == kUpdateDots ? k : k - 8 * c] = V[ld * k + o + i + u * stride];
-        if (M == kUpdateDots) continue;
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int k = 8 * c; k < 8 * c + 8 && k < NVMAX; k++)
-                if (k < nv) {
-                    if (M == kDots) acc[k] += (double)vv[u][k - 8 * c] * wi[u];
-                    else wi[u] = wi[u] - h[k] * (double)vv[u][k - 8 * c];
-                }
+                if (k < nv) wi[u] = wi[u] - h[k] * (double)vv[u][k - 8 * c];
     }
     if (M == kDots) return;
-    if (M == kUpdateDots) {
+    if (HOLD) {
 #pragma unroll
         for (int k = 0; k < NVMAX; k++)
             if (k < nv) {
                 const double hk = h[k];
 #pragma unroll
-                for (int u = 0; u < U; u++) wi[u] = wi[u] - hk * (double)vv[u][M == kUpdateDots ? k : 0];
+                for (int u = 0; u < U; u++) wi[u] = wi[u] - hk * (double)vv[u][HOLD ? k : 0];
             }
     }
 #pragma unroll
@@ -2082,7 +2100,8 @@ __device__ __forceinline__ void gs_entries(size_t o, size_t i, size_t stride, in
         wi[u] = (double)wt;
         if (M == kUpdateNorm) acc[0] += wi[u] * wi[u];
     }
-    if (M == kUpdateDots) {
+    if (M == kUpdateNorm) return;
+    if (HOLD) {
         // (the empty asm: an FP32 value is converted again rather than kept in
         // FP64 from the update on, which would double its registers)
         if (sizeof(TV) == 4) {
@@ -2090,14 +2109,16 @@ __device__ __forceinline__ void gs_entries(size_t o, size_t i, size_t stride, in
             for (int k = 0; k < NVMAX; k++)
 #pragma unroll
                 for (int u = 0; u < U; u++)
-                    if (k < nv) asm volatile("" : "+v"(vv[u][M == kUpdateDots ? k : 0]));
+                    if (k < nv) asm volatile("" : "+v"(vv[u][HOLD ? k : 0]));
         }
+    } else {
+        asm volatile("" ::: "memory");  // V is read again rather than kept
+    }
 #pragma unroll
-        for (int k = 0; k < NVMAX; k++)
-            if (k < nv) {
-#pragma unroll
-                for (int u = 0; u < U; u++) acc[k] += (double)vv[u][M == kUpdateDots ? k : 0] * wi[u];
-            }
+    for (int c = 0; c < NC; c++) {
+        if (8 * c >= nv) continue;
+        if (!HOLD) load(c);
+        dots(c);
     }
 }
 
@@ -2561,7 +2582,7 @@ template <class TV, int NVMAX>
 constexpr int gs_unroll(GsMode M) {
     if (M != kUpdateDots || NVMAX == 8) return 4;
     if (sizeof(TV) == 4) return NVMAX <= 32 ? 4 : NVMAX <= 41 ? 2 : 1;
-    return NVMAX <= 16 ? 2 : 1;
+    return NVMAX <= 16 || NVMAX > 41 ? 2 : 1;
 }
 
 // One Gram-Schmidt pass of w against V_0..V_{nv-1} (coefficients at m->redout +
