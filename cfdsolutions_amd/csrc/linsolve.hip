@@ -1736,7 +1736,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sell_half(int N, const int *__r
 }
 
 // ---------------------------------------------------------------------------
-// Reference sweeps (MATH/src/MC_Iterative_Jacobi.c), one level per launch
+// Reference sweeps (MATH/src/MC_Iterative_Jacobi.c): Gauss-Seidel sweeps in one
+// launch as a pipeline, LU-SGS one launch a half sweep
 // ---------------------------------------------------------------------------
 // No-pivot LU of the diagonal blocks, MC_Iterative_Jacobi.c:381-396
 __global__ __launch_bounds__(kBlock) void k_gs_lu(int N, const int *iau, const double *a, double *lu) {
@@ -2039,7 +2040,7 @@ __device__ __forceinline__ double wave_sum4(double v0, double v1, double v2, dou
 // vectors of 4.08M FP32 entries, this 130 us with the final sums).  More than 41
 // values of FP64 do not fit beside their sums: there V is read again, two
 // entries at a time (gs_hold; steps 42 to 64 of the 192x64x64 mesh took 2.50 ms
-// each with values spilled, 2.35 so; up to 41 five spilled words lose less).
+// each with values spilled, 2.34 so).
 enum GsMode { kDots, kUpdateDots, kUpdateNorm };
 
 template <class TV, int NVMAX, GsMode M>
@@ -2733,7 +2734,6 @@ template <class TM, class TV>
 void arnoldi_step(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V, TV *Z, TV *w, int j) {
     const size_t L = 5 * (size_t)m->N;
     const int gN = grid_cap(L, 4096);
-    const int gS = (int)((L + kBlock - 1) / kBlock);
     TV *vj = V + L * j, *zj = Z + L * j;
     const double *norm2 = j > 0 ? m->redout + 2 * (kMaxKrylov + 1) : nullptr;
     bool product = false;
@@ -2828,7 +2828,6 @@ template <class TM, class TV>
 void arnoldi_step_batch(cfd_mesh *m, const TM *a, const TM *lu, const TM *dinv, TV *V, TV *Z, TV *w, int j) {
     const size_t L = 5 * (size_t)m->N;
     const int gN = grid_cap(L, 4096);
-    const int gS = (int)((L + kBlock - 1) / kBlock);
     TV *vj = V + L * j, *zj = Z + L * j;
     if (j > 0)
         hipLaunchKernelGGL((k_scale_dev_seg<TV, TV>), dim3(gN), dim3(kBlock), 0, m->stream, L, m->ecase, w, vj,
@@ -2917,7 +2916,6 @@ int fgmres_batch(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM 
     const int K = m->ncase, mk = o->krylov_m;
     const size_t L = 5 * (size_t)m->N;
     const int gN = grid_cap(L, 4096);
-    const int gS = (int)((L + kBlock - 1) / kBlock);
     const size_t ldc = kMaxKrylov + 1;
     hipLaunchKernelGGL(k_fill, dim3(gN), dim3(kBlock), 0, m->stream, L, 0.0, m->x);
     CFD_HIP(m, hipMemcpyAsync(m->r, m->b, sizeof(double) * L, hipMemcpyDeviceToDevice, m->stream));
@@ -3043,7 +3041,6 @@ int fgmres(cfd_mesh *m, const cfd_linsolve_opts *o, const TM *a, const TM *lu, c
     const int mk = o->krylov_m;
     const size_t L = 5 * (size_t)m->N;
     const int gN = grid_cap(L, 4096);
-    const int gS = (int)((L + kBlock - 1) / kBlock);
     double *hr = m->hred;
     // x0 = 0; r0 = b
     hipLaunchKernelGGL(k_fill, dim3(gN), dim3(kBlock), 0, m->stream, L, 0.0, m->x);
@@ -3472,7 +3469,7 @@ int prepare_fgmres(cfd_mesh *m, const cfd_linsolve_opts *o) {
     const size_t nw = (size_t)(kMaxKrylov + 1) * (m->ncase ? m->seg_dot.nblocks : dot_parts(5 * (size_t)m->N));
     hipLaunchKernelGGL(k_flow_unset<double>, dim3(grid_cap(nw, 4096)), dim3(kBlock), 0, m->stream, nw,
                        m->ncase ? m->bpart : m->red, (int *)nullptr);
-    if (flow_sweeps(m, o->precond)) {
+    if (o->precond == CFD_PREC_ILU0_MC && flow_sweeps(m, o->precond)) {
         rc = ensure_slots12(m, m->mc_lower);
         if (!rc) rc = ensure_slots12(m, m->mc_upper);
         if (rc) return rc;

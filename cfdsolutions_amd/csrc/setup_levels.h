@@ -1,6 +1,8 @@
-// Host-side set-up of the ILU(0) factorisation and sweep schedules, on up to
-// 16 threads (cfd_parallel_for must be visible where this is included).  The
-// results equal those of one sequential pass over the rows.
+// Host-side set-up of the sweep schedules, on up to 16 threads (cfd_parallel_for
+// must be visible where this is included).  The results equal those of one
+// sequential pass over the rows.  The library uses group_by_level; the merge map
+// and build_levels_by_colour are host statements of what its kernels do now
+// (k_ilu0_level's search, k_mc_levels) and are held by a host test.
 #pragma once
 
 #include <algorithm>
