@@ -715,8 +715,11 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         }
         hipMemsetAsync(m->d.qb, 0, sizeof(double) * kQB * (size_t)N, m->stream);
         hipMemsetAsync(m->roe_blk, 0, sizeof(int) * (size_t)((N + 4095) / 4096), m->stream);
-        hipMemsetAsync(m->flag, 0, sizeof(int) * kFlagWords, m->stream);
-        hipMemcpyAsync(m->flag + kFlagSpin, &m->spin_max, sizeof(int), hipMemcpyHostToDevice, m->stream);
+        hipMemsetAsync(m->flag, 0, sizeof(int) * kFlagSpin, m->stream);
+        if (cfd_memcpy(m->flag + kFlagSpin, &m->spin_max, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
+            cfd_mesh_destroy(m);
+            return cfd_set_error(ctx, CFD_E_HIP, "hipMemcpy failed");
+        }
         hipMemsetAsync(m->d.res, 0, sizeof(double) * kRES * (size_t)N, m->stream);
         phase("workspaces");
         rc = launch_lsq_coef(m);
