@@ -477,7 +477,11 @@ int cfd_mesh_create_cases(cfd_ctx *ctx, const cfd_mesh_desc *d, const cfd_params
         for (int i = 0; i < N; i++) m->h_ia[i + 1] = m->h_ia[i] + (d->n2n_ia[i + 1] - d->n2n_ia[i]) + 1;
         m->nnz = m->h_ia[N];
         int over = 0;
-        for (int i = 0; i < N; i++) over += m->h_ia[i + 1] - m->h_ia[i] > kIluKeep;
+        for (int i = 0; i < N; i++) {
+            const int n = m->h_ia[i + 1] - m->h_ia[i];
+            over += n > kIluKeep;
+            m->ilu_row = std::max(m->ilu_row, n);
+        }
         m->ilu_long = over >= std::max(1, N / 16);
         m->h_ja.resize(m->nnz);
         m->h_iau.resize(N);

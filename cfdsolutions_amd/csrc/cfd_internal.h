@@ -257,6 +257,7 @@ struct cfd_mesh {
     double *dt = nullptr;     // [N]
     int nnz = 0;
     std::vector<int> h_ia, h_ja, h_iau;
+    int ilu_row = 0;          // blocks of the longest row
     bool ilu_long = false;    // one row in 16 or more has over kIluKeep blocks
     int *ia = nullptr, *ja = nullptr, *iau = nullptr;
     double *a = nullptr, *b = nullptr, *x = nullptr;

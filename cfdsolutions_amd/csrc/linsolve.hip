@@ -570,7 +570,8 @@ __device__ __forceinline__ void block_update(TM *B, const TM *L, const TM *__res
     }
 }
 
-template <class TM, int G>
+// MORE: rows may have blocks that stay in lu (4% of the time where none has).
+template <class TM, int G, bool MORE>
 __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__restrict__ rows,
                                                       const int *__restrict__ ia, const int *__restrict__ ja,
                                                       const int *__restrict__ iau, const int *__restrict__ src,
@@ -606,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
             }
         }
     }
-    const bool more = __any(n > NS * G);  // a row has blocks that stay in lu: the columns of the next NX per lane
+    const bool more = MORE && __any(n > NS * G);  // a row has blocks that stay in lu: the columns of the next NX per lane
     int xcol[NX];
     if (more) {
 #pragma unroll
@@ -776,7 +777,7 @@ __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__r
 constexpr int kIluCols = kIluKeep / 5;                           // blocks of a row kept in LDS, the rest stay in lu:
 constexpr int kIluMore = 4, kIluSeen = kIluKeep + 5 * kIluMore;  // of these so many have their columns in registers
 
-template <class TM>
+template <class TM, bool MORE>
 __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restrict__ rows, const int *__restrict__ ia,
                                                   const int *__restrict__ ja, const int *__restrict__ iau,
                                                   const int *__restrict__ src, const TM *__restrict__ a, TM *lu,
@@ -823,7 +824,7 @@ __global__ __launch_bounds__(64) void k_ilu0_rows(int nrows, const int *__restri
 #pragma unroll
                 for (int c = 0; c < 5; c++) keep[5 * h + b][c][lane] = A[b][c];
     }
-    const bool more = __any(n > kIluKeep);
+    const bool more = MORE && __any(n > kIluKeep);
     int xcol[kIluMore];
     if (more) {
 #pragma unroll
@@ -2435,15 +2436,20 @@ void ilu0_levels(cfd_mesh *m, const LevelSchedule &ls, const int *ia, const int 
     const int narrow = !m->ilu_long ? kIluNarrowRows : sizeof(TM) == 4 ? INT_MAX : kIluLongRows;
     for (int l = 0; l < ls.nlevels; l++) {
         const int b0 = ls.ptr[l], nr = ls.ptr[l + 1] - b0;
-#define CFD_ILU(G)                                                                                                    \
-    hipLaunchKernelGGL((k_ilu0_level<TM, G>), dim3((nr + 4 * (12 / G) - 1) / (4 * (12 / G))), dim3(kBlock), 0,         \
-                       m->stream, nr, ls.rows + b0, ia, ja, iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, \
-                       m->flag)
-        if (nr <= narrow) CFD_ILU(12);
-        else if (nr <= kIluFewRows) CFD_ILU(4);
-        else
-            hipLaunchKernelGGL(k_ilu0_rows<TM>, dim3((nr + 11) / 12), dim3(64), 0, m->stream, nr, ls.rows + b0, ia, ja,
-                               iau, src, a, lu, dinv, (const TM *)lu, (const TM *)dinv, m->flag);
+#define CFD_ILU(KERNEL, GRID, BLOCK)                                                                              \
+    hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(BLOCK), 0, m->stream, nr, ls.rows + b0, ia, ja, iau, src, a, lu, \
+                       dinv, (const TM *)lu, (const TM *)dinv, m->flag)
+#define CFD_ILU_LEVEL(G)                                                                               \
+    do {                                                                                               \
+        const int rows = 4 * (12 / G);                                                                 \
+        if (m->ilu_row > kIluSets<G> * G) CFD_ILU((k_ilu0_level<TM, G, true>), (nr + rows - 1) / rows, kBlock); \
+        else CFD_ILU((k_ilu0_level<TM, G, false>), (nr + rows - 1) / rows, kBlock);                    \
+    } while (0)
+        if (nr <= narrow) CFD_ILU_LEVEL(12);
+        else if (nr <= kIluFewRows) CFD_ILU_LEVEL(4);
+        else if (m->ilu_row > kIluKeep) CFD_ILU((k_ilu0_rows<TM, true>), (nr + 11) / 12, 64);
+        else CFD_ILU((k_ilu0_rows<TM, false>), (nr + 11) / 12, 64);
+#undef CFD_ILU_LEVEL
 #undef CFD_ILU
     }
 }
