@@ -570,7 +570,7 @@ __device__ __forceinline__ void block_update(TM *B, const TM *L, const TM *__res
     }
 }
 
-// MORE: rows may have blocks that stay in lu (4% of the time where none has).
+// MORE: rows may have blocks that stay in lu (2 to 4% of the time where none has).
 template <class TM, int G, bool MORE>
 __global__ __launch_bounds__(kBlock) void k_ilu0_level(int nrows, const int *__restrict__ rows,
                                                       const int *__restrict__ ia, const int *__restrict__ ja,
@@ -3149,7 +3149,7 @@ void drop_krylov_graphs(cfd_mesh *m) {
 // On unstructured meshes hardly any lag is below the jumps, and p rises without
 // end: a lag is given up when p passes twice the levels.  (Lags tried in turn
 // up to the levels, sixteen passes each, took 600 ms for 200,000 rows of a
-// Delaunay mesh, this 30.)  reach: the largest number of chunks from a row to
+// Delaunay mesh, this 40.)  reach: the largest number of chunks from a row to
 // an upper neighbour.
 static int ensure_gs_schedule(cfd_mesh *m) {
     if (m->gs.slots12) return CFD_OK;
